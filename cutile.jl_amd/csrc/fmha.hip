@@ -961,6 +961,10 @@ extern "C" int mi_fmha_kernel(const mi_tile_array* Q, const mi_tile_array* K, co
             fmha::pipe_launch(pr, s);
             return launch_status();
         }
+        if (!no_pipe && fmha::pipe128_applicable(pr)) {
+            fmha::pipe128_launch(pr, s);
+            return launch_status();
+        }
     }
     if (dt == MI_F16) {
         if (D == 64) launch<F16, 64>(grid, s, causal, Q, K, V, Out, H, QUERY_GROUP_SIZE, scale2, input_pos, vec_ok);

@@ -42,46 +42,9 @@ constexpr int kSlotBytes = kSlot * 2;
 constexpr int kPre = 1;           // issue slots of a step that run before its wait and barrier
 constexpr float kRaise = 8.0f;    // raise m only when the new maximum exceeds it by this much
 
-#pragma clang diagnostic ignored "-Winline-asm"  // m0 is named as clobbered on purpose
-
-// One 1 KB global->LDS transfer: lane l moves 16 bytes from sbase + voff to lds_base + 16*l.
-__device__ __forceinline__ void dma16(unsigned voff, const char* sbase, unsigned lds_base) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :
-                 : "v"(voff), "s"(sbase), "s"(lds_base)
-                 : "memory", "m0");
-}
-
-__device__ __forceinline__ void fence() { asm volatile("" ::: "memory"); }
-
 // s_waitcnt immediates (gfx9 encoding): lgkmcnt(0) with vmcnt(N)
 constexpr int kWaitVm0 = 0x0070, kWaitVm4 = 0x0074, kWaitVm8 = 0x0078, kWaitVm2 = 0x0072, kWaitVm6 = 0x0076,
               kWaitLgkm = 0xc07f;   // lgkmcnt(0) alone
-
-template <int IMM>
-__device__ __forceinline__ void wait_and_barrier() {
-    __builtin_amdgcn_s_waitcnt(IMM);
-    fence();
-    __builtin_amdgcn_s_barrier();
-    fence();
-}
-
-// max(a, b, c) as one instruction (v_maximum3_f32: the IEEE 754-2019 maximum, which propagates NaN).  fmaxf() is
-// preceded by a quieting v_max_f32 x, x of every operand the compiler can not prove to be no signalling NaN, and
-// MFMA results are such operands; an inline-asm v_max3_f32 makes the compiler put a wait state after every one.
-__device__ __forceinline__ float max3(float a, float b, float c) {
-    return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c);
-}
-
-// max / sum over the lane pair (l, l ^ 32)
-__device__ __forceinline__ float xhalf_max(float v) {
-    auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return max3(__uint_as_float(r[0]), __uint_as_float(r[1]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float xhalf_sum(float v) {
-    auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
 
 // RG: the sequence length is not a multiple of 128.  The grid is that of the next multiple; the halves that exist are
 // walked as usual, the last of them re-reads its last row in place of the rows past the end (ragged_offsets), halves
@@ -249,22 +212,6 @@ __device__ __forceinline__ void exp_stage1(const f32x16& s, int h, float (&p)[2]
     p[0] = __builtin_amdgcn_exp2f(s[2 * h]);
     p[1] = __builtin_amdgcn_exp2f(s[2 * h + 1]);
 }
-template <typename E>
-__device__ __forceinline__ void exp_stage2(const float (&p)[2], int h, float& l, unsigned (&pf)[2][4]) {
-    const unsigned pk = Pack<E>::pack(p[0], p[1]);
-    pf[h >> 2][h & 3] = pk;
-    if constexpr (Pack<E>::kChunkSum) {
-        if ((h & 3) == 3) l = Pack<E>::sum_chunk(pf[h >> 2], l);   // the chunk is complete
-    } else {
-        l = Pack<E>::sum2(pk, p[0], p[1], l);
-    }
-}
-
-// Closes an issue slot: nothing is scheduled across it.
-__device__ __forceinline__ void slot_end() {
-    __builtin_amdgcn_sched_barrier(0);
-}
-
 constexpr int popcount2(int m) { return (m & 1) + ((m >> 1) & 1); }
 // k-th stream (0-based) of a non-empty 2-bit stream mask
 constexpr int nth_stream(int m, int k) { return (m & 1) ? k : 1; }

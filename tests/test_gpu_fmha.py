@@ -164,6 +164,34 @@ def test_fmha_pipelined_kernel_ragged_without_the_causal_mask(ct, orc, batch, he
     check(orc, out, ref, 2e-2 if T == torch.float16 else 3e-2)
 
 
+@pytest.mark.parametrize("batch,heads,sq,skv,qg,causal,pos,T", [
+    (1, 8, 128, 128, 1, True, 0, torch.float16), (2, 3, 65, 32, 1, False, 0, torch.bfloat16),    # fewest queries and keys; one half
+    (1, 8, 129, 129, 4, True, 0, torch.float16), (1, 2, 127, 33, 2, False, 0, torch.float16),    # one past / short of a block, of a half
+    (1, 4, 191, 95, 1, True, 0, torch.bfloat16), (1, 16, 257, 257, 4, True, 0, torch.bfloat16),  # fewer keys than queries; nine halves
+    (2, 4, 100, 290, 2, True, 190, torch.float16), (1, 3, 200, 333, 3, True, 7, torch.float16),  # decode offsets, on and off 32
+    (1, 6, 130, 225, 1, False, 0, torch.bfloat16), (3, 8, 320, 320, 2, True, 0, torch.float16),
+    (1, 40, 500, 500, 5, True, 0, torch.float16),                                                # heads walked in two uneven chunks per XCD
+])
+@pytest.mark.parametrize("rising", [False, True])
+def test_fmha_pipelined_kernel_for_heads_of_128(ct, orc, batch, heads, sq, skv, qg, causal, pos, T, rising):
+    """The D = 128 kernel at the edges of its 32-key halves, 64-query waves and 128-query workgroups: walks of one to
+    many halves, a ragged last half (which re-reads keys of the half before and masks them), decode offsets, grouped
+    heads, head counts that are and are not multiples of 8.  `rising`: scores that grow along the keys, so that the
+    running maximum is raised again and again.  The output sits in a wider buffer that must stay as it was."""
+    data = fmha.prepare(batch=batch, heads=heads, seq_q=sq, seq_kv=skv, d_k=128, d_v=128, query_group_size=qg, causal=causal, T=T)
+    if rising:
+        data.Q = (data.Q.float() * 0.25 + 1.0).to(T)
+        data.K = ((data.K.float() * 0.25 + 1.0) * (1.0 + 6.0 * torch.arange(skv, device="cuda") / skv)[None, None, :, None]).to(T)
+    big = torch.full((batch, heads, sq + 9, 128), 777.0, dtype=T, device="cuda")
+    out = big[:, :, :sq, :]
+    out.fill_(float("nan"))
+    fmha.cutile_fmha(data.Q, data.K, data.V, query_group_size=qg, causal=causal, input_pos=pos, out=out)
+    assert ct.last_variant() == "fmha_pipe_d128_q128_kv32_ring4"
+    assert bool((big[:, :, sq:, :] == 777.0).all())
+    ref = orc.fmha_general(*(orc.to_julia(t) for t in (data.Q, data.K, data.V)), causal=causal, input_pos=pos)
+    check(orc, out, ref, 2e-2 if T == torch.float16 else 3e-2)
+
+
 def test_fmha_more_keys_than_queries_takes_the_general_kernel(ct, orc):
     data = fmha.prepare(batch=1, heads=2, seq_q=200, seq_kv=333, causal=False)
     r = run(data)
