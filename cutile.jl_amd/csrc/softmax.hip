@@ -52,97 +52,140 @@ template <> __device__ __forceinline__ void vset<__hip_bfloat16>(Raw<__hip_bfloa
 
 // A 16-byte vector at an address that is aligned for its elements only: global memory takes such accesses, in one
 // instruction (a column of 50257 floats starts anywhere).
-template <typename V, typename T>
-__device__ __forceinline__ V ld_unaligned(const T* p) {
-    V v;
-    __builtin_memcpy(&v, p, sizeof(V));
-    return v;
+template <bool STREAM, typename V, typename T>
+__device__ __forceinline__ V ld_vec(const T* p) {
+    typedef V U __attribute__((aligned(alignof(T))));
+    const U* q = reinterpret_cast<const U*>(p);
+    return STREAM ? __builtin_nontemporal_load(q) : *q;
 }
 template <typename V, typename T>
-__device__ __forceinline__ void st_unaligned(const V& v, T* p) {
-    __builtin_memcpy(p, &v, sizeof(V));
+__device__ __forceinline__ void st_vec(V v, T* p) {
+    typedef V U __attribute__((aligned(alignof(T))));
+    __builtin_nontemporal_store(v, reinterpret_cast<U*>(p));
+}
+
+// Barrier that waits for this wave's LDS accesses only: loads and stores stay in flight across it.
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xc07f);   // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+// All-reduce over the workgroup, one barrier: `red` (NW floats) has to be another array than the reduction's before.
+template <int NW, typename Op>
+__device__ __forceinline__ float reduce(float v, float* red, Op op) {
+    v = wave_reduce(v, op);
+    if constexpr (NW == 1) return v;
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    lds_barrier();
+    v = red[threadIdx.x & (NW - 1)];
+#pragma unroll
+    for (int off = NW / 2; off >= 1; off >>= 1) v = op(v, __shfl_xor(v, off, 64));
+    return v;
 }
 
 // ---- single-tile kernel: column cached in registers -----------------------------------
-// Capacity BLOCK*VPT*EV elements.  ALIGNED: every column starts on a 16-byte boundary (plain and streaming vector
-// accesses); otherwise the vectors inside the column move unaligned and only the one across its end element-wise.
-template <typename T, int BLOCK, int VPT, bool ALIGNED, bool STREAM>
-__global__ __launch_bounds__(BLOCK) void softmax_regs_kernel(T* __restrict__ out, int64_t ldo,
-                                                             const T* __restrict__ in, int64_t ldi,
-                                                             int L, int64_t M) {
+// Capacity BLOCK*VPT*EV elements.  A column is a scalar head up to its first 16-byte boundary, whole vectors, and a scalar
+// tail; head and tail are one element in each of the first lanes.  (Where input and output do not sit at the same
+// offset from such a boundary there is no head and the vectors move unaligned.)
+// What bounds it is HBM, so everything is about keeping loads in flight:
+//   - a lane's vectors are requested together, from addresses clamped to the last vector of the column (its value
+//     again changes no maximum, and is left out of the sum and of the stores); behind a per-vector bounds branch each
+//     load was waited for before the next was sent;
+//   - 16-bit columns stay packed in the registers and their exponentials are made twice, for the sum and for the result:
+//     at 1024 lanes a column of 65536 takes 32 of a lane's 64 registers, so two workgroups share a CU;
+// Before / now, in three rotating buffers: bf16 1024 x 50257 57 -> 41 us (5.0 TB/s), 4096 x 32768 239 -> 93, 1682 x 28672
+// 102 -> 34; f16 2048 x 8191 18.6 -> 12.0, 4096 x 4096 13.2 -> 11.1; fp32 1024 x 50257 91 -> 83, 3000 x 20000 93 -> 81.
+// Workgroups that walk the columns and request the next one while they store were no faster (1024 lanes, fp32
+// 4096 x 32768: 190 us against 179 with a workgroup per column).
+template <typename T, int BLOCK, int VPT, bool STREAM>
+__global__ __launch_bounds__(BLOCK, BLOCK == 1024 && VPT <= 8 ? 8 : 1) void softmax_regs_kernel(
+    T* __restrict__ out, int64_t ldo, const T* __restrict__ in, int64_t ldi, int L) {
     constexpr int EV = Raw<T>::EV;
+    constexpr bool PACKED = sizeof(T) == 2;
     using V = typename Raw<T>::V;
     constexpr int NW = BLOCK / 64;
-    __shared__ float red[NW > 1 ? NW : 1];
+    __shared__ float red_max[NW], red_sum[NW];
     const float NEG_INF = -INFINITY;
+    const int t = threadIdx.x;
 
-    for (int64_t col = blockIdx.x; col < M; col += gridDim.x) {
-        const T* ip = in + col * ldi;
-        T* op = out + col * ldo;
-        float x[VPT][EV];
+    const T* ip = in + blockIdx.x * ldi;
+    T* op = out + blockIdx.x * ldo;
+    int head = 0;
+    {
+        const uintptr_t ai = (uintptr_t)ip, ao = (uintptr_t)op;
+        if ((ai & 15) == (ao & 15)) head = (int)(((16 - (ai & 15)) & 15) / sizeof(T));
+        if (head > L) head = L;
+    }
+    const int nv = (L - head) / EV;                        // whole vectors
+    const bool has1 = t < L - nv * EV;                     // the lane holds an element of head or tail, this one:
+    const int e1 = t < head ? t : nv * EV + t;
+    V x[VPT];
+    if (nv > 0) {
 #pragma unroll
         for (int v = 0; v < VPT; ++v) {
-            const int e0 = (threadIdx.x + v * BLOCK) * EV;
-            if (e0 + EV <= L) {
-                V raw;
-                if (ALIGNED) raw = ld_global<STREAM>(reinterpret_cast<const V*>(ip + e0));
-                else raw = ld_unaligned<V>(ip + e0);
-#pragma unroll
-                for (int q = 0; q < EV; ++q) x[v][q] = vget<T>(raw, q);
-            } else {
-#pragma unroll
-                for (int q = 0; q < EV; ++q) x[v][q] = (e0 + q < L) ? to_f32<T>(ip[e0 + q]) : NEG_INF;
-            }
+            const int i = t + v * BLOCK;
+            x[v] = ld_vec<STREAM, V>(ip + head + (i < nv ? i : nv - 1) * EV);
         }
-        float mx = NEG_INF;
+    } else {
 #pragma unroll
         for (int v = 0; v < VPT; ++v)
 #pragma unroll
-            for (int q = 0; q < EV; ++q) mx = fmaxf(mx, x[v][q]);
-        mx = block_reduce<NW>(mx, red, MaxOp{}, NEG_INF);
-        float sum = 0.f;
-        if constexpr (BLOCK == 1024) {
-            // One workgroup holds the CU here, so nothing runs under this loop: 64 library exponentials per lane
-            // (about twenty instructions each) were as long as the column's load.  The hardware's 2^x on
-            // (x - max) * log2(e), the product formed by one fma: two instructions, and an error of the argument's
-            // rounding, |x - max| * 2^-24 relative (3e-6 at 50 below the maximum, where the value is 2e-22).
-            const float l2e = 1.4426950408889634f, mxl = mx == NEG_INF ? 0.f : mx * l2e;
-#pragma unroll
-            for (int v = 0; v < VPT; ++v)
-#pragma unroll
-                for (int q = 0; q < EV; ++q) {
-                    x[v][q] = __builtin_amdgcn_exp2f(__builtin_fmaf(x[v][q], l2e, -mxl));
-                    sum += x[v][q];
-                }
-        } else {
-#pragma unroll
-            for (int v = 0; v < VPT; ++v)
-#pragma unroll
-                for (int q = 0; q < EV; ++q) {
-                    x[v][q] = expf(x[v][q] - mx);
-                    sum += x[v][q];
-                }
-        }
-        sum = block_reduce<NW>(sum, red, SumOp{}, 0.f);
-        // one correctly rounded reciprocal per column, then multiplies: within 1.5 ulp of the
-        // element-wise quotient, at a tenth of the instructions
-        const float rsum = 1.0f / sum;
-#pragma unroll
-        for (int v = 0; v < VPT; ++v) {
-            const int e0 = (threadIdx.x + v * BLOCK) * EV;
-            if (e0 + EV <= L) {
-                V raw;
-#pragma unroll
-                for (int q = 0; q < EV; ++q) vset<T>(raw, q, x[v][q] * rsum);
-                if (ALIGNED) st_global<true>(raw, reinterpret_cast<V*>(op + e0));
-                else st_unaligned<V>(raw, op + e0);
-            } else {
-#pragma unroll
-                for (int q = 0; q < EV; ++q)
-                    if (e0 + q < L) op[e0 + q] = from_f32<T>(x[v][q] * rsum);
-            }
-        }
+            for (int q = 0; q < EV; ++q) vset<T>(x[v], q, NEG_INF);
     }
+    float x1 = has1 ? to_f32<T>(ip[e1]) : NEG_INF;
+    auto keep_packed = [&]() {   // (or the widened elements of one pass would be kept for the next)
+        if constexpr (PACKED)
+#pragma unroll
+            for (int v = 0; v < VPT; ++v) asm volatile("" : "+v"(x[v]));
+    };
+    float mx = x1;
+#pragma unroll
+    for (int v = 0; v < VPT; ++v)
+#pragma unroll
+        for (int q = 0; q < EV; ++q) mx = fmaxf(mx, vget<T>(x[v], q));
+    mx = reduce<NW>(mx, red_max, MaxOp{});
+    keep_packed();
+    // exp(x - max).  Where a lane makes many of them and little else runs under them (1024 lanes, or exponentials made
+    // twice) as the hardware's 2^x on (x - max) * log2(e), the product formed by one fma: two instructions where the
+    // library's takes about twenty, and an error of the argument's rounding, |x - max| * 2^-24 relative (3e-6 at 50
+    // below the maximum, where the value is 2e-22).
+    const float l2e = 1.4426950408889634f, mxl = mx == NEG_INF ? 0.f : mx * l2e;
+    auto ex = [&](float v) {
+        if constexpr (BLOCK == 1024 || PACKED) return __builtin_amdgcn_exp2f(__builtin_fmaf(v, l2e, -mxl));
+        else return expf(v - mx);
+    };
+    x1 = ex(x1);
+    float sum = has1 ? x1 : 0.f;
+#pragma unroll
+    for (int v = 0; v < VPT; ++v) {
+        float s = 0.f;
+#pragma unroll
+        for (int q = 0; q < EV; ++q) {
+            const float e = ex(vget<T>(x[v], q));
+            if constexpr (!PACKED) vset<T>(x[v], q, e);
+            s += e;
+        }
+        sum += t + v * BLOCK < nv ? s : 0.f;
+    }
+    sum = reduce<NW>(sum, red_sum, SumOp{});
+    keep_packed();
+    // one correctly rounded reciprocal per column, then multiplies: within 1.5 ulp of the
+    // element-wise quotient, at a tenth of the instructions.  (16-bit results: 2^(x log2 e - log2(e^max sum)), which
+    // saves the multiply and differs far below their rounding.)
+    const float rsum = 1.0f / sum, shift = PACKED ? -(mxl + __builtin_amdgcn_logf(sum)) : 0.f;
+#pragma unroll
+    for (int v = 0; v < VPT; ++v) {
+        V y;
+#pragma unroll
+        for (int q = 0; q < EV; ++q) {
+            const float e = vget<T>(x[v], q);
+            vset<T>(y, q, PACKED ? __builtin_amdgcn_exp2f(__builtin_fmaf(e, l2e, shift)) : e * rsum);
+        }
+        const int i = t + v * BLOCK;
+        if (i < nv) st_vec<V>(y, op + head + i * EV);
+    }
+    if (has1) op[e1] = from_f32<T>(x1 * rsum);
 }
 
 // ---- three-pass kernel: any column length ---------------------------------------------
@@ -240,17 +283,13 @@ template <typename T, int BLOCK, int VPT>
 void launch_regs(const mi_tile_array* output, const mi_tile_array* input, int L, bool al,
                  hipStream_t s) {
     const int64_t M = input->sizes[1];
-    // The 1024-lane variants hold a CU's registers with one workgroup (two when a lane keeps 32 elements): a workgroup
-    // per CU slot walks the columns, so that the stores of one column, once issued, drain under the loads of the next.
-    const int64_t slots = 256 * (VPT * Raw<T>::EV <= 32 ? 2 : 1);
-    dim3 grid((unsigned)(BLOCK == 1024 && M > slots ? slots : M)), block(BLOCK);
-#define GO(AL, ST)                                                                              \
-    hipLaunchKernelGGL((softmax_regs_kernel<T, BLOCK, VPT, AL, ST>), grid, block, 0, s, (T*)output->ptr, \
-                       output->strides[1], (const T*)input->ptr, input->strides[1], L, M)
-    if (!al) GO(false, false);
-    else if (stream_hint(2 * M * (int64_t)L * (int64_t)sizeof(T))) GO(true, true);
-    else GO(true, false);
-#undef GO
+    dim3 grid((unsigned)M), block(BLOCK);
+    if (al && stream_hint(2 * M * (int64_t)L * (int64_t)sizeof(T)))
+        hipLaunchKernelGGL((softmax_regs_kernel<T, BLOCK, VPT, true>), grid, block, 0, s, (T*)output->ptr, output->strides[1],
+                           (const T*)input->ptr, input->strides[1], L);
+    else
+        hipLaunchKernelGGL((softmax_regs_kernel<T, BLOCK, VPT, false>), grid, block, 0, s, (T*)output->ptr, output->strides[1],
+                           (const T*)input->ptr, input->strides[1], L);
 }
 
 template <typename T>
@@ -283,10 +322,23 @@ int launch_len(const mi_tile_array* output, const mi_tile_array* input, int64_t 
     const bool al = vec_ok<T>(output, input);
     const int vecs = (int)cld(L, EV);
     if (vecs > 256 * 16) {
-        // Up to 65536 elements in the registers of 1024 lanes (64 per lane), one workgroup per CU: one pass over HBM
-        // where the three-pass kernel re-reads the column twice (1024 x 50257 fp32: 121 us).
-        if (L > 32768) { launch_regs<T, 1024, 64 / EV>(output, input, L, al, s); set_variant("softmax_regs_b1024_e64"); }
-        else { launch_regs<T, 1024, 32 / EV>(output, input, L, al, s); set_variant("softmax_regs_b1024_e32"); }
+        // Up to 65536 elements in the registers of 1024 lanes: one pass over HBM where the three-pass kernel re-reads the
+        // column twice (1024 x 50257 fp32: 121 us).  As many vectors per lane as the column needs: a lane past the end
+        // requests the last vector again, which costs an access all the same (2000 x 40000 bf16: 5 per lane 56.3 us, 8
+        // per lane 59.1).
+        const int per = (int)cld(vecs, 1024);
+#define WIDE(V) launch_regs<T, 1024, V>(output, input, L, al, s)
+        if (per <= 5) WIDE(5);
+        else if (per <= 6) WIDE(6);
+        else if (per <= 7) WIDE(7);
+        else if (per <= 8) WIDE(8);
+        if constexpr (EV == 4) {
+            if (per > 12) WIDE(16);
+            else if (per > 10) WIDE(12);
+            else if (per > 8) WIDE(10);
+        }
+#undef WIDE
+        set_variant(L > 32768 ? "softmax_regs_b1024_e64" : "softmax_regs_b1024_e32");
         return launch_status();
     }
     if (vecs <= 64) { launch_regs<T, 64, 1>(output, input, L, al, s); set_variant("softmax_regs_b64_v1"); }

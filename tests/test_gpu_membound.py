@@ -298,6 +298,30 @@ def test_softmax_columns_too_long_for_registers(ct, orc, M, N, T, variant):
             assert bool((ob[:, :oo] == 0).all()) and bool((ob[:, oo + N:] == 0).all())
 
 
+@pytest.mark.parametrize("T", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("N", [1, 3, 7, 8, 9, 23, 511, 513, 2049, 4097, 16383, 20481, 24577, 32769, 40961, 40969, 49153, 57343, 65535])
+def test_softmax_heads_tails_and_clamped_vectors(ct, orc, T, N):
+    """Columns that start 0 to 7 elements off a 16-byte boundary (odd leading dimensions), with input and output at the
+    same and at different offsets: every count of vectors per lane at its edges, columns shorter than a vector, and what
+    lies between the columns of the output untouched."""
+    rng = np.random.default_rng(N)
+    M = 9
+    x = torch.from_numpy((2 * rng.standard_normal((M, N))).astype(np.float32)).to(T).cuda()
+    for pad_in, off_in, pad_out, off_out in ((1, 0, 1, 0), (3, 2, 3, 2), (1, 0, 2, 1)):
+        src = torch.full((M, N + pad_in), float("nan"), dtype=T, device="cuda")
+        dst = torch.full((M, N + pad_out), 77.0, dtype=T, device="cuda")
+        src[:, off_in:off_in + N] = x
+        ct.softmax_tma_kernel(dst[:, off_out:off_out + N], src[:, off_in:off_in + N], 1 << max(N - 1, 0).bit_length())
+        ref = orc.softmax(orc.to_julia(x).astype(np.float64))
+        got = orc.to_julia(dst[:, off_out:off_out + N]).astype(np.float64)
+        # fp32: as close_f32 asks; 16 bits: one rounding of the result (2^-8 / 2^-11 of it, or the f16 subnormal step)
+        eps, tiny = {torch.float32: (1e-5, 0.0), torch.float16: (2.0 ** -11, 2.0 ** -24), torch.bfloat16: (2.0 ** -8, 0.0)}[T]
+        assert np.all(np.abs(got - ref) <= 1.01 * eps * ref + tiny), np.max(np.abs(got - ref) / ref)
+        keep = torch.ones(N + pad_out, dtype=torch.bool, device="cuda")
+        keep[off_out:off_out + N] = False
+        assert bool((dst[:, keep] == 77.0).all())
+
+
 def test_softmax_tile_smaller_than_column_and_padding(ct, orc):
     """A TILE_SIZE below N covers rows 1..TILE_SIZE only (softmax.jl:29-38); the chunked
     kernel walks cld(n_elems, TILE)*TILE rows, clipped to the array."""
