@@ -19,6 +19,7 @@ import os
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # MI355TILE_LIB selects another build of the same library (e.g. an experimental variant).
 LIB_PATH = os.environ.get("MI355TILE_LIB") or os.path.join(_HERE, "libmi355tile.so")
+NATIVE_PATH = os.path.join(_HERE, "_mi355tile_launch.so")
 
 MI_F32, MI_F64, MI_F16, MI_BF16, MI_F8E4M3FN, MI_I32, MI_I64, MI_BOOL, MI_I8, MI_I16, MI_F8E5M2 = range(11)
 MI_MAX_RANK = 4
@@ -101,11 +102,13 @@ _SIGNATURES = {
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)
 
 _lib = None
+_native = None    # the module of native launches (csrc/py/launch.cpp), bound to the loaded library
+_streams = False  # whether this process has looked a current stream up (which sets torch's GPU side up, or refuses to)
 
 
 def lib() -> ctypes.CDLL:
     """Load libmi355tile.so (built in-tree by ``__graft_entry__.build``).  Raises if absent."""
-    global _lib
+    global _lib, _native
     if _lib is None:
         if not os.path.exists(LIB_PATH):
             raise RuntimeError(
@@ -119,8 +122,29 @@ def lib() -> ctypes.CDLL:
             fn = getattr(cdll, name)  # AttributeError if the library lacks a declared symbol
             fn.argtypes = argtypes
             fn.restype = restype
+        _native = _load_native(cdll)
         _lib = cdll
     return _lib
+
+
+def _load_native(cdll):
+    if not os.path.exists(NATIVE_PATH):
+        raise RuntimeError(f"{NATIVE_PATH} is missing: it is built together with the library, see there")
+    import importlib.machinery
+    import importlib.util
+    loader = importlib.machinery.ExtensionFileLoader("_mi355tile_launch", NATIVE_PATH)
+    native = importlib.util.module_from_spec(importlib.util.spec_from_loader("_mi355tile_launch", loader))
+    loader.exec_module(native)
+    native.bind_library({name: ctypes.cast(getattr(cdll, name), ctypes.c_void_p).value for name in _SIGNATURES})
+    return native
+
+
+def _after_fork():
+    global _streams
+    _streams = False   # torch refuses the GPU to the child of a process that has used it: let the look-up say so
+
+
+os.register_at_fork(after_in_child=_after_fork)
 
 
 def strerror(code: int) -> str:
@@ -187,11 +211,27 @@ def _call(name: str, *args):
         raise MiError(name, rc, strerror(rc))
 
 
+def _launch(name: str, *args, stream=None):
+    """Entry point ``name`` with torch tensors for its arrays, on the current stream or on ``stream``.  The native module
+    converts plain tensors, ints and floats (a matmul call 11.5 us of host time by ctypes, 5.1 by it; LayerNorm's three calls and a fill 51 and 21); it
+    returns None, having called nothing, where anything else is among them, and ctypes then converts or refuses it."""
+    global _streams
+    if stream is None and _streams:
+        rc = getattr(_native, name)(*args, None)
+        if rc == 0:
+            return
+        if rc is not None:
+            raise MiError(name, rc, strerror(rc))
+    args = [_ref(a) if t is _A else a for t, a in zip(_SIGNATURES[name][0], args)]
+    handle = _stream(stream)
+    _streams = _streams or stream is None
+    _call(name, *args, handle)
+
+
 def fft_kernel(x_packed_in, y_packed_out, W0, W1, W2, T0, T1, N: int, F0: int, F1: int, F2: int, BS: int,
                D: int, stream=None):
     """examples/fft.jl:22-126"""
-    _call("mi_fft_kernel", _ref(x_packed_in), _ref(y_packed_out), _ref(W0), _ref(W1), _ref(W2), _ref(T0),
-          _ref(T1), N, F0, F1, F2, BS, D, _stream(stream))
+    _launch("mi_fft_kernel", x_packed_in, y_packed_out, W0, W1, W2, T0, T1, N, F0, F1, F2, BS, D, stream=stream)
 
 
 def bind(name: str, *args, stream=None):
@@ -216,32 +256,32 @@ def bind(name: str, *args, stream=None):
 
 def vec_add_kernel_1d(a, b, c, tile: int, stream=None):
     """examples/vadd.jl:10-17"""
-    _call("mi_vec_add_kernel_1d", _ref(a), _ref(b), _ref(c), tile, _stream(stream))
+    _launch("mi_vec_add_kernel_1d", a, b, c, tile, stream=stream)
 
 
 def vec_add_kernel_2d(a, b, c, tile_x: int, tile_y: int, stream=None):
     """examples/vadd.jl:20-28"""
-    _call("mi_vec_add_kernel_2d", _ref(a), _ref(b), _ref(c), tile_x, tile_y, _stream(stream))
+    _launch("mi_vec_add_kernel_2d", a, b, c, tile_x, tile_y, stream=stream)
 
 
 def vec_add_kernel_1d_gather(a, b, c, tile: int, stream=None):
     """examples/vadd.jl:31-45"""
-    _call("mi_vec_add_kernel_1d_gather", _ref(a), _ref(b), _ref(c), tile, _stream(stream))
+    _launch("mi_vec_add_kernel_1d_gather", a, b, c, tile, stream=stream)
 
 
 def transpose_kernel(x, y, tm: int, tn: int, stream=None):
     """examples/transpose.jl:11-19"""
-    _call("mi_transpose_kernel", _ref(x), _ref(y), tm, tn, _stream(stream))
+    _launch("mi_transpose_kernel", x, y, tm, tn, stream=stream)
 
 
 def matmul_kernel(A, B, C, tm: int, tn: int, tk: int, stream=None):
     """examples/matmul.jl:28-60"""
-    _call("mi_matmul_kernel", _ref(A), _ref(B), _ref(C), tm, tn, tk, _stream(stream))
+    _launch("mi_matmul_kernel", A, B, C, tm, tn, tk, stream=stream)
 
 
 def batch_matmul_kernel(A, B, C, tm: int, tn: int, tk: int, stream=None):
     """examples/batchmatmul.jl:15-56"""
-    _call("mi_batch_matmul_kernel", _ref(A), _ref(B), _ref(C), tm, tn, tk, _stream(stream))
+    _launch("mi_batch_matmul_kernel", A, B, C, tm, tn, tk, stream=stream)
 
 
 def swizzle_2d(M, N, tm, tn, GROUP_SIZE_M, bid):
@@ -253,36 +293,35 @@ def swizzle_2d(M, N, tm, tn, GROUP_SIZE_M, bid):
 
 def layer_norm_fwd(X, W, B, Y, Mean, Rstd, eps: float, TILE_N: int, stream=None):
     """examples/layernorm.jl:27-68"""
-    _call("mi_layer_norm_fwd", _ref(X), _ref(W), _ref(B), _ref(Y), _ref(Mean), _ref(Rstd),
-          ctypes.c_float(eps), TILE_N, _stream(stream))
+    _launch("mi_layer_norm_fwd", X, W, B, Y, Mean, Rstd, eps if type(eps) is float else ctypes.c_float(eps), TILE_N,
+            stream=stream)
 
 
 def layer_norm_bwd_dx_partial_dwdb(DX, DY, DW, DB, X, W, Mean, Rstd, Locks, GROUP_SIZE_M: int,
                                    TILE_N: int, stream=None):
     """examples/layernorm.jl:118-171"""
-    _call("mi_layer_norm_bwd_dx_partial_dwdb", _ref(DX), _ref(DY), _ref(DW), _ref(DB), _ref(X),
-          _ref(W), _ref(Mean), _ref(Rstd), _ref(Locks), GROUP_SIZE_M, TILE_N, _stream(stream))
+    _launch("mi_layer_norm_bwd_dx_partial_dwdb", DX, DY, DW, DB, X, W, Mean, Rstd, Locks, GROUP_SIZE_M, TILE_N,
+            stream=stream)
 
 
 def layer_norm_bwd_dwdb(DW, DB, FINAL_DW, FINAL_DB, TILE_M: int, TILE_N: int, stream=None):
     """examples/layernorm.jl:186-205"""
-    _call("mi_layer_norm_bwd_dwdb", _ref(DW), _ref(DB), _ref(FINAL_DW), _ref(FINAL_DB), TILE_M,
-          TILE_N, _stream(stream))
+    _launch("mi_layer_norm_bwd_dwdb", DW, DB, FINAL_DW, FINAL_DB, TILE_M, TILE_N, stream=stream)
 
 
 def layer_norm_bwd_static(DX, DY, X, W, Mean, Rstd, FINAL_DW, FINAL_DB, GROUP_SIZE_M: int, TILE_M: int,
                           TILE_N: int, stream=None):
     """The whole backward of examples/layernorm.jl:245-251 in one call that allocates nothing: the
     partial slots live in the library's static scratch (MiError with MI_E_SCRATCH beyond its size)."""
-    _call("mi_layer_norm_bwd_static", _ref(DX), _ref(DY), _ref(X), _ref(W), _ref(Mean), _ref(Rstd),
-          _ref(FINAL_DW), _ref(FINAL_DB), GROUP_SIZE_M, TILE_M, TILE_N, _stream(stream))
+    _launch("mi_layer_norm_bwd_static", DX, DY, X, W, Mean, Rstd, FINAL_DW, FINAL_DB, GROUP_SIZE_M, TILE_M, TILE_N,
+            stream=stream)
 
 
 def softmax_tma_kernel(output, input, TILE_SIZE: int, num_programs: int | None = None, stream=None):
     """examples/softmax.jl:18-42"""
     if num_programs is None:
         num_programs = max(1, min(input.shape[0] if input.dim() == 2 else 1, (1 << 24) - 1))
-    _call("mi_softmax_tma_kernel", _ref(output), _ref(input), TILE_SIZE, num_programs, _stream(stream))
+    _launch("mi_softmax_tma_kernel", output, input, TILE_SIZE, num_programs, stream=stream)
 
 
 def softmax_chunked_kernel(output, input, n_elems: int, TILE_SIZE: int,
@@ -290,16 +329,15 @@ def softmax_chunked_kernel(output, input, n_elems: int, TILE_SIZE: int,
     """examples/softmax.jl:48-100"""
     if num_programs is None:
         num_programs = max(1, min(input.shape[0] if input.dim() == 2 else 1, (1 << 24) - 1))
-    _call("mi_softmax_chunked_kernel", _ref(output), _ref(input), n_elems, TILE_SIZE, num_programs,
-          _stream(stream))
+    _launch("mi_softmax_chunked_kernel", output, input, n_elems, TILE_SIZE, num_programs, stream=stream)
 
 
 def fmha_kernel(Q, K, V, Out, qk_scale: float, input_pos: int, TILE_D: int, H: int, TILE_M: int,
                 TILE_N: int, QUERY_GROUP_SIZE: int, CAUSAL: bool, EVEN_K: bool, stream=None):
     """examples/fmha.jl:20-139"""
-    _call("mi_fmha_kernel", _ref(Q), _ref(K), _ref(V), _ref(Out), ctypes.c_float(qk_scale),
-          ctypes.c_int32(input_pos), TILE_D, H, TILE_M, TILE_N, QUERY_GROUP_SIZE, int(bool(CAUSAL)),
-          int(bool(EVEN_K)), _stream(stream))
+    _launch("mi_fmha_kernel", Q, K, V, Out, qk_scale if type(qk_scale) is float else ctypes.c_float(qk_scale),
+            input_pos if type(input_pos) is int else ctypes.c_int32(input_pos), TILE_D, H, TILE_M, TILE_N, QUERY_GROUP_SIZE,
+            int(bool(CAUSAL)), int(bool(EVEN_K)), stream=stream)
 
 
 def moe_align_tile_size(topk_ids, tile_m: int, num_experts: int):
@@ -344,11 +382,11 @@ def moe_align_tile_size_device(topk_ids, tile_m: int, num_experts: int, sorted_t
     if sorted_expert_ids is None:
         sorted_expert_ids = torch.empty(blocks, dtype=torch.int32, device=topk_ids.device)
     if clear is None:
-        _call("mi_moe_align_tile_size_device", _ref(topk_ids), tile_m, num_experts, _ref(sorted_token_ids),
-              _ref(sorted_expert_ids), _stream(stream))
+        _launch("mi_moe_align_tile_size_device", topk_ids, tile_m, num_experts, sorted_token_ids, sorted_expert_ids,
+                stream=stream)
     else:
-        _call("mi_moe_align_tile_size_device_clear", _ref(topk_ids), tile_m, num_experts, _ref(sorted_token_ids),
-              _ref(sorted_expert_ids), _ref(clear), _stream(stream))
+        _launch("mi_moe_align_tile_size_device_clear", topk_ids, tile_m, num_experts, sorted_token_ids,
+                sorted_expert_ids, clear, stream=stream)
     return sorted_token_ids, sorted_expert_ids
 
 
@@ -363,7 +401,7 @@ def moe_route_topk(logits, topk: int, weight_dtype=None, topk_weights=None, topk
         topk_weights = torch.empty((topk, num_tokens), dtype=weight_dtype or logits.dtype, device=logits.device)
     if topk_ids is None:
         topk_ids = torch.empty((topk, num_tokens), dtype=torch.int64, device=logits.device)
-    _call("mi_moe_route_topk", _ref(logits), _ref(topk_weights), _ref(topk_ids), _stream(stream))
+    _launch("mi_moe_route_topk", logits, topk_weights, topk_ids, stream=stream)
     return topk_weights, topk_ids
 
 
@@ -371,9 +409,8 @@ def fused_moe_kernel(A, B, C, topk_weights, sorted_token_ids, sorted_expert_ids,
                      num_token_replicas: int, mul_routed_weight: bool, TILE_M: int, TILE_N: int,
                      TILE_K: int, b_scale=None, stream=None):
     """examples/moe.jl:45-105 (``b_scale``: per-(n, expert) fp32 scales of fp8 weights)."""
-    _call("mi_fused_moe_kernel", _ref(A), _ref(B), _ref(C), _ref(topk_weights),
-          _ref(sorted_token_ids), _ref(sorted_expert_ids), num_token_replicas,
-          int(bool(mul_routed_weight)), TILE_M, TILE_N, TILE_K, _ref(b_scale), _stream(stream))
+    _launch("mi_fused_moe_kernel", A, B, C, topk_weights, sorted_token_ids, sorted_expert_ids, num_token_replicas,
+            int(bool(mul_routed_weight)), TILE_M, TILE_N, TILE_K, b_scale, stream=stream)
 
 
 def fused_moe_accumulate_kernel(A, B, Out, topk_weights, sorted_token_ids, sorted_expert_ids, TILE_M: int, TILE_N: int,
@@ -383,8 +420,8 @@ def fused_moe_accumulate_kernel(A, B, Out, topk_weights, sorted_token_ids, sorte
     replica's weighted row, rounded to the storage type as cache3 would hold it, by memory-side packed atomic adds.
     top-k of 1 or 2 only (two terms add up the same in either order), ``topk_weights`` as the (num_tokens, topk)
     matrix, N even."""
-    _call("mi_fused_moe_accumulate_kernel", _ref(A), _ref(B), _ref(Out), _ref(topk_weights), _ref(sorted_token_ids),
-          _ref(sorted_expert_ids), TILE_M, TILE_N, TILE_K, _ref(b_scale), _stream(stream))
+    _launch("mi_fused_moe_accumulate_kernel", A, B, Out, topk_weights, sorted_token_ids, sorted_expert_ids, TILE_M,
+            TILE_N, TILE_K, b_scale, stream=stream)
 
 
 def fused_moe_silu_kernel(A, B, C, topk_weights, sorted_token_ids, sorted_expert_ids,
@@ -392,14 +429,13 @@ def fused_moe_silu_kernel(A, B, C, topk_weights, sorted_token_ids, sorted_expert
                           TILE_K: int, b_scale=None, stream=None):
     """fused_moe_kernel (moe.jl:45-105) on the gate / up projection with silu_and_mul_kernel
     (moe.jl:110-128) as its epilogue: ``C`` is (N/2, total_tokens)."""
-    _call("mi_fused_moe_silu_kernel", _ref(A), _ref(B), _ref(C), _ref(topk_weights),
-          _ref(sorted_token_ids), _ref(sorted_expert_ids), num_token_replicas,
-          int(bool(mul_routed_weight)), TILE_M, TILE_N, TILE_K, _ref(b_scale), _stream(stream))
+    _launch("mi_fused_moe_silu_kernel", A, B, C, topk_weights, sorted_token_ids, sorted_expert_ids, num_token_replicas,
+            int(bool(mul_routed_weight)), TILE_M, TILE_N, TILE_K, b_scale, stream=stream)
 
 
 def silu_and_mul_kernel(A, B, C, TILE_N: int, stream=None):
     """examples/moe.jl:110-128"""
-    _call("mi_silu_and_mul_kernel", _ref(A), _ref(B), _ref(C), TILE_N, _stream(stream))
+    _launch("mi_silu_and_mul_kernel", A, B, C, TILE_N, stream=stream)
 
 
 def quantize_e4m3fn(x, codes=None, scale=None, workspace=None, stream=None, fold=None, fold_out=None):
@@ -416,13 +452,12 @@ def quantize_e4m3fn(x, codes=None, scale=None, workspace=None, stream=None, fold
     if fold is not None:
         if fold_out is None:
             fold_out = torch.empty_like(fold)
-        _call("mi_quantize_e4m3fn_fold", _ref(x), _ref(codes), _ref(scale), _ref(workspace), _ref(fold), _ref(fold_out),
-              _stream(stream))
+        _launch("mi_quantize_e4m3fn_fold", x, codes, scale, workspace, fold, fold_out, stream=stream)
         return codes, scale, fold_out
-    _call("mi_quantize_e4m3fn", _ref(x), _ref(codes), _ref(scale), _ref(workspace), _stream(stream))
+    _launch("mi_quantize_e4m3fn", x, codes, scale, workspace, stream=stream)
     return codes, scale
 
 
 def moe_sum_topk(inp, out, stream=None):
     """The ``sum(cache3; dims=2)`` of examples/moe.jl:256."""
-    _call("mi_moe_sum_topk", _ref(inp), _ref(out), _stream(stream))
+    _launch("mi_moe_sum_topk", inp, out, stream=stream)
