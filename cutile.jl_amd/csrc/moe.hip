@@ -106,9 +106,11 @@ __device__ __forceinline__ void lds_barrier() {
 // E: activation/output element traits; W8: weights are E4M3FN bytes (else same type as A).
 // NTW: waves side by side along n (workgroup strip = 32*NTW channels); the other 4/NTW waves
 // split each K step between them and their accumulators are added through LDS at the end.
-// kKT: K step.  Two shapes are used: (NTW=4, kKT=128) when N is large enough to give every CU
-// several strips, and (NTW=1, kKT=256) for small N, where 32-channel strips with a 4-way
-// in-workgroup K split keep ~4x more workgroups (and bytes) in flight.
+// kKT: K step.  Three shapes are used: (NTW=4, kKT=128) when N is large enough to give every CU
+// several strips, (NTW=1, kKT=256) for small N, where 32-channel strips with a 4-way
+// in-workgroup K split keep ~4x more workgroups (and bytes) in flight, and (NTW=2, kKT=256) for
+// e4m3 weights between the two: a K step of a 32-channel strip moves 8 KB of e4m3 weights and 16 KB
+// of activations, a strip of 64 channels 16 KB of each (see the launch).
 // Workgroup = (one tile of up to 32 consecutive sorted slots, one strip of 32*NTW channels).
 // With ~16 tokens per expert most 32-slot tiles of a TILE_M block hold only padding; their
 // workgroups leave at once, so the expert's weight strip is streamed by exactly as many
@@ -292,9 +294,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TS == 1 ? 4
     // that run at the same time would otherwise all read the same few hundred bytes of every weight row
     // at the same moment, i.e. the same slice of every 4 KB of address space.
     const int nsteps = (K + kKT - 1) / kKT;
-    // (the narrow shape only: 27.9 against 29.5 us there, 49 against 45 us on the wide shape)
+    // (the narrow shapes only: 27.9 against 29.5 us there, 49 against 45 us on the wide shape)
     const unsigned rot_seed = (unsigned)(3 * expert + grp);
-    const int rot = NTW != 1 ? 0 : (nsteps & (nsteps - 1)) == 0 ? (int)(rot_seed & (unsigned)(nsteps - 1)) : (int)(rot_seed % (unsigned)nsteps);   // (not a function of the strip: the fused-SiLU and the plain kernel then add in the same order)
+    const int rot = NTW == 4 ? 0 : (nsteps & (nsteps - 1)) == 0 ? (int)(rot_seed & (unsigned)(nsteps - 1)) : (int)(rot_seed % (unsigned)nsteps);   // (not a function of the strip: the fused-SiLU and the plain kernel then add in the same order)
     auto k_of = [&](int it) {
         int st = it + rot;
         if (st >= nsteps) st -= nsteps;
@@ -650,7 +652,14 @@ static int fused_moe_impl(const mi_tile_array* A, const mi_tile_array* B, const 
     // wide shape its workgroups, and a weight strip is streamed once per 64 tokens.
     const bool dense = tile_slots == kTT && (TILE_M / kTT) % 2 == 0 && total >= (int64_t)kTT * E;
     const bool narrow = !silu && !dense && m_blocks * cld(N, (int64_t)128) < 768 && K >= 512;
-    const int n_blocks = silu ? (int)cld(N / 2, (int64_t)64) : (int)cld(N, (int64_t)(narrow ? 32 : 128));
+    // 64-channel strips for e4m3 weights: half the activation traffic, which outweighs the weights' with 32 channels, at
+    // half the workgroups -- where those still come to two per CU.  Whole cutile_moe, 32 -> 64 channels (1024 hidden, 2048
+    // inter, top-2): 256 tokens 32 experts 53.4 -> 52.3 us, 400 tokens 62.9 -> 58.8, 256 tokens 64 experts 91.4 -> 83.4; but
+    // 100 tokens 8 experts (128 strips) 30.7 -> 31.9 and 16 tokens 32 experts (20 of them hit) 37.3 -> 39.2.  A K that ends
+    // in a partial step: 44.1 -> 44.4 (1408).  With 16-bit weights the two differ by 1-2 % either way.
+    const bool pair = narrow && w8 && K % 256 == 0 && E * cld(N, (int64_t)64) >= 512 && total >= 2 * E;
+    const int strip = pair ? 64 : narrow ? 32 : 128;
+    const int n_blocks = silu ? (int)cld(N / 2, (int64_t)64) : (int)cld(N, (int64_t)strip);
     // (Two tiles per workgroup cover 64 tokens; with that many per expert on average every second expert has a
     // third tile, whose workgroup streams the expert's weights once more.  A variant that takes the whole 128-slot
     // block per workgroup reads every weight once and is no faster -- 69 against 66 us for the gate / up projection
@@ -665,7 +674,7 @@ static int fused_moe_impl(const mi_tile_array* A, const mi_tile_array* B, const 
     // every tile of the launch inside the arrays and 16-byte aligned: the kernels without load predicates
     // (a K step of 512 for the e4m3 down projection, whose steps move half the weight bytes: 29.8 us against 20.4)
     const int kt = narrow ? 256 : 128;
-    const bool fast = vecA && vecB && K % kt == 0 && (silu ? (N / 2) % 64 == 0 : N % (narrow ? 32 : 128) == 0);
+    const bool fast = vecA && vecB && K % kt == 0 && (silu ? (N / 2) % 64 == 0 : N % strip == 0);
 #define LAUNCH(ET, W8, NTW, KT, SILU, TS)                                                                           \
     do {                                                                                                            \
         if (fast) LAUNCH1(ET, W8, NTW, KT, SILU, TS, true);                                                         \
@@ -679,13 +688,14 @@ static int fused_moe_impl(const mi_tile_array* A, const mi_tile_array* B, const 
                        w8 ? (const float*)b_scale->ptr : nullptr, w8 ? b_scale->strides[1] : 0, (int)K, (int)N,     \
                        (int)E, num_token_replicas, mul_routed_weight != 0, TILE_M, tile_slots, n_blocks, vecA, vecB,     \
                        (int)w_topk, w2d ? topk_weights->strides[0] : (int64_t)1, w2d ? topk_weights->strides[1] : (int64_t)0, acc_shift)
-#define LAUNCH_SHAPE(ET, W8)                                  \
-    do {                                                      \
-        if (silu && ts == 2) LAUNCH(ET, W8, 4, 128, true, 2); \
-        else if (silu) LAUNCH(ET, W8, 4, 128, true, 1);       \
-        else if (narrow) LAUNCH(ET, W8, 1, 256, false, 1);    \
-        else if (ts == 2) LAUNCH(ET, W8, 4, 128, false, 2);   \
-        else LAUNCH(ET, W8, 4, 128, false, 1);                \
+#define LAUNCH_SHAPE(ET, W8)                                    \
+    do {                                                        \
+        if (silu && ts == 2) LAUNCH(ET, W8, 4, 128, true, 2);   \
+        else if (silu) LAUNCH(ET, W8, 4, 128, true, 1);         \
+        else if (pair) LAUNCH(ET, true, 2, 256, false, 1);      \
+        else if (narrow) LAUNCH(ET, W8, 1, 256, false, 1);      \
+        else if (ts == 2) LAUNCH(ET, W8, 4, 128, false, 2);     \
+        else LAUNCH(ET, W8, 4, 128, false, 1);                  \
     } while (0)
     if (A->dtype == MI_F16) {
         if (w8) LAUNCH_SHAPE(F16, true);
@@ -699,6 +709,7 @@ static int fused_moe_impl(const mi_tile_array* A, const mi_tile_array* B, const 
 #undef LAUNCH1
     if (silu && ts == 2) set_variant(w8 ? "fused_moe_silu_t64_n64x2_k128_w8a16" : "fused_moe_silu_t64_n64x2_k128");
     else if (silu) set_variant(w8 ? "fused_moe_silu_t32_n64x2_k128_w8a16" : "fused_moe_silu_t32_n64x2_k128");
+    else if (pair) set_variant("fused_moe_t32_n64_k256_ksplit2_w8a16");
     else if (narrow) set_variant(w8 ? "fused_moe_t32_n32_k256_ksplit4_w8a16" : "fused_moe_t32_n32_k256_ksplit4");
     else if (ts == 2) set_variant(w8 ? "fused_moe_t64_n128_k128_w8a16" : "fused_moe_t64_n128_k128");
     else set_variant(w8 ? "fused_moe_t32_n128_k128_w8a16" : "fused_moe_t32_n128_k128");

@@ -156,6 +156,50 @@ def test_moe_fp8_weights(orc):
     check(J(out), ref)
 
 
+@pytest.mark.parametrize("tokens,E,K,N,dtype,accumulate", [
+    (100, 64, 512, 480, torch.float16, False),    # 7.5 strips of 64 channels, two K steps (the fewest)
+    (64, 32, 768, 1024, torch.bfloat16, True),    # 512 strips in all and two replicas per expert: the smallest of the range
+    (511, 32, 2048, 1024, torch.float16, True),   # almost 32 replicas per expert, most of them two tiles
+    (65, 33, 512, 1022, torch.float16, False),    # a last strip of 62 channels
+])
+def test_e4m3_weights_in_strips_of_64_channels(ct, orc, tokens, E, K, N, dtype, accumulate):
+    """One grouped GEMM against float64 dot products over the dequantised weights.  The products of f16 / bf16 and e4m3
+    are exact in fp32, so a result is off by its sum's roundings (K * 2^-24 of the sum of magnitudes at most) and its
+    own rounding to the storage type (2^-11 / 2^-8 of it, once per addend where replicas are added)."""
+    g = torch.Generator(device="cuda").manual_seed(tokens)
+    A = torch.randn(tokens, K, device="cuda", generator=g).to(dtype)
+    W = torch.randn(E, N, K, device="cuda", generator=g).to(torch.float8_e4m3fn)
+    scale = torch.rand(E, N, device="cuda", generator=g) * 0.1 + 0.05
+    ids = torch.argsort(torch.rand(tokens, E, device="cuda", generator=g), dim=1)[:, :2].t().contiguous() + 1   # (2, tokens)
+    w = torch.rand(2, tokens, device="cuda", generator=g).to(dtype)
+    tok, exp = ct.moe_align_tile_size_device(ids, 128, E)
+    ref, mag = [], []
+    for k in range(2):
+        r, m = torch.empty(tokens, N, dtype=torch.float64, device="cuda"), torch.empty(tokens, N, dtype=torch.float64, device="cuda")
+        for t in range(tokens):
+            x = A[t].double() * W[ids[k, t] - 1].double()
+            f = scale[ids[k, t] - 1].double()
+            r[t], m[t] = x.sum(dim=1) * f, x.abs().sum(dim=1) * f
+        ref.append(r * w[k].double()[:, None])
+        mag.append(m * w[k].double()[:, None])
+    eps = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
+    if accumulate:
+        # (replica r of token t belongs to column t: A's rows, one per token and slot)
+        A2 = A.repeat_interleave(2, dim=0)
+        out = torch.zeros(tokens, N, dtype=dtype, device="cuda")
+        ct.fused_moe_accumulate_kernel(A2, W, out, w, tok, exp, 128, 128, 64, b_scale=scale)
+        r, m = ref[0] + ref[1], mag[0] + mag[1]
+        bound = (K + 2) * 2.0 ** -24 * m + 2 * eps * (ref[0].abs() + ref[1].abs()) + 2.0 ** -23
+    else:
+        out = torch.full((tokens * 2, N), float("nan"), dtype=dtype, device="cuda")
+        ct.fused_moe_kernel(A, W, out, w, tok, exp, 2, True, 128, 128, 64, b_scale=scale)
+        r, m = torch.stack(ref, dim=1).reshape(tokens * 2, N), torch.stack(mag, dim=1).reshape(tokens * 2, N)
+        bound = (K + 2) * 2.0 ** -24 * m + 1.01 * eps * r.abs() + 2.0 ** -23
+    assert ct.last_variant() == "fused_moe_t32_n64_k256_ksplit2_w8a16"
+    err = (out.double() - r).abs()
+    assert bool((err <= bound).all()), float((err / bound).max())
+
+
 def test_fp8_dequant_covers_every_code(ct, orc):
     """Every finite E4M3FN code as a weight: K = 256 codes against a one-hot activation picks
     each dequantised value out exactly (checks subnormals, signs and the exponent rebias)."""
