@@ -84,6 +84,25 @@ __device__ __forceinline__ float reduce(float v, float* red, Op op) {
     return v;
 }
 
+// exp(x - max) as the hardware's 2^x on (x - max) * log2(e), the product formed by one fma: an error of the argument's
+// rounding, |x - max| * 2^-24 relative (3e-6 at 50 below the maximum, where the value is 2e-22).  The rounding of
+// max * log2(e) is a factor that every element and their sum share; it is a power of two of at most 1/16 while |max| is
+// below 2^20.  A larger maximum (a mask value, an offset) is subtracted first, or that factor would overflow.  The
+// subtraction in every column and the multiply by 1 / sum, where 16-bit results once took 2^(x log2 e - (max log2 e +
+// log2 sum)) -- off by the rounding of max log2 e, a factor of 2^31 at -1e9 --, cost 1 us of 40 (bf16 1024 x 50257).  (Two
+// copies of what follows the maximum, one without the subtraction, spill: 48 us.)  Values below 2^-126 come out as 0.
+struct Exp2 {
+    float base, shift;
+    __device__ __forceinline__ explicit Exp2(float mx) {
+        base = fabsf(mx) <= 0x1p20f ? 0.f : mx;   // (an infinite maximum makes the whole column NaN, as x - max does)
+        shift = (mx - base) * kLog2e;
+    }
+    __device__ __forceinline__ float operator()(float x) const {
+        return __builtin_amdgcn_exp2f(__builtin_fmaf(x - base, kLog2e, -shift));
+    }
+    static constexpr float kLog2e = 1.4426950408889634f;
+};
+
 // ---- single-tile kernel: column cached in registers -----------------------------------
 // Capacity BLOCK*VPT*EV elements.  A column is a scalar head up to its first 16-byte boundary, whole vectors, and a scalar
 // tail; head and tail are one element in each of the first lanes.  (Where input and output do not sit at the same
@@ -95,7 +114,7 @@ __device__ __forceinline__ float reduce(float v, float* red, Op op) {
 //   - 16-bit columns stay packed in the registers and their exponentials are made twice, for the sum and for the result:
 //     at 1024 lanes a column of 65536 takes 32 of a lane's 64 registers, so two workgroups share a CU;
 // Before / now, in three rotating buffers: bf16 1024 x 50257 57 -> 41 us (5.0 TB/s), 4096 x 32768 239 -> 93, 1682 x 28672
-// 102 -> 34; f16 2048 x 8191 18.6 -> 12.0, 4096 x 4096 13.2 -> 11.1; fp32 1024 x 50257 91 -> 83, 3000 x 20000 93 -> 81.
+// 102 -> 35; f16 2048 x 8191 18.7 -> 11.7, 4096 x 4096 13.1 -> 11.3; fp32 1024 x 50257 92 -> 85, 3000 x 20000 93 -> 82.
 // Workgroups that walk the columns and request the next one while they store were no faster (1024 lanes, fp32
 // 4096 x 32768: 190 us against 179 with a workgroup per column).
 template <typename T, int BLOCK, int VPT, bool STREAM>
@@ -146,13 +165,11 @@ __global__ __launch_bounds__(BLOCK, BLOCK == 1024 && VPT <= 8 ? 8 : 1) void soft
         for (int q = 0; q < EV; ++q) mx = fmaxf(mx, vget<T>(x[v], q));
     mx = reduce<NW>(mx, red_max, MaxOp{});
     keep_packed();
-    // exp(x - max).  Where a lane makes many of them and little else runs under them (1024 lanes, or exponentials made
-    // twice) as the hardware's 2^x on (x - max) * log2(e), the product formed by one fma: two instructions where the
-    // library's takes about twenty, and an error of the argument's rounding, |x - max| * 2^-24 relative (3e-6 at 50
-    // below the maximum, where the value is 2e-22).
-    const float l2e = 1.4426950408889634f, mxl = mx == NEG_INF ? 0.f : mx * l2e;
+    // exp(x - max): where a lane makes many of them and little else runs under them (1024 lanes, or exponentials made
+    // twice) by Exp2, three instructions where the library's takes about twenty.
+    const Exp2 ex2(mx);
     auto ex = [&](float v) {
-        if constexpr (BLOCK == 1024 || PACKED) return __builtin_amdgcn_exp2f(__builtin_fmaf(v, l2e, -mxl));
+        if constexpr (BLOCK == 1024 || PACKED) return ex2(v);
         else return expf(v - mx);
     };
     x1 = ex(x1);
@@ -171,16 +188,15 @@ __global__ __launch_bounds__(BLOCK, BLOCK == 1024 && VPT <= 8 ? 8 : 1) void soft
     sum = reduce<NW>(sum, red_sum, SumOp{});
     keep_packed();
     // one correctly rounded reciprocal per column, then multiplies: within 1.5 ulp of the
-    // element-wise quotient, at a tenth of the instructions.  (16-bit results: 2^(x log2 e - log2(e^max sum)), which
-    // saves the multiply and differs far below their rounding.)
-    const float rsum = 1.0f / sum, shift = PACKED ? -(mxl + __builtin_amdgcn_logf(sum)) : 0.f;
+    // element-wise quotient, at a tenth of the instructions
+    const float rsum = 1.0f / sum;
 #pragma unroll
     for (int v = 0; v < VPT; ++v) {
         V y;
 #pragma unroll
         for (int q = 0; q < EV; ++q) {
             const float e = vget<T>(x[v], q);
-            vset<T>(y, q, PACKED ? __builtin_amdgcn_exp2f(__builtin_fmaf(e, l2e, shift)) : e * rsum);
+            vset<T>(y, q, (PACKED ? ex(e) : e) * rsum);
         }
         const int i = t + v * BLOCK;
         if (i < nv) st_vec<V>(y, op + head + i * EV);

@@ -322,6 +322,39 @@ def test_softmax_heads_tails_and_clamped_vectors(ct, orc, T, N):
         assert bool((dst[:, keep] == 77.0).all())
 
 
+@pytest.mark.parametrize("T", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("N", [500, 1999, 9001, 32768, 40007])
+def test_softmax_maxima_far_from_zero(ct, orc, T, N):
+    """Columns whose largest element is a mask value, the type's lowest or highest, or a large offset, in every kernel
+    (one wave, 256 and 1024 lanes): each element within one rounding of float64, head and tail included,
+    and columns of -Inf, with a +Inf or with a NaN are NaN as the formula makes them."""
+    lim = torch.finfo(T)
+    noise = torch.from_numpy(np.random.default_rng(N).standard_normal(N).astype(np.float32))
+    big = 6e4 if T == torch.float16 else 1e9
+    one = torch.full((N,), lim.min)
+    one[N // 3], one[N - 1] = 1.5, 0.25
+    ninf = torch.full((N,), -np.inf)
+    ninf[2] = -3.0
+    ends = torch.full((N,), lim.min)
+    ends[::2] = lim.max
+    cols = [torch.full((N,), v) for v in (-big, big, lim.min, lim.max, 1024.0)] + \
+           [noise * 8 + v for v in (1e4, -3e4, 6e4 if T == torch.float16 else 1e6)] + [noise * big / 8, one, ninf, ends]
+    nan = [torch.full((N,), -np.inf), noise.clone(), noise.clone()]
+    nan[1][N - 2], nan[2][1] = np.inf, np.nan
+    x = torch.stack(cols + nan).to(T).cuda()
+    src = torch.zeros(x.shape[0], N + 3, dtype=T, device="cuda")[:, 2:N + 2]
+    dst = torch.full((x.shape[0], N + 3), 7.0, dtype=T, device="cuda")[:, 2:N + 2]
+    src.copy_(x)
+    ct.softmax_tma_kernel(dst, src, 1 << (N - 1).bit_length())
+    got = dst.double().cpu().numpy()
+    assert np.isnan(got[len(cols):]).all()
+    ref = torch.softmax(x[:len(cols)].double(), dim=1).cpu().numpy()
+    # fp32: as close_f32 asks; 16 bits: one rounding of the result; below the type's normal range one of its steps
+    eps, tiny = {torch.float32: (1e-5, 2.0 ** -126), torch.float16: (2.0 ** -11, 2.0 ** -24), torch.bfloat16: (2.0 ** -8, 2.0 ** -126)}[T]
+    err = np.abs(got[:len(cols)] - ref) - (1.01 * eps * ref + tiny)
+    assert (err <= 0).all(), [i for i in range(len(cols)) if not (err[i] <= 0).all()]
+
+
 def test_softmax_tile_smaller_than_column_and_padding(ct, orc):
     """A TILE_SIZE below N covers rows 1..TILE_SIZE only (softmax.jl:29-38); the chunked
     kernel walks cld(n_elems, TILE)*TILE rows, clipped to the array."""
