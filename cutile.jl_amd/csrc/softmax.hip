@@ -247,10 +247,8 @@ __global__ __launch_bounds__(BLOCK) void softmax_3pass_kernel(T* __restrict__ ou
         }
         for (int64_t e = threadIdx.x; e < nscalar; e += BLOCK) mx = fmaxf(mx, to_f32<T>(ip[at(e)]));
         mx = block_reduce<NW>(mx, red, MaxOp{}, NEG_INF);
-        // exp(x - max) as the hardware's 2^x of one fma (see the 1024-lane register kernel): a column this long is
-        // walked by one workgroup per CU, and the library exponential was most of passes 2 and 3
-        const float l2e = 1.4426950408889634f, mxl = mx == NEG_INF ? 0.f : mx * l2e;
-        auto ex = [&](float v) { return __builtin_amdgcn_exp2f(__builtin_fmaf(v, l2e, -mxl)); };
+        // (a column this long is walked by one workgroup per CU: the library exponential was most of passes 2 and 3)
+        const Exp2 ex(mx);
         // pass 2: per-lane partial denominators, one reduction at the end
         float den = 0.f;
 #pragma unroll 4

@@ -323,10 +323,10 @@ def test_softmax_heads_tails_and_clamped_vectors(ct, orc, T, N):
 
 
 @pytest.mark.parametrize("T", [torch.float32, torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("N", [500, 1999, 9001, 32768, 40007])
+@pytest.mark.parametrize("N", [500, 1999, 9001, 32768, 40007, 70001])
 def test_softmax_maxima_far_from_zero(ct, orc, T, N):
     """Columns whose largest element is a mask value, the type's lowest or highest, or a large offset, in every kernel
-    (one wave, 256 and 1024 lanes): each element within one rounding of float64, head and tail included,
+    (one wave, 256 and 1024 lanes, three passes): each element within one rounding of float64, head and tail included,
     and columns of -Inf, with a +Inf or with a NaN are NaN as the formula makes them."""
     lim = torch.finfo(T)
     noise = torch.from_numpy(np.random.default_rng(N).standard_normal(N).astype(np.float32))
