@@ -16,14 +16,18 @@
 // K and V travel through two rings of four 8 KB LDS slots filled by direct global->LDS loads three steps ahead.  The loop
 // over unmasked halves is unrolled by four so that ring slots are immediate offsets.
 //
-// Measured (2 x 32 heads in groups of 4, S = 2048, bf16): causal 117 -> 72 us (0.59 -> 0.95 PFLOP/s), not causal 151 -> 121 us
-// (0.91 -> 1.13), S = 2000 causal 114 -> 72 us.  In the long walk the matrix pipes are 55 % busy at 1.92 GHz, which is the
-// MFMA rate at which the power limit also stops the 4096^3 GEMM (77 % at 1.43 GHz): one barrier per two halves, four waves
-// per K / V ring (256 queries) and row sums by the matrix cores (ones times P: 40 instructions less per step, 4 MFMAs
-// more, 131 us) were tried and did not help.  Causal pays for its diagonals and for the last, unequal workgroups.
+// The running maximum is the true one at every half, as in the general kernel: the row's largest weight is exactly 1, and
+// the weights' rounding costs no more than there (error against float64, 2 x 32 heads, S = 2000 causal bf16: 1.746e-3 of the
+// result, the general kernel 1.756e-3).  A stream's sums are rescaled when any of its 32 rows has a new maximum, which is
+// most halves: 64 multiplies that nothing hides, a fifth of the time in all.  Raising only what had outgrown its maximum
+// by 2^8 (P in (0, 2^8]) took 75 instead of 86 us and was off by 1.831e-3 (scores of three times the spread: 2.15e-3
+// against 1.75e-3); the multiplies spread over slots 0..15 behind a branch each took 91 us.  Scores are scaled in fp32.
 //
-// The running maximum is raised only when a row outgrows it by 2^8 (as in fmha_pipe.hip: P stays in (0, 2^8] of the
-// storage type, same function of the inputs).  Scores are scaled in fp32.
+// Measured (2 x 32 heads in groups of 4, bf16, against the general kernel): S = 2048 causal 120 -> 86 us (0.57 -> 0.80
+// PFLOP/s), not causal 153 -> 142 us (0.90 -> 0.97), S = 2000 causal 117 -> 87 us.  What bounds it is the issue of one wave per
+// SIMD: one barrier per two halves, four waves per K / V ring (256 queries) and row sums by the matrix cores (ones times P:
+// 40 instructions less per step, 4 MFMAs more) were tried and did not help.  Causal pays for its diagonals and for the
+// last, unequal workgroups.
 #include "fmha_common.h"
 
 #include <utility>
@@ -42,7 +46,6 @@ constexpr int kDT = kD / 32;      // 32-channel tiles of the output
 constexpr int T = kSlotBytes / 1024 / NW;   // 1 KB transfers per wave and half, for K and for V each
 constexpr int KO = 2;             // distinct K lane offsets: transfers 16 keys apart share theirs
 constexpr int kPre = 1;           // the slot that waits for the transfers and for the other waves
-constexpr float kRaise = 8.0f;
 
 // f(0), f(1), ... f(N - 1) with the argument a constant: the slots of a step are laid out at compile time.
 template <typename F, int... I>
@@ -82,8 +85,8 @@ struct Acc {
     s16x8 qf[2][kKS];
     f32x16 o[2][kDT];
     float l[2];         // row sums of the weights over the lane's half of the keys
-    float m[2];         // running maximum (exp2 domain)
-    float thr[2];       // raw score above which m is raised
+    float top[2];       // running maximum
+    float m[2];         // the same, scaled (exp2 domain)
 };
 
 // Transfer d = 0 .. 2T-1 of a half's worth: d < T is transfer d of the next K half, the others of the next V half.  The
@@ -177,11 +180,12 @@ template <typename E, bool NEXT, bool MASK, int SLOT>
 __device__ __forceinline__ void step(const unsigned short* Ks, const unsigned short* Vs, Lane& c, Acc& a, int j, float scale2,
                                      f32x16 (&s_cur)[2], f32x16 (&s_next)[2], s16x8 (&kf)[kKS], float (&cand)[2]) {
     const int s0 = SLOT >= 0 ? SLOT : j & 3;
-    // ---- raise the running maxima if some row outgrew its own by 2^kRaise (every row sees key 0 in the first half) ----
-    if (__builtin_expect(__any(cand[0] > a.thr[0] || cand[1] > a.thr[1]), 0)) {
+    // ---- raise the running maxima of a stream if some row has a new one (every row sees key 0 in the first half) ----
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            const float m_new = fmaxf(a.m[q], xhalf_max(cand[q]) * scale2);
+    for (int q = 0; q < 2; ++q) {
+        if (__any(cand[q] > a.top[q])) {
+            a.top[q] = fmaxf(a.top[q], xhalf_max(cand[q]));
+            const float m_new = a.top[q] * scale2;
             const float alpha = __builtin_amdgcn_exp2f(a.m[q] - m_new);   // (0 at the first half: l and O are zero)
             a.l[q] *= alpha;
 #pragma unroll
@@ -189,7 +193,6 @@ __device__ __forceinline__ void step(const unsigned short* Ks, const unsigned sh
 #pragma unroll
                 for (int r = 0; r < 16; ++r) a.o[q][dt][r] *= alpha;
             a.m[q] = m_new;
-            a.thr[q] = (m_new + kRaise) * __builtin_amdgcn_rcpf(scale2);
         }
     }
     pin(a);
@@ -392,7 +395,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
 #pragma unroll
         for (int dt = 0; dt < kDT; ++dt) a.o[q][dt] = f32x16{0};
         a.l[q] = 0.f;
-        a.m[q] = a.thr[q] = -INFINITY;
+        a.m[q] = a.top[q] = -INFINITY;
     }
 
     // ---- prologue: S(0), its row maxima, the K(1) fragments -----------------------------------------------------

@@ -192,6 +192,29 @@ def test_fmha_pipelined_kernel_for_heads_of_128(ct, orc, batch, heads, sq, skv, 
     check(orc, out, ref, 2e-2 if T == torch.float16 else 3e-2)
 
 
+@pytest.mark.parametrize("causal", [False, True])
+def test_fmha_heads_of_128_the_largest_weight_is_not_rounded(ct, causal):
+    """Rows whose score rises once, from key 5 to key 200, by 0.2 to 8 powers of two, with a value at key 200 alone: the
+    result is that value times 1 / (1 + 2^-rise).  With the weights relative to the row's true maximum the larger one
+    is exactly 1 and nothing is rounded but the result (2^-8 of it; the rest of the bound is for fp32)."""
+    S, D = 256, 128
+    Q = torch.zeros(1, 8, S, D, dtype=torch.bfloat16, device="cuda")
+    Q[..., 0] = 1
+    Q[:, :, 200:, 1] = torch.linspace(1, 29, S - 200, device="cuda").to(torch.bfloat16)
+    K = torch.zeros(1, 8, S, D, dtype=torch.bfloat16, device="cuda")
+    K[:, :, 5, 0], K[:, :, 200, 0], K[:, :, 200, 1] = 64, 64, 0.1875
+    V = torch.zeros(1, 8, S, D, dtype=torch.bfloat16, device="cuda")
+    V[:, :, 200] = torch.randn(1, 8, D, device="cuda").to(torch.bfloat16)
+    out = fmha.cutile_fmha(Q, K, V, causal=causal, qk_scale=1.0)[:, :, 200:].double()
+    assert ct.last_variant() == "fmha_pipe_d128_q128_kv32_ring4"
+    s = Q[0, 0, 200:].double() @ K[0, 0].double().t().contiguous()
+    if causal:
+        s = s.masked_fill(torch.arange(S, device="cuda")[None] > torch.arange(200, S, device="cuda")[:, None], -float("inf"))
+    ref = torch.softmax(s, dim=1)[None, None] @ V.double()
+    assert float((s[:, 200] - s[:, 5]).min()) > 0
+    assert bool(((out - ref).abs() <= 1.01 * 2.0 ** -8 * ref.abs() + 1e-20).all())
+
+
 def test_fmha_more_keys_than_queries_takes_the_general_kernel(ct, orc):
     data = fmha.prepare(batch=1, heads=2, seq_q=200, seq_kv=333, causal=False)
     r = run(data)
