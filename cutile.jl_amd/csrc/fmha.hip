@@ -962,8 +962,13 @@ extern "C" int mi_fmha_kernel(const mi_tile_array* Q, const mi_tile_array* K, co
             return launch_status();
         }
         if (!no_pipe && fmha::pipe128_applicable(pr)) {
-            fmha::pipe128_launch(pr, s);
-            return launch_status();
+            // (pipe: the kernel for heads of 128 whenever it can run; read at every call)
+            const char* e = getenv("MI_FMHA_KERNEL");
+            if ((e && strcmp(e, "pipe") == 0) ||
+                fmha::pipe128_pays(pr, pick_parts(cld(Sq, (int64_t)kQB) * B * H, B * H * Sq, 128, (int)Sq, (int)Skv, causal, input_pos))) {
+                fmha::pipe128_launch(pr, s);
+                return launch_status();
+            }
         }
     }
     if (dt == MI_F16) {

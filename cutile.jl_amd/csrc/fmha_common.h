@@ -174,8 +174,10 @@ struct Problem {
 };
 bool pipe_applicable(const Problem& p);
 void pipe_launch(const Problem& p, hipStream_t stream);
-// The same for head dimension 128 (fmha_pipe128.hip).
+// The same for head dimension 128 (fmha_pipe128.hip); `pipe128_pays` says whether it is the quicker one for a problem that
+// the kernel of fmha.hip would take in `parts` parts of the keys (0 = undivided).
 bool pipe128_applicable(const Problem& p);
+bool pipe128_pays(const Problem& p, int parts);
 void pipe128_launch(const Problem& p, hipStream_t stream);
 
 }  // namespace fmha

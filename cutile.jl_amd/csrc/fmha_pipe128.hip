@@ -531,19 +531,30 @@ bool pipe128_applicable(const Problem& p) {
     const int64_t nqb = (Q->sizes[1] + 127) / 128, nbh = Q->sizes[2] * Q->sizes[3], wgs = nqb * nbh;
     if (wgs * (128 + 2 * nqb) >= (1ll << 32) || nbh * (p.H > 128 ? p.H : 128) >= (1ll << 32)) return false;
     if (K->sizes[1] < kHK) return false;   // (the last half is the last 32 keys)
-    // Few queries are split over the keys (fmha.hip), and so are grids whose few workgroups would walk many keys each: this
-    // kernel takes 5 us + 0.6 us per half of the longest walk as long as every workgroup has a SIMD pair of its own, the
-    // split one 14 us + 5 ns per half of all walks together.  (4 heads, S = 2048: causal 42 against 29 us, not causal 41
-    // against 31; 8 heads: 43 : 43 and 42 : 50; 16 heads, S = 1024: 25 : 26 and 24 : 30.)
-    const int64_t Sq = Q->sizes[1], Skv = K->sizes[1];
-    if (Sq <= 64) return false;
-    int64_t longest = Skv, sum = Skv * nqb;   // keys walked by the last / by all workgroups of a head
+    return Q->sizes[1] > 64;               // (few queries: a group's heads are stacked in one tile, fmha.hip)
+}
+
+bool pipe128_pays(const Problem& p, int parts) {
+    const int64_t Sq = p.Q->sizes[1], Skv = p.K->sizes[1], nqb = (Sq + 127) / 128, wgs = nqb * p.Q->sizes[2] * p.Q->sizes[3];
+    int64_t longest = Skv, shortest = Skv;   // keys walked by the last / by the first workgroup of a head
     if (p.causal) {
-        if (p.input_pos + Sq < longest) longest = p.input_pos + Sq;
-        const int64_t shortest = p.input_pos + 128 < longest ? p.input_pos + 128 : longest;
-        sum = (longest + shortest) / 2 * nqb;
+        longest = p.input_pos + Sq < Skv ? p.input_pos + Sq : Skv;
+        shortest = p.input_pos + 128 < longest ? p.input_pos + 128 : longest;
     }
-    return 0.6 * (double)(longest / kHK) <= 9.0 + 0.005 * (double)(sum / kHK * nbh);
+    const double halves = (double)((longest + kHK - 1) / kHK), all = (double)(longest + shortest) / (2 * kHK) * (double)wgs;
+    // Times of both kernels on 950 shapes (1 to 8 batches of 1 to 64 heads, 65 to 4096 queries, up to 16384 keys, bf16):
+    // against the kernel that is split over the keys this one is quicker where its longest walk, 9 us + 0.8 us per half,
+    // ends before the split one's 18 us + 2.8 ns per half of all walks together.  (Quicker / slower, this kernel : the split
+    // one: 1 x 32 heads, 996 queries and keys, causal 34 : 42 us, 1200 of them not causal 45 : 58; 2 heads, 2034 causal 57 : 28,
+    // 16 heads, 1024 of 8192 causal 191 : 117.)
+    if (parts > 1) return 0.8 * halves <= 9.0 + 0.0028 * all;
+    // Where the other kernel walks the keys alone as well, the grid has to fill most of its last round of 512 workgroups
+    // (two per CU) and the walks be long enough to pay for the ramp: 2 x 32 heads, S = 2000 causal 82 : 115 us, 8 x 32 heads,
+    // S = 506 causal 38 : 45, 1 x 32 heads, S = 2048 causal 64 : 70; but 640 workgroups of 19 halves, not causal, 54 : 45, 4 x
+    // 32 heads, S = 1171 causal (1280 workgroups) 90 : 81, and 8 x 16 heads, S = 173 12.1 : 11.3.  On 700 further shapes,
+    // 220 of them taken, the times were 0.49 to 1.11 of the other kernel's, 0.76 in the mean.
+    const int64_t rounds = (wgs + 511) / 512;
+    return wgs >= 448 && wgs * 100 >= rounds * 512 * (rounds <= 2 ? 78 : 90) && halves >= (wgs < 800 ? 32 : 8) && (p.causal || rounds <= 2);
 }
 
 void pipe128_launch(const Problem& p, hipStream_t stream) {

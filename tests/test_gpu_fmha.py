@@ -173,11 +173,12 @@ def test_fmha_pipelined_kernel_ragged_without_the_causal_mask(ct, orc, batch, he
     (1, 40, 500, 500, 5, True, 0, torch.float16),                                                # heads walked in two uneven chunks per XCD
 ])
 @pytest.mark.parametrize("rising", [False, True])
-def test_fmha_pipelined_kernel_for_heads_of_128(ct, orc, batch, heads, sq, skv, qg, causal, pos, T, rising):
+def test_fmha_pipelined_kernel_for_heads_of_128(ct, orc, monkeypatch, batch, heads, sq, skv, qg, causal, pos, T, rising):
     """The D = 128 kernel at the edges of its 32-key halves, 64-query waves and 128-query workgroups: walks of one to
     many halves, a ragged last half (which re-reads keys of the half before and masks them), decode offsets, grouped
     heads, head counts that are and are not multiples of 8.  `rising`: scores that grow along the keys, so that the
     running maximum is raised again and again.  The output sits in a wider buffer that must stay as it was."""
+    monkeypatch.setenv("MI_FMHA_KERNEL", "pipe")   # (sizes at the edges; most are quicker on the other kernel)
     data = fmha.prepare(batch=batch, heads=heads, seq_q=sq, seq_kv=skv, d_k=128, d_v=128, query_group_size=qg, causal=causal, T=T)
     if rising:
         data.Q = (data.Q.float() * 0.25 + 1.0).to(T)
@@ -193,10 +194,11 @@ def test_fmha_pipelined_kernel_for_heads_of_128(ct, orc, batch, heads, sq, skv, 
 
 
 @pytest.mark.parametrize("causal", [False, True])
-def test_fmha_heads_of_128_the_largest_weight_is_not_rounded(ct, causal):
+def test_fmha_heads_of_128_the_largest_weight_is_not_rounded(ct, monkeypatch, causal):
     """Rows whose score rises once, from key 5 to key 200, by 0.2 to 8 powers of two, with a value at key 200 alone: the
     result is that value times 1 / (1 + 2^-rise).  With the weights relative to the row's true maximum the larger one
     is exactly 1 and nothing is rounded but the result (2^-8 of it; the rest of the bound is for fp32)."""
+    monkeypatch.setenv("MI_FMHA_KERNEL", "pipe")
     S, D = 256, 128
     Q = torch.zeros(1, 8, S, D, dtype=torch.bfloat16, device="cuda")
     Q[..., 0] = 1
