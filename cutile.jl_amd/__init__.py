@@ -216,16 +216,16 @@ def _launch(name: str, *args, stream=None):
     converts plain tensors, ints and floats (a matmul call 11.5 us of host time by ctypes, 5.1 by it; LayerNorm's three calls and a fill 51 and 21); it
     returns None, having called nothing, where anything else is among them, and ctypes then converts or refuses it."""
     global _streams
-    if stream is None and _streams:
-        rc = getattr(_native, name)(*args, None)
+    native = _native
+    if stream is None and _streams and native is not None:
+        rc = getattr(native, name)(*args, None)
         if rc == 0:
             return
         if rc is not None:
             raise MiError(name, rc, strerror(rc))
     args = [_ref(a) if t is _A else a for t, a in zip(_SIGNATURES[name][0], args)]
-    handle = _stream(stream)
+    _call(name, *args, _stream(stream))
     _streams = _streams or stream is None
-    _call(name, *args, handle)
 
 
 def fft_kernel(x_packed_in, y_packed_out, W0, W1, W2, T0, T1, N: int, F0: int, F1: int, F2: int, BS: int,

@@ -1,6 +1,8 @@
 """The native launch route (csrc/py/launch.cpp) against the ctypes one: the same descriptors for every form of tensor it
 takes, nothing called for the forms it leaves, and the same errors."""
 import ctypes
+import threading
+import time
 
 import pytest
 import torch
@@ -31,6 +33,47 @@ def test_other_numbers_are_left_to_ctypes(ct, tile):
 def test_wrong_number_of_arguments_is_left_to_ctypes(ct):
     ct.lib()
     assert ct._native.mi_vec_add_kernel_1d(None, None, 16, None) is None
+
+
+@pytest.fixture
+def unloaded(ct, monkeypatch):
+    """The package as before its first call, with a stream look-up that needs no GPU."""
+    ct.lib()
+    for name, value in (("_lib", None), ("_native", None), ("_streams", False), ("_stream", lambda stream=None: ctypes.c_void_p(0))):
+        monkeypatch.setattr(ct, name, value)
+    return ct
+
+
+def _empty_call(ct):
+    e = torch.zeros(0)
+    ct.vec_add_kernel_1d(e, e, e, 16)   # (nothing to do: MI_OK before any GPU call)
+
+
+def test_first_calls_from_several_threads(unloaded, monkeypatch):
+    """Calls that come while the first one is still loading the library."""
+    ct, load, errors = unloaded, unloaded._load_native, []
+    monkeypatch.setattr(ct, "_load_native", lambda cdll: (time.sleep(0.2), load(cdll))[1])
+
+    def work():
+        try:
+            for _ in range(20):
+                _empty_call(ct)
+        except Exception as e:   # noqa: BLE001
+            errors.append(e)
+    threads = [threading.Thread(target=work) for _ in range(8)]
+    for t in threads:
+        t.start()
+        time.sleep(0.01)
+    for t in threads:
+        t.join()
+    assert not errors and ct._native is not None
+
+
+def test_a_missing_library_is_named_by_every_call(unloaded, monkeypatch):
+    monkeypatch.setattr(unloaded, "LIB_PATH", "/nowhere/libmi355tile.so")
+    for _ in range(3):
+        with pytest.raises(RuntimeError, match="/nowhere/libmi355tile.so is missing"):
+            _empty_call(unloaded)
 
 
 @pytest.mark.gpu
