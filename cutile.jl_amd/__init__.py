@@ -19,7 +19,6 @@ import os
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # MI355TILE_LIB selects another build of the same library (e.g. an experimental variant).
 LIB_PATH = os.environ.get("MI355TILE_LIB") or os.path.join(_HERE, "libmi355tile.so")
-NATIVE_PATH = os.path.join(_HERE, "_mi355tile_launch.so")
 
 MI_F32, MI_F64, MI_F16, MI_BF16, MI_F8E4M3FN, MI_I32, MI_I64, MI_BOOL, MI_I8, MI_I16, MI_F8E5M2 = range(11)
 MI_MAX_RANK = 4
@@ -102,7 +101,7 @@ _SIGNATURES = {
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)
 
 _lib = None
-_native = None    # the module of native launches (csrc/py/launch.cpp), bound to the loaded library
+_native = None    # the module of native launches (csrc/py/launch.cpp), bound to the loaded library; None: ctypes only
 _streams = False  # whether this process has looked a current stream up (which sets torch's GPU side up, or refuses to)
 
 
@@ -127,12 +126,24 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+def _native_path():
+    """Where the module of native launches for this interpreter and this torch lies.  It reads both's structures, so a
+    module that was built for other versions has another name (csrc/Makefile) and is not found."""
+    import sysconfig
+    import torch
+    return os.path.join(_HERE, f"_mi355tile_launch.torch{torch.__version__}{sysconfig.get_config_var('EXT_SUFFIX')}")
+
+
 def _load_native(cdll):
-    if not os.path.exists(NATIVE_PATH):
-        raise RuntimeError(f"{NATIVE_PATH} is missing: it is built together with the library, see there")
+    path = _native_path()
+    if not os.path.exists(path):
+        import warnings
+        warnings.warn(f"{path} is missing (make -C {os.path.join(_HERE, 'csrc')} builds it): launches convert their "
+                      "arguments by ctypes, at two to three times the host time", RuntimeWarning, stacklevel=2)
+        return None
     import importlib.machinery
     import importlib.util
-    loader = importlib.machinery.ExtensionFileLoader("_mi355tile_launch", NATIVE_PATH)
+    loader = importlib.machinery.ExtensionFileLoader("_mi355tile_launch", path)
     native = importlib.util.module_from_spec(importlib.util.spec_from_loader("_mi355tile_launch", loader))
     loader.exec_module(native)
     native.bind_library({name: ctypes.cast(getattr(cdll, name), ctypes.c_void_p).value for name in _SIGNATURES})

@@ -76,6 +76,16 @@ def test_a_missing_library_is_named_by_every_call(unloaded, monkeypatch):
             _empty_call(unloaded)
 
 
+def test_without_the_module_launches_take_the_ctypes_route(unloaded, monkeypatch):
+    monkeypatch.setattr(unloaded, "_native_path", lambda: "/nowhere/launch.so")
+    with pytest.warns(RuntimeWarning, match="/nowhere/launch.so is missing"):
+        _empty_call(unloaded)
+    _empty_call(unloaded)
+    assert unloaded._native is None
+    with pytest.raises(unloaded.MiError):
+        unloaded.vec_add_kernel_1d(torch.zeros(0), torch.zeros(0), torch.zeros(0), 7)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["float32", "float64", "float16", "bfloat16", "int32", "int64", "float8_e4m3fn", "float8_e5m2"])
 def test_descriptors_are_those_of_the_ctypes_route(ct, dtype):
