@@ -652,12 +652,18 @@ static int fused_moe_impl(const mi_tile_array* A, const mi_tile_array* B, const 
     // wide shape its workgroups, and a weight strip is streamed once per 64 tokens.
     const bool dense = tile_slots == kTT && (TILE_M / kTT) % 2 == 0 && total >= (int64_t)kTT * E;
     const bool narrow = !silu && !dense && m_blocks * cld(N, (int64_t)128) < 768 && K >= 512;
+    const bool vecA = aligned(A->ptr, 16) && A->strides[1] % 8 == 0;
+    const bool vecB = aligned(B->ptr, 16) && B->strides[1] % (w8 ? 16 : 8) == 0 && B->strides[2] % (w8 ? 16 : 8) == 0;
     // 64-channel strips for e4m3 weights: half the activation traffic, which outweighs the weights' with 32 channels, at
     // half the workgroups -- where those still come to two per CU.  Whole cutile_moe, 32 -> 64 channels (1024 hidden, 2048
     // inter, top-2): 256 tokens 32 experts 53.4 -> 52.3 us, 400 tokens 62.9 -> 58.8, 256 tokens 64 experts 91.4 -> 83.4; but
     // 100 tokens 8 experts (128 strips) 30.7 -> 31.9 and 16 tokens 32 experts (20 of them hit) 37.3 -> 39.2.  A K that ends
     // in a partial step: 44.1 -> 44.4 (1408).  With 16-bit weights the two differ by 1-2 % either way.
-    const bool pair = narrow && w8 && K % 256 == 0 && E * cld(N, (int64_t)64) >= 512 && total >= 2 * E;
+    // Off the grid the kernel has load predicates and spills 18 registers.  This launch alone, 32 -> 64 channels: weight rows
+    // off 16 bytes 256 tokens 32 experts 79 -> 96 us; N = 1000 or 1022 there 21.4 -> 22.7, 64 tokens 17.6 -> 19.1, but 400 tokens
+    // (25 per expert) 28.7 -> 25.8 and with K = 512 64 tokens 10.7 -> 9.5; activation rows off 16 bytes 46 -> 36.
+    const bool pair = narrow && w8 && vecB && K % 256 == 0 && E * cld(N, (int64_t)64) >= 512 && total >= 2 * E &&
+                      (N % 64 == 0 || K <= 512 || total >= 24 * E);
     const int strip = pair ? 64 : narrow ? 32 : 128;
     const int n_blocks = silu ? (int)cld(N / 2, (int64_t)64) : (int)cld(N, (int64_t)strip);
     // (Two tiles per workgroup cover 64 tokens; with that many per expert on average every second expert has a
@@ -668,8 +674,6 @@ static int fused_moe_impl(const mi_tile_array* A, const mi_tile_array* B, const 
     // with one tile per workgroup and 49 us with two, against 43 us for the wide shape.)
     const int ts = dense ? 2 : 1;
     if (tiles * n_blocks > 0x7fffffffLL) return MI_E_GRID;
-    const bool vecA = aligned(A->ptr, 16) && A->strides[1] % 8 == 0;
-    const bool vecB = aligned(B->ptr, 16) && B->strides[1] % (w8 ? 16 : 8) == 0 && B->strides[2] % (w8 ? 16 : 8) == 0;
     dim3 grid((unsigned)(tiles / ts * n_blocks));
     // every tile of the launch inside the arrays and 16-byte aligned: the kernels without load predicates
     // (a K step of 512 for the e4m3 down projection, whose steps move half the weight bytes: 29.8 us against 20.4)

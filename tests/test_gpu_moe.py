@@ -200,6 +200,30 @@ def test_e4m3_weights_in_strips_of_64_channels(ct, orc, tokens, E, K, N, dtype, 
     assert bool((err <= bound).all()), float((err / bound).max())
 
 
+def test_e4m3_weight_rows_off_16_bytes_take_strips_of_32_channels(ct):
+    """The same weights in rows that are and are not 16-byte aligned (views of a wider buffer): two kernels, each off
+    the exact sum by K * 2^-24 of the sum of magnitudes and by the result's rounding at most."""
+    tokens, E, K, N = 64, 32, 512, 1024
+    g = torch.Generator(device="cuda").manual_seed(3)
+    A = torch.randn(tokens, K, device="cuda", generator=g).half()
+    W = torch.randn(E, N, K + 8, device="cuda", generator=g).to(torch.float8_e4m3fn)[:, :, :K]
+    scale = torch.rand(E, N, device="cuda", generator=g) * 0.1 + 0.05
+    ids = torch.argsort(torch.rand(tokens, E, device="cuda", generator=g), dim=1)[:, :2].t().contiguous() + 1
+    w = torch.rand(2, tokens, device="cuda", generator=g).half()
+    tok, exp = ct.moe_align_tile_size_device(ids, 128, E)
+    out, variant = [], []
+    for weights in (W.contiguous(), W):
+        out.append(torch.full((tokens * 2, N), float("nan"), dtype=torch.float16, device="cuda"))
+        ct.fused_moe_kernel(A, weights, out[-1], w, tok, exp, 2, True, 128, 128, 64, b_scale=scale)
+        variant.append(ct.last_variant())
+    assert variant == ["fused_moe_t32_n64_k256_ksplit2_w8a16", "fused_moe_t32_n32_k256_ksplit4_w8a16"]
+    f = (scale[ids.t().reshape(-1) - 1] * w.t().reshape(-1, 1)).double()      # (slot, channel)
+    x = W.double()[ids.t().reshape(-1) - 1] * A.double().repeat_interleave(2, dim=0)[:, None]
+    ref, mag = x.sum(dim=2) * f, x.abs().sum(dim=2) * f
+    for o in out:
+        assert bool(((o.double() - ref).abs() <= (K + 2) * 2.0 ** -24 * mag + 1.01 * 2.0 ** -11 * ref.abs() + 2.0 ** -23).all())
+
+
 def test_fp8_dequant_covers_every_code(ct, orc):
     """Every finite E4M3FN code as a weight: K = 256 codes against a one-hot activation picks
     each dequantised value out exactly (checks subnormals, signs and the exponent rebias)."""
