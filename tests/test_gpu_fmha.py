@@ -333,6 +333,45 @@ def test_fmha_pipelined_kernel_strided_views(ct, orc, causal):
     assert torch.all(out_buf[..., :D] == 0)
 
 
+@pytest.mark.parametrize("S", [256, 301])
+@pytest.mark.parametrize("causal", [True, False])
+def test_fmha_heads_of_128_strided_views(ct, orc, monkeypatch, causal, S):
+    """The same for heads of 128: Q / K / V as views of one packed (B, S, 3, H, D) buffer, Out of a wider one."""
+    monkeypatch.setenv("MI_FMHA_KERNEL", "pipe")
+    rng = np.random.default_rng(5)
+    B, H, D = 2, 4, 128
+    packed = torch.from_numpy(rng.standard_normal((B, S, 3, H, D), dtype=np.float32)).to(torch.bfloat16).cuda()
+    Q, K, V = (packed[:, :, i].permute(0, 2, 1, 3) for i in range(3))
+    out_buf = torch.zeros((B, H, S, 2 * D), dtype=torch.bfloat16, device="cuda")
+    out = out_buf[..., D:]
+    fmha.cutile_fmha(Q, K, V, causal=causal, out=out)
+    assert ct.last_variant() == "fmha_pipe_d128_q128_kv32_ring4"
+    ref = orc.ref_fmha(orc.to_julia(Q), orc.to_julia(K), orc.to_julia(V), causal=causal, dtype=np.float64)
+    check(orc, out, ref, 3e-2)
+    assert torch.all(out_buf[..., :D] == 0)
+
+
+def test_fmha_heads_of_128_rows_at_the_limit_of_their_offsets(ct, orc, monkeypatch):
+    """Keys and values so far apart that the last byte offset of a head lies just below 2^32, and just above what the
+    pipelined kernel addresses (rows * stride of 2^31 elements), which the general kernel takes."""
+    monkeypatch.setenv("MI_FMHA_KERNEL", "pipe")
+    S, D = 96, 128
+    limit = (1 << 31) // (S + 64)                    # the kernel's rule: (S + 64) * stride below 2^31
+    stride = limit // 8 * 8
+    g = torch.Generator(device="cuda").manual_seed(1)
+    Q = torch.empty(1, 1, S, D, dtype=torch.float16, device="cuda").normal_(0, 1, generator=g)
+    buf = torch.empty((S - 1) * (stride + 8) + 2 * D, dtype=torch.float16, device="cuda")
+    for st, piped in ((stride, True), (stride + 8, False)):
+        K = torch.as_strided(buf, (1, 1, S, D), (S * st, S * st, st, 1), 0)
+        V = torch.as_strided(buf, (1, 1, S, D), (S * st, S * st, st, 1), D)
+        k, v = (torch.empty(1, 1, S, D, dtype=torch.float16, device="cuda").normal_(0, 1, generator=g) for _ in range(2))
+        K.copy_(k)
+        V.copy_(v)
+        out = fmha.cutile_fmha(Q, K, V, causal=True)
+        assert (ct.last_variant() == "fmha_pipe_d128_q128_kv32_ring4") == piped
+        check(orc, out, orc.ref_fmha(*(orc.to_julia(t) for t in (Q, k, v)), causal=True, dtype=np.float64))
+
+
 @pytest.mark.parametrize("causal", [True, False])
 def test_fmha_running_maximum_keeps_rising(ct, orc, causal):
     """Scores that grow with the key index by far more than the kernel's lazy-rescale threshold:
