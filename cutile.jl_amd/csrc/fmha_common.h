@@ -106,16 +106,8 @@ template <> struct Pack<BF16> {
 
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
-// ---- pieces of the software-pipelined kernels (fmha_pipe.hip, fmha_pipe128.hip) ---------------
+// ---- what both software-pipelined kernels (fmha_pipe.hip, fmha_pipe128.hip) use ---------------
 #pragma clang diagnostic ignored "-Winline-asm"  // m0 is named as clobbered on purpose
-
-// One 1 KB global->LDS transfer: lane l moves 16 bytes from sbase + voff to lds_base + 16*l.
-__device__ __forceinline__ void dma16(unsigned voff, const char* sbase, unsigned lds_base) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :
-                 : "v"(voff), "s"(sbase), "s"(lds_base)
-                 : "memory", "m0");
-}
 
 __device__ __forceinline__ void fence() { asm volatile("" ::: "memory"); }
 
@@ -142,19 +134,6 @@ __device__ __forceinline__ float xhalf_max(float v) {
 __device__ __forceinline__ float xhalf_sum(float v) {
     auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
-// Second stage of the weights of one score pair h = 0..7 of a 32-key half: round and pack for the P.V MFMAs, add to
-// the row sum (f16: once per 16-key chunk, see Pack<F16>).
-template <typename E>
-__device__ __forceinline__ void exp_stage2(const float (&p)[2], int h, float& l, unsigned (&pf)[2][4]) {
-    const unsigned pk = Pack<E>::pack(p[0], p[1]);
-    pf[h >> 2][h & 3] = pk;
-    if constexpr (Pack<E>::kChunkSum) {
-        if ((h & 3) == 3) l = Pack<E>::sum_chunk(pf[h >> 2], l);   // the chunk is complete
-    } else {
-        l = Pack<E>::sum2(pk, p[0], p[1], l);
-    }
 }
 
 // Closes an issue slot: nothing is scheduled across it.

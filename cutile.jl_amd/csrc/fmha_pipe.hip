@@ -42,6 +42,14 @@ constexpr int kSlotBytes = kSlot * 2;
 constexpr int kPre = 1;           // issue slots of a step that run before its wait and barrier
 constexpr float kRaise = 8.0f;    // raise m only when the new maximum exceeds it by this much
 
+// One 1 KB global->LDS transfer: lane l moves 16 bytes from sbase + voff to lds_base + 16*l.
+__device__ __forceinline__ void dma16(unsigned voff, const char* sbase, unsigned lds_base) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :
+                 : "v"(voff), "s"(sbase), "s"(lds_base)
+                 : "memory", "m0");
+}
+
 // s_waitcnt immediates (gfx9 encoding): lgkmcnt(0) with vmcnt(N)
 constexpr int kWaitVm0 = 0x0070, kWaitVm4 = 0x0074, kWaitVm8 = 0x0078, kWaitVm2 = 0x0072, kWaitVm6 = 0x0076,
               kWaitLgkm = 0xc07f;   // lgkmcnt(0) alone
@@ -212,6 +220,19 @@ __device__ __forceinline__ void exp_stage1(const f32x16& s, int h, float (&p)[2]
     p[0] = __builtin_amdgcn_exp2f(s[2 * h]);
     p[1] = __builtin_amdgcn_exp2f(s[2 * h + 1]);
 }
+// Second stage of the weights of one score pair h = 0..7 of a 32-key half: round and pack for the P.V MFMAs, add to
+// the row sum (f16: once per 16-key chunk, see Pack<F16>).
+template <typename E>
+__device__ __forceinline__ void exp_stage2(const float (&p)[2], int h, float& l, unsigned (&pf)[2][4]) {
+    const unsigned pk = Pack<E>::pack(p[0], p[1]);
+    pf[h >> 2][h & 3] = pk;
+    if constexpr (Pack<E>::kChunkSum) {
+        if ((h & 3) == 3) l = Pack<E>::sum_chunk(pf[h >> 2], l);   // the chunk is complete
+    } else {
+        l = Pack<E>::sum2(pk, p[0], p[1], l);
+    }
+}
+
 constexpr int popcount2(int m) { return (m & 1) + ((m >> 1) & 1); }
 // k-th stream (0-based) of a non-empty 2-bit stream mask
 constexpr int nth_stream(int m, int k) { return (m & 1) ? k : 1; }

@@ -21,7 +21,9 @@
 // result, the general kernel 1.756e-3).  A stream's sums are rescaled when any of its 32 rows has a new maximum, which is
 // most halves: 64 multiplies that nothing hides, a fifth of the time in all.  Raising only what had outgrown its maximum
 // by 2^8 (P in (0, 2^8]) took 75 instead of 86 us and was off by 1.831e-3 (scores of three times the spread: 2.15e-3
-// against 1.75e-3); the multiplies spread over slots 0..15 behind a branch each took 91 us.  Scores are scaled in fp32.
+// against 1.75e-3); the multiplies spread over slots 0..15 behind a branch each took 91 us, and maxima raised once per two
+// halves 90 us: half the multiplies, but a third set of scores, which with O takes 224 of the 256 registers that vector
+// instructions reach, and what else is there moves to and fro.  Scores are scaled in fp32.
 //
 // Measured (2 x 32 heads in groups of 4, bf16, against the general kernel): S = 2048 causal 120 -> 86 us (0.57 -> 0.80
 // PFLOP/s), not causal 153 -> 142 us (0.90 -> 0.97), S = 2000 causal 117 -> 87 us.  What bounds it is the issue of one wave per

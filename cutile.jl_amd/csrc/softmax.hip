@@ -5,12 +5,13 @@
 // column at a time.  The single-tile kernel keeps the whole column in registers, so HBM is
 // touched exactly once per element each way (algorithmic traffic 2*M*N*sizeof(T)): 16-byte
 // loads, wave64 shuffle reductions, one LDS exchange per reduction across the waves of the
-// workgroup.  Columns too long for that (more than 16384 elements per 256 lanes' registers) take
-// the reference's three passes (max, denominator, normalise), re-reading the column from L2;
-// softmax_chunked_kernel uses the register kernel too whenever its column fits.
+// workgroup.  Columns of more than 65536 elements take the reference's three passes (max, denominator,
+// normalise), re-reading the column from L2; softmax_chunked_kernel uses the register kernel too whenever
+// its column fits.
 //
-// Numerics follow the reference: fp32 math, max ignores NaN, full-precision exp (not
-// exp2), IEEE division, padding rows read as -Inf and are never written.
+// Numerics follow the reference: fp32 math, max ignores NaN, the exponential of x - max, one correctly rounded
+// reciprocal of the sum per column, padding rows read as -Inf and are never written.  The exponential is the library's
+// for fp32 columns of up to 16384 elements, else the hardware's 2^x (struct Exp2).
 #include "common.h"
 #include <math.h>
 
@@ -352,7 +353,7 @@ int launch_len(const mi_tile_array* output, const mi_tile_array* input, int64_t 
             else if (per > 8) WIDE(10);
         }
 #undef WIDE
-        set_variant(L > 32768 ? "softmax_regs_b1024_e64" : "softmax_regs_b1024_e32");
+        set_variant(L > 32768 ? "softmax_regs_b1024_e64" : "softmax_regs_b1024_e32");   // (at most 64 / 32 elements per lane)
         return launch_status();
     }
     if (vecs <= 64) { launch_regs<T, 64, 1>(output, input, L, al, s); set_variant("softmax_regs_b64_v1"); }
