@@ -297,14 +297,16 @@ bool vec_ok(const mi_tile_array* output, const mi_tile_array* input) {
 template <typename T, int BLOCK, int VPT>
 void launch_regs(const mi_tile_array* output, const mi_tile_array* input, int L, bool al,
                  hipStream_t s) {
-    const int64_t M = input->sizes[1];
-    dim3 grid((unsigned)M), block(BLOCK);
-    if (al && stream_hint(2 * M * (int64_t)L * (int64_t)sizeof(T)))
-        hipLaunchKernelGGL((softmax_regs_kernel<T, BLOCK, VPT, true>), grid, block, 0, s, (T*)output->ptr, output->strides[1],
-                           (const T*)input->ptr, input->strides[1], L);
-    else
-        hipLaunchKernelGGL((softmax_regs_kernel<T, BLOCK, VPT, false>), grid, block, 0, s, (T*)output->ptr, output->strides[1],
-                           (const T*)input->ptr, input->strides[1], L);
+    const int64_t M = input->sizes[1], ldi = input->strides[1], ldo = output->strides[1];
+    const bool stream = al && stream_hint(2 * M * (int64_t)L * (int64_t)sizeof(T));
+    constexpr int64_t kMost = 0xffffffffll / BLOCK;   // workgroups of a launch: fewer than 2^32 lanes
+    for (int64_t c = 0; c < M; c += kMost) {
+        const dim3 grid((unsigned)(M - c < kMost ? M - c : kMost)), block(BLOCK);
+        T* op = (T*)output->ptr + c * ldo;
+        const T* ip = (const T*)input->ptr + c * ldi;
+        if (stream) hipLaunchKernelGGL((softmax_regs_kernel<T, BLOCK, VPT, true>), grid, block, 0, s, op, ldo, ip, ldi, L);
+        else hipLaunchKernelGGL((softmax_regs_kernel<T, BLOCK, VPT, false>), grid, block, 0, s, op, ldo, ip, ldi, L);
+    }
 }
 
 template <typename T>

@@ -355,6 +355,19 @@ def test_softmax_maxima_far_from_zero(ct, orc, T, N):
     assert (err <= 0).all(), [i for i in range(len(cols)) if not (err[i] <= 0).all()]
 
 
+def test_softmax_more_columns_than_workgroups_of_a_launch(ct):
+    """2^22 + 3 columns in workgroups of 1024 lanes are more lanes than one launch takes.  All columns are the same one (a view
+    with a column stride of 0); their results lie one element apart, so the last element is the last column's alone."""
+    M, N = (1 << 22) + 3, 16388
+    g = torch.Generator(device="cuda").manual_seed(2)
+    x = torch.empty(1, N, device="cuda").normal_(0, 2, generator=g)
+    y = torch.full((M + N - 1,), float("nan"), device="cuda")
+    ct.softmax_tma_kernel(y.as_strided((M, N), (1, 1)), x.expand(M, N), 32768, num_programs=1024)
+    p = torch.softmax(x[0].double(), dim=0).cpu().numpy()
+    close_f32(y[[0, -1]].cpu().numpy(), p[[0, -1]])
+    assert not bool(y.isnan().any())
+
+
 def test_softmax_tile_smaller_than_column_and_padding(ct, orc):
     """A TILE_SIZE below N covers rows 1..TILE_SIZE only (softmax.jl:29-38); the chunked
     kernel walks cld(n_elems, TILE)*TILE rows, clipped to the array."""
