@@ -351,6 +351,25 @@ def test_fmha_heads_of_128_strided_views(ct, orc, monkeypatch, causal, S):
     assert torch.all(out_buf[..., :D] == 0)
 
 
+@pytest.mark.parametrize("batch,heads,qg,sq,skv,causal,piped", [
+    (1, 32, 4, 900, 1500, False, True), (1, 16, 4, 256, 4096, True, False),      # split by the other kernel: many, few workgroups
+    (2, 32, 4, 1000, 1000, True, True), (8, 32, 4, 500, 500, True, True),        # not split: rounds of the chip filled ...
+    (8, 32, 4, 300, 300, True, False), (8, 16, 1, 173, 173, False, False),       # ... and not
+])
+def test_fmha_heads_of_128_both_sides_of_the_rule(ct, monkeypatch, batch, heads, qg, sq, skv, causal, piped):
+    """The rule's choice against the pipelined kernel: they differ by the weights' rounding relative to maxima of other
+    key ranges, 2^-8 of a weight at most, and by the result's, 2^-8 of it."""
+    data = fmha.prepare(batch=batch, heads=heads, seq_q=sq, seq_kv=skv, d_k=128, d_v=128, query_group_size=qg, causal=causal, T=torch.bfloat16)
+    a = fmha.cutile_fmha(data.Q, data.K, data.V, query_group_size=qg, causal=causal, input_pos=skv - sq)
+    assert (ct.last_variant() == "fmha_pipe_d128_q128_kv32_ring4") == piped
+    monkeypatch.setenv("MI_FMHA_KERNEL", "pipe")
+    b = fmha.cutile_fmha(data.Q, data.K, data.V, query_group_size=qg, causal=causal, input_pos=skv - sq)
+    assert ct.last_variant() == "fmha_pipe_d128_q128_kv32_ring4"
+    a, b = a.double(), b.double()
+    assert bool(((a - b).abs() <= 2.0 ** -7 * (b.abs() + data.V.double().abs().max())).all())
+    assert float((a - b).norm() / b.norm()) < 2.0 ** -8
+
+
 def test_fmha_heads_of_128_rows_at_the_limit_of_their_offsets(ct, orc, monkeypatch):
     """Keys and values so far apart that the last byte offset of a head lies just below 2^32, and just above what the
     pipelined kernel addresses (rows * stride of 2^31 elements), which the general kernel takes."""
