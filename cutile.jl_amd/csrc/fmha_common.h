@@ -45,10 +45,7 @@ struct BF16 {
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
     }
     static __device__ __forceinline__ short cvt(float v) {
-        unsigned u = __float_as_uint(v);
-        if ((u & 0x7fffffffu) > 0x7f800000u) return (short)((u >> 16) | 0x40);
-        u += 0x7fffu + ((u >> 16) & 1u);
-        return (short)(u >> 16);
+        return (short)to_bf16(v);
     }
     static __device__ __forceinline__ float to_f32(short v) { return __uint_as_float((unsigned)(unsigned short)v << 16); }
     static __device__ __forceinline__ s16x8 scale8(s16x8 q, float s) {

@@ -47,8 +47,7 @@ template <> __device__ __forceinline__ void vset<__half>(Raw<__half>::V& v, int 
     v[q] = (_Float16)f;
 }
 template <> __device__ __forceinline__ void vset<__hip_bfloat16>(Raw<__hip_bfloat16>::V& v, int q, float f) {
-    __hip_bfloat16 h = __float2bfloat16(f);
-    v[q] = *reinterpret_cast<unsigned short*>(&h);
+    v[q] = to_bf16(f);
 }
 
 // A 16-byte vector at an address that is aligned for its elements only: global memory takes such accesses, in one
