@@ -26,6 +26,11 @@ struct F16 {
         _Float16 h = (_Float16)v;
         return __builtin_bit_cast(unsigned short, h);
     }
+    static __device__ __forceinline__ float round(float v) { return (float)(_Float16)v; }   // to the type and back
+    static __device__ __forceinline__ unsigned pack(float lo, float hi) {
+        typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+        return __builtin_bit_cast(unsigned, h2{(_Float16)lo, (_Float16)hi});
+    }
 };
 struct BF16 {
     static __device__ __forceinline__ f32x16 mfma32(s16x8 a, s16x8 b, f32x16 c) {
@@ -34,6 +39,11 @@ struct BF16 {
     }
     static __device__ __forceinline__ unsigned short from_f32(float v) {
         return to_bf16(v);
+    }
+    static __device__ __forceinline__ float round(float v) { return (float)(__bf16)v; }
+    static __device__ __forceinline__ unsigned pack(float lo, float hi) {
+        typedef __bf16 h2 __attribute__((ext_vector_type(2)));
+        return __builtin_bit_cast(unsigned, h2{(__bf16)lo, (__bf16)hi});
     }
 };
 

@@ -35,12 +35,16 @@
 
 #include "gemm_direct.h"
 #include "moe_dense.h"
+#include "moe_tiles.h"
 
 namespace {
 
 using namespace mi;
 using namespace mi::gemm;
 using mi::moe::DenseArgs;
+using mi::moe::accumulate_tile;
+using mi::moe::store_tile_slot_lane;
+using mi::moe::widen16;
 
 constexpr int BK = 32;
 constexpr int kRows = 128;            // slots, and weight rows, per workgroup tile
@@ -49,10 +53,6 @@ constexpr int MODE_PLAIN = 0, MODE_SILU = 1, MODE_ACC = 2;
 
 // Source of every chunk that lies past K.
 __device__ __attribute__((aligned(16))) const unsigned zeros16d[4] = {0u, 0u, 0u, 0u};
-
-__device__ __forceinline__ float widen16(bool bf16, unsigned short h) {
-    return bf16 ? __uint_as_float(((unsigned)h) << 16) : (float)__builtin_bit_cast(_Float16, h);
-}
 
 // J: MFMA column tiles (32 channels each) per wave.  J = 2: tile of 128 weight rows, ring of four stages of 16 KB;
 // J = 4: 256 weight rows, ring of three stages of 24 KB.  Either way two workgroups fit a CU.
@@ -490,42 +490,6 @@ struct Meta {
     int tw[4];              // (stages of 64 k) entries of the rows of this lane's four transfers
 };
 
-// Stores one 32-slot x 32-channel tile held slot-per-lane (o[r]: channel 8 * (r / 4) + 4 * hb + r % 4 of the lane's
-// slot) as 16-byte pieces: four registers are four consecutive channels; the two half-waves of a lane pair (l, l + 32)
-// hold the two halves of every group of eight, and two lane-half swaps per pair of groups leave every lane with eight
-// consecutive channels of its slot's row.  `row`: the slot's output row at the tile's first channel; n_left: channels
-// from there to the end of the row.
-template <typename E>
-__device__ __forceinline__ void store_tile_slot_lane(const float (&o)[16], unsigned short* row, bool valid, int n_left,
-                                                     bool vec_ok, int hb) {
-    unsigned P[4][2];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        P[q][0] = (unsigned)E::from_f32(o[4 * q]) | ((unsigned)E::from_f32(o[4 * q + 1]) << 16);
-        P[q][1] = (unsigned)E::from_f32(o[4 * q + 2]) | ((unsigned)E::from_f32(o[4 * q + 3]) << 16);
-    }
-#pragma unroll
-    for (int q = 0; q < 4; q += 2) {
-        // lower half-wave: own group q, then the partner's half of it; upper: the partner's half of group q + 1, then own
-        const auto s0 = __builtin_amdgcn_permlane32_swap(P[q][0], P[q + 1][0], false, false);
-        const auto s1 = __builtin_amdgcn_permlane32_swap(P[q][1], P[q + 1][1], false, false);
-        const u32x4 v = {s0[0], s1[0], s0[1], s1[1]};
-        const int c = 8 * q + 8 * hb;   // first of this lane's eight channels
-        if (valid) {
-            if (vec_ok && c + 8 <= n_left) {
-                // (an ordinary store: what is written here is read again by the next launch -- the down projection
-                // or the sum over the slots -- and a streaming store would send it past the L2 it can be found in;
-                // measured 1-7 % on both launches, most at 16 384 tokens)
-                *reinterpret_cast<u32x4*>(row + c) = v;
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    if (c + e < n_left) row[c + e] = (unsigned short)(v[e >> 1] >> (16 * (e & 1)));
-            }
-        }
-    }
-}
-
 // Stores of one tile.
 // A8: the products are those of unscaled fp8 codes and every channel is multiplied by its fp32 scale first (scale_of:
 // b_scale entry of a weight row of the tile's expert, 1 for rows past N).
@@ -594,42 +558,12 @@ __device__ __forceinline__ void epilogue(const DenseArgs& a, const f32x16 (&acc)
                 store_tile_slot_lane<E>(o, a.C + (int64_t)(tokv ? tokv - 1 : 0) * a.ldc + ch0, tokv != 0, a.N - ch0, vec_ok, hb);
             }
         } else {
-            // lane = channel; rows of a 32 x 32 tile = slots 8 * (r / 4) + 4 * hb + r % 4.  Two neighbouring MFMA column
-            // tiles are 64 consecutive channels: swapping the upper half of the first one's register with the lower half
-            // of the second one's gives one register with all 64 channels of row R and one with those of row R + 4.
-            // Column (token_id - 1) >> acc_shift receives the replica's value as rounded to the storage type, by a
-            // packed atomic add of two adjacent channels: even lanes send row R, odd lanes row R + 4, each row 128
-            // consecutive bytes.
+            // lane = channel (two neighbouring MFMA column tiles are 64 consecutive channels)
 #pragma unroll
             for (int jp = 0; jp < J; jp += 2) {
-                const int gn = bid_n * (64 * J) + 32 * J * wn + 32 * jp + lane;
-                // (before the swap a lane holds channel lane % 32 of both column tiles)
-                const int gn0 = bid_n * (64 * J) + 32 * J * wn + 32 * jp + (lane & 31);
-                const float s0 = scale_of(gn0), s1 = scale_of(gn0 + 32);
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int R = 8 * (r >> 2) + (r & 3);
-                    const int tokA = __builtin_amdgcn_readlane(tokv, R), tokB = __builtin_amdgcn_readlane(tokv, R + 4);
-                    float v0 = acc[i][jp][r], v1 = acc[i][jp + 1][r];
-                    if constexpr (A8) {
-                        v0 *= s0;
-                        v1 *= s1;
-                    }
-                    if (a.mul_routed_weight) {
-                        const float wA = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wtv), R));
-                        const float wB = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, wtv), R + 4));
-                        const float w = hb ? wB : wA;
-                        v0 *= w;
-                        v1 *= w;
-                    }
-                    const auto sw = __builtin_amdgcn_permlane32_swap((unsigned)E::from_f32(v0), (unsigned)E::from_f32(v1), false, false);
-                    const unsigned rowA = sw[0], rowB = sw[1];   // this lane's channel of row R / of row R + 4
-                    const unsigned nbrA = (unsigned)__shfl_xor((int)rowA, 1, 64), nbrB = (unsigned)__shfl_xor((int)rowB, 1, 64);
-                    const int tok = (lane & 1) ? tokB : tokA;
-                    const unsigned pair = (lane & 1) ? (nbrB | (rowB << 16)) : (rowA | (nbrA << 16));
-                    if (tok && gn < a.N)
-                        mi::moe::atomic_add2(a.bf16, a.C + (gn & ~1) + (int64_t)((tok - 1) >> a.acc_shift) * a.ldc, pair);
-                }
+                const int ch0 = bid_n * (64 * J) + 32 * J * wn + 32 * jp;
+                accumulate_tile<E, A8>(a, acc[i][jp], acc[i][jp + 1], scale_of(ch0 + (lane & 31)), scale_of(ch0 + 32 + (lane & 31)),
+                                       s_tok + 64 * ws + 32 * i, s_wt + 64 * ws + 32 * i, ch0, lane);
             }
         }
     }
@@ -652,8 +586,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WIDE ? 1 : 
     constexpr int kLast = J == 2 ? 1 : 0;  // the ring of three has no fourth stage
     __shared__ __attribute__((aligned(1024))) unsigned short Ts0[kStageT], Ts1[kStageT], Ts2[kStageT], Ts3[kLast ? kStageT : 8];
     __shared__ __attribute__((aligned(1024))) unsigned short Ws0[kStageW], Ws1[kStageW], Ws2[kStageW], Ws3[kLast ? kStageW : 8];
-    __shared__ int s_tok[2][kRows];      // 1-based replica id of every slot, 0 = no token (two tiles: current and next)
-    __shared__ float s_wt[2][kRows];     // its routed weight (1 where none is applied)
+    __shared__ __attribute__((aligned(16))) int s_tok[2][kRows];      // 1-based replica id of every slot, 0 = no token (two tiles: current and next)
+    __shared__ __attribute__((aligned(16))) float s_wt[2][kRows];     // its routed weight (1 where none is applied)
     __shared__ unsigned s_live[2][2];    // per half of the block: bit i = its 32-slot tile i holds a token
     const int tid = threadIdx.x, lane = tid & 63, hb = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -930,6 +864,9 @@ static int pick_j(const DenseArgs& a) {
 }
 
 void dense_launch(const DenseArgs& a, hipStream_t s) {
+    // (a forced shape of this kernel is this kernel)
+    if (!getenv("MI_MOE_DENSE_J") && !getenv("MI_MOE_DENSE_WIDE") && !getenv("MI_MOE_DENSE_STREAM"))
+        if (const int rows = prefill_rows(a)) return prefill_launch(a, rows, s);
     const int J = pick_j(a);
     const int n_blocks = a.silu ? (int)cld((int64_t)a.N / 2, (int64_t)(32 * J)) : (int)cld((int64_t)a.N, (int64_t)(64 * J));
     const int64_t tiles = (int64_t)a.num_blocks * (a.TILE_M / kRows) * n_blocks;

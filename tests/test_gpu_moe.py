@@ -794,3 +794,74 @@ def test_fp8_activations_are_refused_where_no_kernel_takes_them(ct):
         moe.invoke_fused_moe_kernel(h8, d.w1, c, d.topk_weights, tok, exp, mul_routed_weight=False, num_token_replicas=2,
                                     tile_m=128, tile_n=128, tile_k=64)
     assert e.value.code == ct.MI_E_DTYPE
+
+
+def _routed(counts, topk=1, **kw):
+    """moe.prepare with expert e taking counts[e] replicas (in shuffled order; topk slots of a token may name one expert twice)."""
+    total = sum(counts)
+    assert total % topk == 0
+    d = moe.prepare(num_tokens=total // topk, num_experts=len(counts), topk=topk, **kw)
+    ids = np.repeat(np.arange(1, len(counts) + 1), counts)
+    np.random.default_rng(11).shuffle(ids)
+    d.topk_ids = torch.from_numpy(ids.reshape(topk, -1).astype(np.int64)).cuda()
+    return d
+
+
+@pytest.mark.parametrize("rows", ["2", "4"])
+@pytest.mark.parametrize("make", [
+    # replicas per expert on the edges of 32-slot sub-tiles and of the tiles of 5 / 6 of them, none, and several tiles
+    lambda: _routed([1, 31, 32, 33, 0, 127, 128, 160, 161, 192, 193, 700], hidden_size=256, intermediate_size=264),
+    lambda: _routed([150, 170, 330, 250], topk=2, hidden_size=1000, intermediate_size=328, T=torch.bfloat16),   # K and N off 64 / 128 / 256
+    lambda: moe.prepare(num_tokens=1024, hidden_size=256, num_experts=160, intermediate_size=256, topk=8),       # more runs than the table holds
+    lambda: moe.prepare(num_tokens=2048, hidden_size=512, num_experts=8, intermediate_size=512, topk=2, router="top2_logits"),
+], ids=["edges", "ragged", "many_runs", "prefill"])
+def test_prefill_kernel_gives_the_streaming_kernels_bits(ct, orc, make, rows, monkeypatch):
+    """The grouped GEMM whose transfers have waves of their own: k in the order of the streaming kernels, so the same bits on
+    plain, SiLU-fused and accumulating launches, with both of its tiles (128 and 256 weight rows)."""
+    d = make()
+    with _dense_knob("0"):
+        want = _every_path(d, 128)
+    monkeypatch.setenv("MI_MOE_PREFILL", rows)
+    with _dense_knob("1"):
+        got = _every_path(d, 128)
+        got256 = _every_path(d, 256)
+        c = torch.full((d.num_tokens * d.topk, 2 * d.intermediate_size), float("nan"), dtype=d.hidden_states.dtype, device="cuda")
+        tok, exp = ct.moe_align_tile_size_device(d.topk_ids, 128, d.num_experts)
+        moe.invoke_fused_moe_kernel(d.hidden_states, d.w1, c, d.topk_weights, tok, exp, mul_routed_weight=True,
+                                    num_token_replicas=d.topk, tile_m=128, tile_n=128, tile_k=64)
+        assert ct.last_variant() == ("fused_moe_dense_t128_to160_n256_k64_ring3" if rows == "4" else "fused_moe_dense_t128_to192_n128_k64_ring3")
+        assert not torch.isnan(c.float()).any()
+    for k in want:
+        assert torch.equal(got[k], want[k]), k
+        assert torch.equal(got256[k], want[k]), k
+    J = orc.to_julia
+    ref = orc.ref_moe(J(d.hidden_states), J(d.w1), J(d.w2), J(d.topk_weights), J(d.topk_ids), dtype=np.float64)
+    check(J(got["separate"]), ref, 5e-2 if d.hidden_states.dtype == torch.bfloat16 else 2e-2)
+
+
+@pytest.mark.parametrize("rows", ["2", "4"])
+def test_prefill_kernel_on_arrays_that_no_sort_made(ct, rows, monkeypatch):
+    """Slots without a token anywhere in a block, whole blocks without one, blocks of one expert apart from each other, blocks
+    without an expert, and rows of C off 16 bytes: what the arrays name is computed, nothing else is written."""
+    d = moe.prepare(num_tokens=1500, hidden_size=256, num_experts=5, intermediate_size=160, topk=1)
+    rng = np.random.default_rng(3)
+    exp = torch.from_numpy(np.array([2, 2, 0, 2, 5, 5, 5, 1, 4, 4, 9, 3, 2], dtype=np.int32)).cuda()
+    ids = rng.permutation(1500)[:13 * 128 - 300].astype(np.int32) + 1
+    ids = np.concatenate([ids, np.zeros(13 * 128 - ids.size, dtype=np.int32)])
+    rng.shuffle(ids)
+    ids[128:256] = 0                       # a run whose second block holds nothing
+    ids[4 * 128 + 40:5 * 128] = 0          # a first block with one sub-tile and a part, followed by full ones
+    ids[7 * 128 + 1:8 * 128] = 0           # a block with one token
+    ids[11 * 128:11 * 128 + 100] = 0       # tokens in the last sub-tile only
+    tok = torch.from_numpy(ids[:-3].copy()).cuda()   # (the last block ends early)
+    def run(knob):
+        c = torch.full((1500, 2 * 160 + 4), 7.0, dtype=torch.float16, device="cuda")
+        with _dense_knob(knob):
+            moe.invoke_fused_moe_kernel(d.hidden_states, d.w1, c[:, :2 * 160], d.topk_weights, tok, exp, mul_routed_weight=False,
+                                        num_token_replicas=1, tile_m=128, tile_n=128, tile_k=64)
+        return c, ct.last_variant()
+    want, _ = run("0")
+    monkeypatch.setenv("MI_MOE_PREFILL", rows)
+    got, name = run("1")
+    assert "_to1" in name
+    assert torch.equal(got, want)
