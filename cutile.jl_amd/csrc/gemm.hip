@@ -19,9 +19,11 @@
 //                    not 16-byte aligned, K below 256).
 //   gemm16_big       (gemm_big.hip) f16/bf16, 256x256 workgroup tile, 4 waves of 128x128 (or 256x128 /
 //                    128x128 tiles for problems with few tiles), K step 32 through a ring of four LDS
-//                    stages filled by direct global->LDS loads, XOR-swizzled LDS layouts; used when M
-//                    and K are multiples of 8, K >= 256, everything is 16-byte aligned and there are
-//                    at least 16 tiles of 128x128 (ragged edges in M, N and K are handled on the way in).
+//                    stages filled by direct global->LDS loads, XOR-swizzled LDS layouts; used from K = 256
+//                    and 16 tiles of 128x128, or K = 320, on (any alignment and ragged edges in M, N and K are
+//                    handled on the way in; few tiles and a long K are split over K).
+//   gemm16_pc        (gemm_pc.hip) f16/bf16, 128x128 and 256x128 tiles with waves of their own for the
+//                    transfers, for rows off 16-byte boundaries and K >= 1000.
 //   gemm32           fp32 via v_mfma_f32_32x32x2_f32 (gfx950 has no TF32-class MFMA;
 //                    the reference rounds fp32 operands to TF32, matmul.jl:49-52), 128x128x16 tile,
 //                    any shape; gemm32_big (gemm32_big.hip), the fp32 sibling of gemm16_big, takes
@@ -428,10 +430,10 @@ bool edge_split(const Problem& p, hipStream_t s, int* status) {
         }
         return big32_cost(q) * 59.0 * ks;
     };
-    // a strip of r rows or columns by itself (us): f16 splits it over K (two launches, 10 us) unless K is off the chunks;
-    // f32 walks K in one launch of small tiles
+    // a strip of r rows or columns by itself (us): f16 splits it over K (two launches; with K off the chunks its rows are
+    // misaligned as well: 15 us for 8 x 4096 x 4097, 21 for 256); f32 walks K in one launch of small tiles
     auto strip = [&](int64_t r, int64_t other) {
-        if (f16) return p.K % 8 ? 6.0 + 22.0 * ks : 10.0 + 9.5 * ks * (double)(r * other) / (256.0 * 4096.0);
+        if (f16) return p.K % 8 ? 8.0 + 6.5 * ks + 7.0 * ks * (double)(r * other) / (256.0 * 4096.0) : 10.0 + 9.5 * ks * (double)(r * other) / (256.0 * 4096.0);
         return 4.0 + 62.0 * ks * (other > 8192 ? other / 8192.0 : 1.0);
     };
     const double full = whole(p);

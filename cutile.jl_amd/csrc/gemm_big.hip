@@ -187,9 +187,14 @@ __global__ __launch_bounds__(256) void gemm16_big(const unsigned short* __restri
     if (ksplit > 1) {
         ks_part = L % ksplit;
         L /= ksplit;
-        K = K - ks_part * kchunk < kchunk ? K - ks_part * kchunk : kchunk;
+        if (ks_part < ksplit - 1) {
+            K = kchunk;
+            kpeel = 0;   // (the values behind the transfers belong to the last part)
+        } else {
+            K -= ks_part * kchunk;
+        }
     }
-    if (total_all % 8 == 0) L = (L & 7) * (total_all >> 3) + (L >> 3);
+    L = xcd_tile(L, total_all);
     const int bz = L / total;
     L -= bz * total;
     constexpr int GM = 4;
@@ -290,8 +295,8 @@ __global__ __launch_bounds__(256) void gemm16_big(const unsigned short* __restri
     if (kpeel > 0) {   // (same for the whole grid)
         // k = K .. K + kpeel - 1 as the first values of one 16-wide MFMA step: the lower half-wave holds k 0..7 of its
         // row of B / column of A, the upper half-wave zeros.
-        const unsigned short* Ap = A + (int64_t)bz * sa + (int64_t)K * lda;
-        const unsigned short* Bp = B + (int64_t)bz * sb + K;
+        const unsigned short* Ap = A + (int64_t)bz * sa + (k_first + K) * lda;
+        const unsigned short* Bp = B + (int64_t)bz * sb + k_first + K;
         Frag fp;
         const bool lower = lane < 32;
 #pragma unroll
@@ -309,44 +314,17 @@ __global__ __launch_bounds__(256) void gemm16_big(const unsigned short* __restri
         mma16<E, I, J>(fp, acc);
     }
 
-    // Epilogue.  The lane's own offset (m within the wave tile, plus its 4*hb rows of n) is a
-    // 32-bit element offset; the part of n that is uniform across the wave goes into the base.
-    const unsigned lane_off = (unsigned)((lane & 31) + (int64_t)(4 * (lane >> 5)) * ldc);
-    OutT* Cw = C + (int64_t)bm * BTM + wm + ((int64_t)bn * BTN + wn) * ldc;
-    if ((bm + 1) * BTM <= M && (bn + 1) * BTN <= N) {   // interior tile (same for the whole workgroup)
-#pragma unroll
-        for (int i = 0; i < I; ++i)
-#pragma unroll
-            for (int j = 0; j < J; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    OutT* cu = Cw + 32 * i + (int64_t)(32 * j + 8 * (r >> 2) + (r & 3)) * ldc;
-                    __builtin_nontemporal_store(cvt_out<E, OutT>(acc[i][j][r]), cu + lane_off);
-                }
-    } else {                                          // edge tile: clip to the matrix
-        int m_left = M - (bm * BTM + wm + (lane & 31)), n_left = N - (bn * BTN + wn + 4 * (lane >> 5));
-#pragma unroll
-        for (int i = 0; i < I; ++i)
-#pragma unroll
-            for (int j = 0; j < J; ++j)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    // the empty statement keeps each test next to its store (256 hoisted lane masks would
-                    // not fit the scalar registers)
-                    asm volatile("" : "+v"(m_left), "+v"(n_left));
-                    const int dn = 32 * j + 8 * (r >> 2) + (r & 3);
-                    if (32 * i < m_left && dn < n_left) {
-                        float v = acc[i][j][r];
-                        asm volatile("" : "+v"(v));   // convert after the test, not 256 values ahead of it
-                        __builtin_nontemporal_store(cvt_out<E, OutT>(v), Cw + 32 * i + (int64_t)dn * ldc + lane_off);
-                    }
-                }
-    }
+    store_tile<E, OutT, I, J>(acc, C, ldc, M, N, bm * BTM, bn * BTN, wm, wn, BTM, BTN, lane);
 }
 
 // The extent of K that the transfers walk: whole chunks of 8, and not the last row of A when a chunk of A can straddle
 // the end of a row (M not a multiple of 8).
 int dma_extent(const Problem& p) { return p.M % 8 ? (p.K - 1) / 8 * 8 : p.K / 8 * 8; }
+
+// Rows of A or B that start off 16-byte boundaries.
+bool misaligned(const Problem& p) {
+    return p.lda % 8 || p.ldb % 8 || (p.batch > 1 && (p.sa % 8 || p.sb % 8)) || !aligned(p.A, 16) || !aligned(p.B, 16);
+}
 
 template <typename E, typename OutT, int I, int J>
 void launch(const Problem& p, hipStream_t s) {
@@ -363,36 +341,51 @@ void launch(const Problem& p, hipStream_t s) {
 // point has no workspace argument (it mirrors the reference's kernel signature), so the partial sums live in a
 // static device array of the library, 16 MiB per GPU.  Launches that use it are ordered by an event when they
 // come from different streams; a stream that is being captured into a graph does not use it.
+// Any M and K: the values of k behind the transfers' extent are the last part's.  (us: 256 x 640 x 2561 84 on 64 x 64 tiles -> 11,
+// 320 x 576 x 3533 119 -> 14.6, 949 x 512 x 3520 38 -> 17, 640 x 704 x 2839 31.8 -> 14.1.)
 constexpr int64_t kSplitFloats = 4 * 1024 * 1024;
 static __device__ __align__(256) float splitk_scratch[kSplitFloats];
 
 template <typename OutT>
 __global__ __launch_bounds__(256) void splitk_reduce(const float* __restrict__ part, int ksplit, OutT* __restrict__ C,
                                                      int64_t ldc, int64_t sc, int M, int N, int batch, bool bf16) {
-    // one lane: 4 consecutive m of one column (M is a multiple of 8)
-    const int64_t quads = (int64_t)(M / 4) * N * batch;
+    // one lane: 4 consecutive m of one column (the last of a column may be fewer)
+    typedef f32x4 f32x4_a4 __attribute__((aligned(4)));
+    const int col = (M + 3) / 4;
+    const int64_t quads = (int64_t)col * N * batch;
     const int64_t MN = (int64_t)M * N;
     for (int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x; q < quads; q += (int64_t)gridDim.x * 256) {
-        const int m4 = (int)(q % (M / 4)), n = (int)((q / (M / 4)) % N), bz = (int)(q / ((int64_t)(M / 4) * N));
+        const int m4 = (int)(q % col), n = (int)((q / col) % N), bz = (int)(q / ((int64_t)col * N));
+        const int have = M - 4 * m4 < 4 ? M - 4 * m4 : 4;
         const float* src = part + (int64_t)bz * ksplit * MN + (int64_t)n * M + 4 * m4;
         // parts added in index order (the result does not depend on timing); four loads in flight at a time
-        f32x4 acc = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(src));
-        int ks = 1;
-        for (; ks + 4 <= ksplit; ks += 4) {
-            f32x4 v[4];
+        f32x4 acc;
+        if (have == 4) {
+            acc = __builtin_nontemporal_load(reinterpret_cast<const f32x4_a4*>(src));
+            int ks = 1;
+            for (; ks + 4 <= ksplit; ks += 4) {
+                f32x4 v[4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) v[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(src + (ks + u) * MN));
+                for (int u = 0; u < 4; ++u) v[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4_a4*>(src + (ks + u) * MN));
 #pragma unroll
-            for (int u = 0; u < 4; ++u) acc += v[u];
-        }
-        for (; ks < ksplit; ++ks) acc += __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(src + ks * MN));
-        OutT* dst = C + (int64_t)bz * sc + (int64_t)n * ldc + 4 * m4;
-        if constexpr (sizeof(OutT) == 4) {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) dst[e] = acc[e];
+                for (int u = 0; u < 4; ++u) acc += v[u];
+            }
+            for (; ks < ksplit; ++ks) acc += __builtin_nontemporal_load(reinterpret_cast<const f32x4_a4*>(src + ks * MN));
         } else {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) dst[e] = bf16 ? BF16::from_f32(acc[e]) : F16::from_f32(acc[e]);
+            for (int e = 0; e < 3; ++e) {
+                acc[e] = 0.f;
+                if (e >= have) continue;
+                acc[e] = src[e];
+                for (int ks = 1; ks < ksplit; ++ks) acc[e] += src[ks * MN + e];
+            }
+        }
+        OutT* dst = C + (int64_t)bz * sc + (int64_t)n * ldc + 4 * m4;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if (e >= have) break;
+            if constexpr (sizeof(OutT) == 4) dst[e] = acc[e];
+            else dst[e] = bf16 ? BF16::from_f32(acc[e]) : F16::from_f32(acc[e]);
         }
     }
 }
@@ -402,23 +395,25 @@ SharedScratch g_split[16];
 // Parts and part length for the problem, or 0 if a split does not apply.
 int pick_split(const Problem& p, int* kchunk) {
     static const int force = [] { const char* e = getenv("MI_GEMM_SPLITK"); return e ? atoi(e) : -1; }();   // 0 = never, n = n parts
-    if (force == 0 || p.M % 8 || p.K % 8) return 0;   // (the parts and the kernel that adds them move whole vectors)
+    if (force == 0) return 0;
     const int64_t tiles = tiles_of(p, 128, 128);
+    const int kd = dma_extent(p);
+    const bool mis = misaligned(p);
     // (up to half a tile per CU: 2048 x 768 x 8192, 96 tiles, 59 -> 41 us with two parts; 1152 x 1024 x 16384 107 -> 55 us
     // with three; beyond 128 tiles the estimate below never favours a split)
-    if (tiles > 128 || p.K < 1024) return 0;
-    // Estimated times in us: one launch walks K / 32 steps of 0.18 us; the split pays a second launch, the partial
-    // sums written and read again (at about 3 bytes per ns), and walks a part's steps only.
-    const double t_plain = 3.0 + 0.18 * (p.K / 32.0);
+    if (tiles > 128 || p.K < (mis ? 768 : 1024)) return 0;
+    // Estimated times in us: one launch walks K / 32 steps of 0.18 us (0.3 where rows are not aligned); the split pays a
+    // second launch, the partial sums written and read again (at about 3 bytes per ns), and walks a part's steps only.
+    const double step = mis ? 0.30 : 0.18, t_plain = 3.0 + step * (p.K / 32.0);
     const double mn_bytes = 4.0 * p.M * p.N * p.batch;
     int best = 0;
     double t_best = 0.85 * t_plain;   // (a split has to be clearly better)
     for (int parts = force > 1 ? force : 2; parts <= (force > 1 ? force : 16); ++parts) {
         if (parts * tiles > 512) break;
-        const int chunk = ((p.K + parts - 1) / parts + 127) / 128 * 128;        // whole groups of four K steps
-        const int n = (p.K + chunk - 1) / chunk;
-        if (n < 2 || chunk < 256 || p.K - (n - 1) * chunk < 256 || (int64_t)n * p.M * p.N * p.batch > kSplitFloats) continue;
-        const double t = 7.0 + 0.18 * (chunk / 32.0) + (n + 1) * mn_bytes / 3.0e6 + (n * tiles > 256 ? 0.18 * (chunk / 32.0) : 0.0);
+        const int chunk = ((kd + parts - 1) / parts + 127) / 128 * 128;         // whole groups of four K steps
+        const int n = (kd + chunk - 1) / chunk;
+        if (n < 2 || chunk < 256 || kd - (n - 1) * chunk < 256 || (int64_t)n * p.M * p.N * p.batch > kSplitFloats) continue;
+        const double t = 7.0 + step * (chunk / 32.0) + (n + 1) * mn_bytes / 3.0e6 + (n * tiles > 256 ? step * (chunk / 32.0) : 0.0);
         if (t < t_best || (force > 1 && !best)) {
             t_best = t;
             best = n;
@@ -437,8 +432,8 @@ bool launch_split(const Problem& p, hipStream_t s, int parts, int kchunk) {
     const int64_t MN = (int64_t)p.M * p.N;
     hipLaunchKernelGGL((gemm16_big<E, float, 2, 2>), dim3((unsigned)(tiles_m * tiles_n * p.batch * parts)), dim3(256), 0, s,
                        (const unsigned short*)p.A, p.lda, p.sa, (const unsigned short*)p.B, p.ldb, p.sb, scratch,
-                       (int64_t)p.M, MN, p.M, p.N, p.K, tiles_m, tiles_n, p.batch, parts, kchunk, 0);
-    const int64_t quads = MN / 4 * p.batch;
+                       (int64_t)p.M, MN, p.M, p.N, dma_extent(p), tiles_m, tiles_n, p.batch, parts, kchunk, p.K - dma_extent(p));
+    const int64_t quads = (int64_t)((p.M + 3) / 4) * p.N * p.batch;
     const unsigned blocks = (unsigned)((quads + 255) / 256 < 2048 ? (quads + 255) / 256 : 2048);
     if (p.out_dtype == MI_F32)
         hipLaunchKernelGGL((splitk_reduce<float>), dim3(blocks), dim3(256), 0, s, scratch, parts, (float*)p.C, p.ldc,
@@ -456,14 +451,14 @@ namespace gemm {
 
 bool big16_applicable(const Problem& p) {
     if (p.in_dtype != MI_F16 && p.in_dtype != MI_BF16) return false;
-    const int64_t tiles = tiles_of(p, 128, 128);   // (from 16 tiles of 128x128 on, this kernel is no slower than 64x64 tiles)
-    int split = 0, kchunk = 0;
+    // From 16 tiles of 128x128 on, this kernel is no slower than 64x64 tiles, and from K = 320 on with fewer (us, 64x64 -> this:
+    // 384 x 256 x 512 12.8 -> 6.5, 448 x 384 x 640 15.5 -> 8.6, 445 x 261 x 512 13.2 -> 9.6).
+    const int64_t tiles = tiles_of(p, 128, 128);
     return p.M >= 8 && p.N >= 1 && p.K >= 256 + 8 * (p.K % 8 != 0 || p.M % 8 != 0) && p.ldc < (1 << 26) &&
            // (the kernel's 32-bit lane offsets assume rows that follow each other upwards in memory)
            p.lda >= p.M && p.ldb >= p.K && p.ldc >= p.M && p.sa >= 0 && p.sb >= 0 && p.sc >= 0 &&
            p.lda < (1 << 26) && p.ldb < (1 << 26) && tiles < (1 << 30) &&
-           // (fewer than 16 tiles only when the split over K multiplies the workgroups)
-           (tiles >= 16 || (split = pick_split(p, &kchunk), (int64_t)split * tiles >= 16));
+           (tiles >= 16 || p.K >= 320);
 }
 
 void big16_launch(const Problem& p, hipStream_t s) {
@@ -479,6 +474,14 @@ void big16_launch(const Problem& p, hipStream_t s) {
             "gemm16_big_128x128x32_ring4_splitk13", "gemm16_big_128x128x32_ring4_splitk14", "gemm16_big_128x128x32_ring4_splitk15",
             "gemm16_big_128x128x32_ring4_splitk16"};
         set_variant(names[parts]);
+        return;
+    }
+    // Rows off 16-byte boundaries cost the path into LDS twice the time, and waves that only transfer lose none of the matrix
+    // cores' meanwhile (gemm_pc.hip; one workgroup per CU).  With K below about 1000 the two kernels are within 3 % either
+    // way, and so they are with aligned rows.
+    if (t != 44 && p.K >= 1000 && misaligned(p) && tiles_of(p, t == 22 ? 128 : 256, 128) <= 256) {
+        pc16_launch(p, t, dma_extent(p), 1, 0, s);
+        set_variant(t == 22 ? "gemm16_big_128x128x64_ring3" : "gemm16_big_256x128x64_ring3");
         return;
     }
 #define BIG(E, O) (t == 22 ? launch<E, O, 2, 2>(p, s) : t == 42 ? launch<E, O, 4, 2>(p, s) : launch<E, O, 4, 4>(p, s))

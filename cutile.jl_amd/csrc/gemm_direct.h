@@ -31,6 +31,55 @@ __device__ __forceinline__ void stage_barrier() {
     asm volatile("" ::: "memory");
 }
 
+// Workgroup ids congruent mod 8 share an XCD and its L2: each XCD gets a contiguous run of the tiles, so that it works on
+// neighbouring ones.  From 64 tiles on also where they are no multiple of 8 (2200 x 1100 x 4000 bf16 38.4 -> 36.8 us,
+// 3667 x 407 x 384 10.0 -> 9.3); fewer are better spread (60 tiles, 1536 x 640 x 1280: 13.5 spread, 14.3 in runs).
+__device__ __forceinline__ int xcd_tile(int id, int total) {
+    const int x = id & 7, each = total >> 3, more = total & 7;
+    if (more && total < 64) return id;
+    return x * each + (x < more ? x : more) + (id >> 3);
+}
+
+// Stores a wave's (32*I) x (32*J) part (wm, wn) of the BTM x BTN tile at (m0, n0): the lane's column of an MFMA tile is m,
+// its rows are n, so a half-wave stores 32 consecutive m of one column of C.
+template <typename E, typename OutT, int I, int J>
+__device__ __forceinline__ void store_tile(const f32x16 (&acc)[I][J], OutT* C, int64_t ldc, int M, int N, int m0, int n0, int wm, int wn,
+                                           int btm, int btn, int lane) {
+    // The lane's own offset (m within the wave tile, plus its 4*hb rows of n) is a 32-bit element offset; the part of n
+    // that is uniform across the wave goes into the base.
+    const unsigned lane_off = (unsigned)((lane & 31) + (int64_t)(4 * (lane >> 5)) * ldc);
+    OutT* Cw = C + (int64_t)m0 + wm + ((int64_t)n0 + wn) * ldc;
+    if (m0 + btm <= M && n0 + btn <= N) {   // interior tile (same for the whole workgroup)
+#pragma unroll
+        for (int i = 0; i < I; ++i)
+#pragma unroll
+            for (int j = 0; j < J; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    OutT* cu = Cw + 32 * i + (int64_t)(32 * j + 8 * (r >> 2) + (r & 3)) * ldc;
+                    __builtin_nontemporal_store(cvt_out<E, OutT>(acc[i][j][r]), cu + lane_off);
+                }
+    } else {                                // edge tile: clip to the matrix
+        int m_left = M - (m0 + wm + (lane & 31)), n_left = N - (n0 + wn + 4 * (lane >> 5));
+#pragma unroll
+        for (int i = 0; i < I; ++i)
+#pragma unroll
+            for (int j = 0; j < J; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    // the empty statement keeps each test next to its store (256 hoisted lane masks would
+                    // not fit the scalar registers)
+                    asm volatile("" : "+v"(m_left), "+v"(n_left));
+                    const int dn = 32 * j + 8 * (r >> 2) + (r & 3);
+                    if (32 * i < m_left && dn < n_left) {
+                        float v = acc[i][j][r];
+                        asm volatile("" : "+v"(v));   // convert after the test, not 256 values ahead of it
+                        __builtin_nontemporal_store(cvt_out<E, OutT>(v), Cw + 32 * i + (int64_t)dn * ldc + lane_off);
+                    }
+                }
+    }
+}
+
 inline int64_t tiles_of(const Problem& p, int btm, int btn) {
     return (int64_t)((p.M + btm - 1) / btm) * ((p.N + btn - 1) / btn) * p.batch;
 }
@@ -51,6 +100,10 @@ inline int pick_direct_tile(const Problem& p, int64_t* cost = nullptr) {
     if (force == 44 || force == 42 || force == 22) return force;
     return t;
 }
+
+// gemm_pc.hip: the kernel whose transfers have waves of their own, with tiles of 256 x 128 (tile = 42) or 128 x 128 (22); kd: the
+// extent of K that the transfers walk; parts > 1: split over K in parts of kchunk into slices of C (see gemm_big.hip).
+void pc16_launch(const Problem& p, int tile, int kd, int parts, int kchunk, hipStream_t s);
 
 }  // namespace gemm
 }  // namespace mi

@@ -220,6 +220,54 @@ def test_matmul_split_over_k_on_misaligned_rows(ct, orc, M, N, K, pad):
     assert np.array_equal(orc.to_julia(C), A @ B)
 
 
+@pytest.mark.parametrize("M,N,K,T,out32,pad,name", [
+    # transfers by waves of their own: rows off 16-byte boundaries, K from 1000 on, at most 256 tiles
+    (1001, 1800, 1000, torch.float16, True, (0, 0), "gemm16_big_128x128x64_ring3"),     # odd M: K - Kd = 8
+    (1408, 1408, 1025, torch.bfloat16, False, (0, 0), "gemm16_big_128x128x64_ring3"),   # whole tiles, odd K
+    (1536, 1500, 1088, torch.float16, True, (3, 5), "gemm16_big_128x128x64_ring3"),     # whole stages, K - Kd = 0
+    (2047, 2051, 1031, torch.bfloat16, True, (0, 0), "gemm16_big_256x128x64_ring3"),
+    (3001, 2000, 1003, torch.float16, False, (1, 2), "gemm16_big_256x128x64_ring3"),
+    # split over K with M and K off the chunks: columns of C that end in 1, 2 and 3 values, K - Kd = 1, 7, 8
+    (257, 640, 2561, torch.float16, True, (0, 0), "gemm16_big_128x128x32_ring4_splitk"),
+    (322, 575, 3535, torch.bfloat16, False, (0, 0), "gemm16_big_128x128x32_ring4_splitk"),
+    (949, 512, 3520, torch.float16, False, (2, 1), "gemm16_big_128x128x32_ring4_splitk"),
+    (9, 300, 2056, torch.float16, True, (0, 0), "gemm16_big_128x128x32_ring4_splitk"),
+    # fewer than 16 tiles from K = 320 on
+    (264, 300, 320, torch.float16, True, (0, 0), "gemm16_big_128x128x32_ring4"),
+    (131, 129, 327, torch.bfloat16, False, (0, 0), "gemm16_big_128x128x32_ring4"),
+])
+def test_matmul_ragged_sizes_split_or_with_transfer_waves_exact(ct, orc, M, N, K, T, out32, pad, name):
+    """Exact integer sums; NaN right behind every row of A and B and behind the arrays, C a view of a buffer with a sentinel."""
+    rng = np.random.default_rng(M + K)
+    A = rng.integers(-1, 2, (M, K)).astype(np.float32); B = rng.integers(-1, 2, (K, N)).astype(np.float32)
+    lda, ldb = M + pad[0], K + pad[1]
+    Aflat = torch.full((K * lda + 16,), float("nan"), dtype=T, device="cuda")
+    Bflat = torch.full((N * ldb + 16,), float("nan"), dtype=T, device="cuda")
+    Av = Aflat[:K * lda].view(K, lda)[:, :M]; Bv = Bflat[:N * ldb].view(N, ldb)[:, :K]
+    Av.copy_(orc.from_julia(A).to(T)); Bv.copy_(orc.from_julia(B).to(T))
+    buf = torch.full((N + 2, M + 9), -77.0, dtype=torch.float32 if out32 else T, device="cuda")
+    C = buf[:N, :M]
+    ct.matmul_kernel(Av, Bv, C, 64, 64, 64)
+    assert ct.last_variant() == name or (name.endswith("splitk") and ct.last_variant().startswith(name)), ct.last_variant()
+    ref = A @ B
+    assert out32 or np.abs(ref).max() <= (2048 if T == torch.float16 else 256)
+    assert np.array_equal(orc.to_julia(C.contiguous()).astype(np.float32), ref)
+    assert bool((buf[N:] == -77.0).all()) and bool((buf[:, M:] == -77.0).all())
+
+
+def test_batch_matmul_ragged_split_and_transfer_waves(ct, orc):
+    """The same through mi_batch_matmul_kernel: odd batch strides, parts of every entry in slices of their own."""
+    rng = np.random.default_rng(12)
+    for M, N, K, nb, name in ((131, 260, 2049, 3, "gemm16_big_128x128x32_ring4_splitk"), (515, 1030, 1001, 3, "gemm16_big_128x128x64_ring3")):
+        A = rng.integers(-1, 2, (M, K, nb)).astype(np.float32); B = rng.integers(-1, 2, (K, N, nb)).astype(np.float32)
+        At = orc.from_julia(A).to(torch.float16).cuda(); Bt = orc.from_julia(B).to(torch.float16).cuda()
+        C = torch.empty((nb, N, M), dtype=torch.float32, device="cuda")
+        ct.batch_matmul_kernel(At, Bt, C, 64, 64, 64)
+        assert ct.last_variant().startswith(name), ct.last_variant()
+        ref = np.stack([np.ascontiguousarray(A[:, :, b]) @ np.ascontiguousarray(B[:, :, b]) for b in range(nb)], axis=2)
+        assert np.array_equal(orc.to_julia(C), ref)
+
+
 def test_matmul_split_over_k_is_reproducible_and_ordered_across_streams(ct, orc):
     """The parts are added in a fixed order, so two runs give the same bits; launches from two streams share the
     scratch and are ordered by the library, so alternating between streams still gives every product its own
