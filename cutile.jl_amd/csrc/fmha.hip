@@ -22,8 +22,10 @@
 //     matching row operand is read from the V tile with the LDS transpose read, whose
 //     4-consecutive-row granularity matches the accumulator's 4-row groups, so P never
 //     moves between lanes.
-// Causal balance: with causal masking a wave takes the 32-query tiles u and NT-1-u, so every
-// wave walks the same number of KV tiles.  All query tiles of a (batch, head) run on one XCD.
+// Causal balance: D = 64, a wave takes the 32-query tiles u and NT-1-u, so every wave walks the same number of KV tiles; D =
+// 128, the long walks of all of an XCD's heads start first (head by head, the last head's longest walk started when most of
+// the chip was idle: 7 x 4 heads, S = 3433 123 us, now 106, 8 x 16, 619 36 -> 26, 5 x 4, 4000 193 -> 113, 4 x 16, 2213 124 -> 107).
+// All query tiles of a (batch, head) run on one XCD, with those of the heads that share its K / V where their number allows it.
 // Causal tile skipping: the KV loop stops at the workgroup's last query, and a wave skips
 // tiles that lie wholly above its own last query.  Masking and the ragged KV tail use -Inf
 // as in the reference (fmha.jl:92-103).
@@ -34,6 +36,12 @@
 // the library, and fmha_combine_kernel adds the parts with the usual exp2(m_part - m) weights.  A part may start
 // above a query's diagonal, so a row can go through tiles without a visible key: its maximum stays -Inf and the
 // weights are taken against 0 instead (SAFE), which keeps them at exp2(-Inf) = 0 rather than exp2(-Inf + Inf).
+//
+// Heads of 128 with about one workgroup per CU and a walk of eight tiles or more (pick_inside): two groups of four waves
+// share a workgroup's queries and take every other tile (KG = 2), so that a SIMD has two waves to choose from; their
+// accumulators meet in LDS.  Bound then by the SIMDs' issue of exponentials and products: 1.03 us a tile, 1.37 with one
+// group.  The weights refer to each tile's own maximum (OWN), so that no result is further from float64 than the split
+// over workgroups, which has a maximum per part, left it (180 shapes: 0.95 to 1.00 of its error; 1.03 with one reference).
 //
 // Grouped heads with few queries (`pack` = QUERY_GROUP_SIZE when Sq <= 64): the heads that share a K / V head are
 // stacked as rows of one query tile -- row r is query r % Sq of head r / Sq of the group -- so their common keys are
@@ -300,6 +308,7 @@ struct FmhaDma {
         s16x8 qf[JT][KSTEPS];
         f32x16 o[JT][DT];
         float m[JT], l[JT];
+        float top[JT];         // OWN: the running maximum; m is then the latest tile's, at most 8 below it
         unsigned kfo[KSTEPS];  // K fragment element offsets per k-step (+ 32*kt*D)
         unsigned vfo[DT];      // V fragment element offsets per d tile (+ (32*kt + 16*c)*D, + 8*D for the high half)
         int my_pos[JT];     // position of this lane's query in column tile j
@@ -324,7 +333,9 @@ struct FmhaDma {
 
     // JM: bit j set = column tile j takes part in this KV tile (a causal wave drops its early
     // query tile once the keys pass that tile's diagonal).
-    template <int JM, bool SAFE = false>
+    // OWN: the weights of a tile refer to that tile's own maximum (at most 2^8 below the running one), so that every tile's
+    // largest weight is rounded without error; the accumulators are then rescaled at nearly every tile.
+    template <int JM, bool SAFE = false, bool OWN = false>
     static __device__ __forceinline__ void compute(const unsigned short* Ks, const unsigned short* Vs, State& st,
                                                    int kv0, int Skv, float scale2, int lane) {
         const int hb = lane >> 5;
@@ -368,8 +379,12 @@ struct FmhaDma {
 #pragma unroll
             for (int r = 1; r < 16; ++r) mx = fmaxf(fmaxf(mx, s[j][0][r]), s[j][1][r]);
             mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-            const float m_new = fmaxf(st.m[j], mx * scale2);
-            if (__any(m_new > st.m[j])) {  // some row's max rose: rescale the wave's accumulators
+            float m_new = fmaxf(st.m[j], mx * scale2);
+            if constexpr (OWN) {
+                st.top[j] = fmaxf(st.top[j], mx * scale2);
+                m_new = fmaxf(mx * scale2, st.top[j] - 8.f);
+            }
+            if (OWN ? __any(m_new != st.m[j]) : __any(m_new > st.m[j])) {  // some row's max rose: rescale the wave's accumulators
                 // (SAFE: a row that has not seen a key yet keeps l = 0 and o = 0)
                 const float alpha = __builtin_amdgcn_exp2f(st.m[j] - (SAFE && m_new == -INFINITY ? 0.f : m_new));
                 st.l[j] *= alpha;
@@ -433,8 +448,10 @@ constexpr int kFuseRows = 64;      // most rows per (batch, head) for that
 constexpr int kFusePairs = 65536;  // most (query block, batch * head) pairs for that
 constexpr int kPartPad = 4;   // a part's row: D accumulator values, running maximum, row sum, two unused (16-byte rows)
 
-template <typename E, int D, int JT, bool CAUSAL, bool SPLIT = false>
-__global__ __launch_bounds__(128 * 2 / JT) __attribute__((amdgpu_waves_per_eu(2, 2))) void fmha_fwd_dma_kernel(
+// KG > 1: KG groups of NW waves share the workgroup's queries and take every KG-th key tile each, on K / V stages of their
+// own; at the end the groups' accumulators meet in LDS.
+template <typename E, int D, int JT, bool CAUSAL, bool SPLIT = false, int KG = 1>
+__global__ __launch_bounds__(128 * 2 / JT * KG) __attribute__((amdgpu_waves_per_eu(2, 2))) void fmha_fwd_dma_kernel(
     const unsigned short* __restrict__ Q, Strides qs, const unsigned short* __restrict__ K, Strides ks,
     const unsigned short* __restrict__ V, Strides vs, unsigned short* __restrict__ O, Strides os, int Sq, int Skv,
     int H, int group, float scale2, int input_pos, int nqb, int nbh, int pack, int kv_stream, int nsplit = 1,
@@ -442,10 +459,14 @@ __global__ __launch_bounds__(128 * 2 / JT) __attribute__((amdgpu_waves_per_eu(2,
     using F = FmhaDma<E, D, JT, CAUSAL>;
     constexpr int NW = F::NW, KSTEPS = F::KSTEPS, DT = F::DT, CH = F::CH, TPW = F::TPW;
     constexpr bool PAIRED = CAUSAL && JT == 2;
-    __shared__ __attribute__((aligned(1024))) unsigned short Ks0[F::TILE], Ks1[F::TILE], Vs0[F::TILE], Vs1[F::TILE];
+    static_assert(KG == 1 || !SPLIT, "keys are split over workgroups or inside one");
+    constexpr bool SAFE = SPLIT || KG > 1;   // a row may have no key in a part
+    __shared__ __attribute__((aligned(1024))) unsigned short Ks0a[KG * F::TILE], Ks1a[KG * F::TILE], Vs0a[KG * F::TILE], Vs1a[KG * F::TILE];
 
     const int tid = threadIdx.x, lane = tid & 63, hb = lane >> 5;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave_wg = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wave = wave_wg % NW, grp = KG > 1 ? wave_wg / NW : 0;
+    unsigned short *const Ks0 = Ks0a + grp * F::TILE, *const Ks1 = Ks1a + grp * F::TILE, *const Vs0 = Vs0a + grp * F::TILE, *const Vs1 = Vs1a + grp * F::TILE;
     // Workgroup -> (query block, batch*head): ids congruent mod 8 share an XCD; give each XCD
     // whole (batch, head) pairs so their K/V stay in that XCD's L2.  Low block index = most work.
     int qb, bh, sp = 0;
@@ -455,14 +476,13 @@ __global__ __launch_bounds__(128 * 2 / JT) __attribute__((amdgpu_waves_per_eu(2,
             sp = L / (nqb * nbh);
             L -= sp * (nqb * nbh);
         }
-        if (nbh % 8 == 0) {
-            const int idx = L >> 3;
-            bh = (L & 7) + 8 * (idx / nqb);
-            qb = idx % nqb;
-        } else {
-            bh = L / nqb;
-            qb = L % nqb;
-        }
+        // Causal with equal query tiles: the long walks of all of an XCD's heads start first, so that what starts last is short
+        // (head by head, the last head's longest walk starts when nearly everything else has ended).
+        constexpr bool LONGEST = CAUSAL && !PAIRED && !SPLIT;
+        const int nx = nbh % 8 == 0 ? 8 : 1, idx = L / nx, per = nbh / nx, j = LONGEST ? idx % per : idx / nqb;
+        qb = LONGEST ? idx / per : idx % nqb;
+        const int gm = nx == 8 && pack == 1 && (nbh / group) % 8 == 0 ? group : 1;   // an XCD gets all heads that share a K / V head
+        bh = (L % nx + nx * (j / gm)) * gm + j % gm;
         if (CAUSAL && !PAIRED) qb = nqb - 1 - qb;
     }
     // (pack > 1: bh counts (batch, K / V head) pairs, H is their number per batch, and a row carries its head)
@@ -517,7 +537,7 @@ __global__ __launch_bounds__(128 * 2 / JT) __attribute__((amdgpu_waves_per_eu(2,
         }
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) st.o[j][dt] = f32x16{0};
-        st.m[j] = -INFINITY;
+        st.m[j] = st.top[j] = -INFINITY;
         st.l[j] = 0.f;
     }
     {
@@ -580,23 +600,88 @@ __global__ __launch_bounds__(128 * 2 / JT) __attribute__((amdgpu_waves_per_eu(2,
         if (JT == 2) {
             const bool a0 = tq[0] >= 0 && (!CAUSAL || kv0 <= last_pos[0]);
             const bool a1 = tq[JT - 1] >= 0 && (!CAUSAL || kv0 <= last_pos[JT - 1]);
-            if (a0 && a1) F::template compute<3, SPLIT>(Ksx, Vsx, st, kv0, Skv, scale2, lane);
-            else if (a1) F::template compute<2, SPLIT>(Ksx, Vsx, st, kv0, Skv, scale2, lane);
-            else if (a0) F::template compute<1, SPLIT>(Ksx, Vsx, st, kv0, Skv, scale2, lane);
+            if (a0 && a1) F::template compute<3, SAFE, KG != 1>(Ksx, Vsx, st, kv0, Skv, scale2, lane);
+            else if (a1) F::template compute<2, SAFE, KG != 1>(Ksx, Vsx, st, kv0, Skv, scale2, lane);
+            else if (a0) F::template compute<1, SAFE, KG != 1>(Ksx, Vsx, st, kv0, Skv, scale2, lane);
         } else {
-            if (tq[0] >= 0 && (!CAUSAL || kv0 <= last_pos[0])) F::template compute<1, SPLIT>(Ksx, Vsx, st, kv0, Skv, scale2, lane);
+            if (tq[0] >= 0 && (!CAUSAL || kv0 <= last_pos[0])) F::template compute<1, SAFE, KG != 1>(Ksx, Vsx, st, kv0, Skv, scale2, lane);
         }
     };
 
-    if (t_begin < t_end) issue_tile(t_begin, Ks0, Vs0);
-    for (int t = t_begin; t < t_end; t += 2) {
+    // (KG > 1: group grp takes the tiles grp, grp + KG, ...; every group passes the same barriers)
+    const int t_first = t_begin + grp, t_meet = KG > 1 ? t_end + KG - 1 - (t_end + KG - 1 - t_begin) % KG : t_end;
+    if (t_first < t_end) issue_tile(t_first, Ks0, Vs0);
+    for (int t = t_first, b = t_begin; b < t_meet; t += 2 * KG, b += 2 * KG) {
         tile_barrier();  // tile t has landed for every wave; every wave is done with the other stage
-        if (t + 1 < t_end) issue_tile(t + 1, Ks1, Vs1);
-        run_tile(Ks0, Vs0, t * kKV);
-        if (t + 1 < t_end) {
+        if (t + KG < t_end) issue_tile(t + KG, Ks1, Vs1);
+        if (KG == 1 || t < t_end) run_tile(Ks0, Vs0, t * kKV);
+        if (b + KG < t_meet) {
             tile_barrier();
-            if (t + 2 < t_end) issue_tile(t + 2, Ks0, Vs0);
-            run_tile(Ks1, Vs1, (t + 1) * kKV);
+            if (t + 2 * KG < t_end) issue_tile(t + 2 * KG, Ks0, Vs0);
+            if (KG == 1 || t + KG < t_end) run_tile(Ks1, Vs1, (t + KG) * kKV);
+        }
+    }
+
+    if constexpr (KG > 1) {
+        // ---- the other groups' accumulators, maxima and row sums through LDS to the first group ----
+        constexpr int REGS = JT * DT * 16;                             // accumulators per lane
+        constexpr int DUMP = REGS * 64 * 4;                            // bytes of a wave's
+        constexpr int PER = KG * F::TILE * 2 / DUMP;                   // waves whose accumulators one array of stages holds
+        static_assert(PER >= 1 && (KG - 1) * NW <= 4 * PER, "the stages hold the accumulators");
+        __shared__ float s_ml[(KG - 1) * NW][2 * JT][64];
+        tile_barrier();   // every wave is done with the stages
+        auto dump = [&](int slot) {
+            const int arr = slot / PER;
+            return (f32x4*)(arr == 0 ? Ks0a : arr == 1 ? Ks1a : arr == 2 ? Vs0a : Vs1a) + (slot % PER) * (DUMP / 16) + lane;
+        };
+        if (grp > 0) {
+            const int slot = (grp - 1) * NW + wave;
+            f32x4* p = dump(slot);
+#pragma unroll
+            for (int j = 0; j < JT; ++j) {
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) {
+                        f32x4 w;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) w[e] = st.o[j][dt][4 * g + e];
+                        p[((j * DT + dt) * 4 + g) * 64] = w;
+                    }
+                s_ml[slot][2 * j][lane] = st.m[j];
+                s_ml[slot][2 * j + 1][lane] = st.l[j];
+            }
+        }
+        tile_barrier();
+        if (grp > 0) return;
+#pragma unroll
+        for (int j = 0; j < JT; ++j) {
+            float m = st.m[j];
+#pragma unroll
+            for (int q = 0; q < KG - 1; ++q) m = fmaxf(m, s_ml[q * NW + wave][2 * j][lane]);
+            // (a group without a visible key for the row has m = -inf, l = 0 and o = 0)
+            const float mref = m == -INFINITY ? 0.f : m;
+            const float w0 = __builtin_amdgcn_exp2f(st.m[j] - mref);
+            st.l[j] *= w0;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) st.o[j][dt][r] *= w0;
+#pragma unroll
+            for (int q = 0; q < KG - 1; ++q) {
+                const int slot = q * NW + wave;
+                const f32x4* p = dump(slot);
+                const float w = __builtin_amdgcn_exp2f(s_ml[slot][2 * j][lane] - mref);
+                st.l[j] += w * s_ml[slot][2 * j + 1][lane];
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) {
+                        const f32x4 v = p[((j * DT + dt) * 4 + g) * 64];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) st.o[j][dt][4 * g + e] += w * v[e];
+                    }
+            }
         }
     }
 
@@ -811,6 +896,34 @@ int pick_parts(int64_t wgs, int64_t rows, int D, int Sq, int Skv, bool causal, i
     return parts >= 2 ? (int)parts : 0;
 }
 
+// Heads of 128, more than 64 queries: true where a workgroup of two groups of waves that share its queries and take every
+// other key tile each (one workgroup per CU) is the quickest.  One walk per wave leaves a CU with one wave per SIMD, which
+// waits for its own chain of products, exponentials and products; a split over workgroups writes and reads 528 bytes a row
+// and part.  Estimates in us, from 270 shapes (1 to 8 batches of 1 to 32 heads, 256 to 5000 queries): two groups 6.5 + 1.03 a
+// tile of 64 keys, the split 5 + its parts at 4 bytes per ns + 1.9 a tile at two workgroups per CU; both come out within 8 %,
+// and near the line (1 x 8, S = 3904 64 : 67, 6 x 1, 2009 38 : 40) the split stays.  Below 8 tiles one walk is as quick (six of
+// them, 192 workgroups: 12.8, 13.2).  Above 256 workgroups only causal launches whose early walks are short: a CU's second
+// workgroup then starts early (up to 440; from 448 the pipelined kernel has its slots filled).  Measured, us, split /
+// pipelined -> two groups: 2 x 8 heads, S = 1715 causal 47 / 50 -> 36, 4 x 4, 3136 85 / 90 -> 58, 1 x 16, 2304 60 -> 47, 1 x 32,
+// 1176 48 / 40 -> 28, 1 x 12, 3858 109 / 99 -> 73, 2 x 8, 1998 not causal 65 / 62 -> 45, 8 x 5, 538 26 / 21 -> 16; left where it
+// was: 1 x 10, 744 of 3527 keys 47 (64), 1 x 4, 3448 49 (62), 6 x 4, 1527 of 7299 173 (219), 5 x 14, 555 of 615 26 (28).
+// MI_FMHA_SPLIT set leaves the choice to it.
+bool pick_inside(int64_t wgs, int64_t rows, int D, int Sq, int Skv, bool causal, int input_pos, float scale2, int parts) {
+    static const bool forced = getenv("MI_FMHA_SPLIT") != nullptr;
+    if (forced || D != 128 || Sq <= 64 || wgs > 440 || !(scale2 > 0.f)) return false;
+    int64_t keys = Skv, first = Skv;   // walked by the last / by the first workgroup of a head
+    if (causal) {
+        keys = (int64_t)input_pos + Sq < Skv ? input_pos + Sq : Skv;
+        first = (int64_t)input_pos + kQB < keys ? input_pos + kQB : keys;
+    }
+    const int64_t tiles = (keys + kKV - 1) / kKV;
+    if (wgs > 256) return tiles >= 16 && 5 * first <= keys;
+    if (tiles < 8 || !parts) return tiles >= 8;
+    const double all = (double)wgs * (keys + first) / (2 * kKV), share = tiles / (double)parts;   // tiles of all walks, of a part
+    const double t_two = 6.5 + 1.03 * tiles, t_split = 5.0 + parts * (double)rows * 2.64e-4 + 1.9 * fmax(share, all / 512.0);
+    return t_two < (tiles <= 40 ? 0.95 : 0.9) * t_split;
+}
+
 bool vec16(const mi_tile_array* a) {
     return aligned(a->ptr, 16) && a->strides[1] % 8 == 0 && a->strides[2] % 8 == 0 && a->strides[3] % 8 == 0;
 }
@@ -839,7 +952,9 @@ void launch(dim3 grid, hipStream_t s, bool causal, const mi_tile_array* Q, const
         const char* env_kv = getenv("MI_FMHA_KV_STREAM");
         const int64_t kv_bytes = 2 * (int64_t)(grid.y / group) * Skv * D * 2;
         const int kv_stream = nqb == 1 && (env_kv ? atoi(env_kv) != 0 : kv_bytes > (320ll << 20)) ? 1 : 0;
-        if (const int parts = pick_parts((int64_t)nqb * nbh, rows, D, Sq, Skv, causal, input_pos)) {
+        const int parts = pick_parts((int64_t)nqb * nbh, rows, D, Sq, Skv, causal, input_pos);
+        const bool inside = pick_inside((int64_t)nqb * nbh, rows, D, Sq, Skv, causal, input_pos, scale2, parts);
+        if (parts && !inside) {
             ScratchLease lease;   // ends behind the combine launch
             if (float* scratch = (float*)lease.acquire(g_part, HIP_SYMBOL(fmha_part_scratch), s)) {
                 dim3 gs((unsigned)(nqb * nbh * parts));
@@ -886,6 +1001,21 @@ void launch(dim3 grid, hipStream_t s, bool causal, const mi_tile_array* Q, const
                                      : (D == 64 ? "fmha_dma_q128_kv64_d64_w64q_splitkv" : "fmha_dma_q128_kv64_d128_w32q_splitkv"));
                 return;
             }
+        }
+        if (inside) {
+            const dim3 b2(128 * 2 / JT * 2);
+            if constexpr (D == 128) {
+                if (causal)
+                    hipLaunchKernelGGL((fmha_fwd_dma_kernel<E, D, JT, true, false, 2>), g1, b2, 0, s, (const unsigned short*)Q->ptr, qs,
+                                       (const unsigned short*)K->ptr, ks, (const unsigned short*)V->ptr, vs,
+                                       (unsigned short*)O->ptr, os, Sq, Skv, Hb, group, scale2, input_pos, nqb, nbh, pack, kv_stream);
+                else
+                    hipLaunchKernelGGL((fmha_fwd_dma_kernel<E, D, JT, false, false, 2>), g1, b2, 0, s, (const unsigned short*)Q->ptr, qs,
+                                       (const unsigned short*)K->ptr, ks, (const unsigned short*)V->ptr, vs,
+                                       (unsigned short*)O->ptr, os, Sq, Skv, Hb, group, scale2, input_pos, nqb, nbh, pack, kv_stream);
+            }
+            set_variant("fmha_dma_q128_kv64_d128_w32q_keys2");
+            return;
         }
         if (causal)
             hipLaunchKernelGGL((fmha_fwd_dma_kernel<E, D, JT, true>), g1, blk, 0, s, (const unsigned short*)Q->ptr, qs,
@@ -964,8 +1094,12 @@ extern "C" int mi_fmha_kernel(const mi_tile_array* Q, const mi_tile_array* K, co
         if (!no_pipe && fmha::pipe128_applicable(pr)) {
             // (pipe: the kernel for heads of 128 whenever it can run; read at every call)
             const char* e = getenv("MI_FMHA_KERNEL");
-            if ((e && strcmp(e, "pipe") == 0) ||
-                fmha::pipe128_pays(pr, pick_parts(cld(Sq, (int64_t)kQB) * B * H, B * H * Sq, 128, (int)Sq, (int)Skv, causal, input_pos))) {
+            const int64_t wgs = cld(Sq, (int64_t)kQB) * B * H;
+            const int parts = pick_parts(wgs, B * H * Sq, 128, (int)Sq, (int)Skv, causal, input_pos);
+            // (not causal, keys of another sequence: as before the kernel with two groups of waves, 45 us : 31 us there)
+            const bool inside = (causal || Sq == Skv) && K->strides[1] < (1 << 24) && V->strides[1] < (1 << 24) &&
+                                pick_inside(wgs, B * H * Sq, 128, (int)Sq, (int)Skv, causal, input_pos, scale2, parts);
+            if ((e && strcmp(e, "pipe") == 0) || (!inside && fmha::pipe128_pays(pr, parts))) {
                 fmha::pipe128_launch(pr, s);
                 return launch_status();
             }

@@ -281,7 +281,7 @@ struct Magic {
 };
 struct Map {
     Magic span, heads, heads_last, gm, H, group;   // see the launch
-    int nx, nloc;
+    int nx, nfull;   // XCDs told apart; groups of `heads` heads, the rest is the last group
 };
 
 template <typename E, bool CAUSAL>
@@ -298,8 +298,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
     int qb, bh;
     {
         const unsigned x = mp.nx == 8 ? blockIdx.x & 7u : 0u, idx = mp.nx == 8 ? blockIdx.x >> 3 : blockIdx.x;
-        const unsigned cg = mp.span.div(idx), r = idx - cg * mp.span.d, h0 = cg * mp.heads.d;
-        const bool last = h0 + mp.heads.d > (unsigned)mp.nloc;
+        unsigned cg = mp.span.div(idx);
+        if (cg > (unsigned)mp.nfull) cg = mp.nfull;
+        const unsigned r = idx - cg * mp.span.d, h0 = cg * mp.heads.d;
+        const bool last = cg == (unsigned)mp.nfull;
         const unsigned qi = last ? mp.heads_last.div(r) : mp.heads.div(r);
         const unsigned b = h0 + r - qi * (last ? mp.heads_last.d : mp.heads.d), bg = mp.gm.div(b);
         qb = CAUSAL ? nqb - 1 - (int)qi : (int)qi;
@@ -505,10 +507,17 @@ void launch_e(const Problem& p, hipStream_t stream) {
     // its L2 at a time (4 x 32 ungrouped heads, S = 2048: 154 us, 158 with all heads at once, 163 with half as many).
     const int nkv = nbh / p.group;
     const int nx = nkv % 8 == 0 || nbh % 8 == 0 ? 8 : 1, gm = nkv % 8 == 0 ? p.group : 1, nloc = nbh / nx;
-    int chunk = (64 + nqb - 1) / nqb;
+    // The last group of a causal launch takes up to two chunks, so that the walks that start last are short ones (us, all
+    // chunks alike -> so: 4 x 12 heads, 2054 87 -> 74, 4 x 6, 4944 210 -> 181, 8 x 8, 1716 76 -> 67, 8 x 16, 673 40 -> 34; heads that
+    // no XCD has to itself, 512 slots: 4 x 7, 3433 149 -> 108, 5 x 6, 3755 164 -> 135).
+    const bool spread = nx == 1 && p.causal && (int64_t)nqb * nbh * (1024 / nqb + 2) < (1ll << 32);   // (the magic divisions)
+    int chunk = ((spread ? 512 : 64) + nqb - 1) / nqb;
     if (chunk > nloc) chunk = nloc;
+    int nfull = (nloc + chunk - 1) / chunk - 1;
+    if (p.causal && nfull > 0) --nfull;
+    const int rest = nloc - nfull * chunk;
     const auto magic = [](int d) { return Magic{(unsigned)d, d <= 1 ? 0u : (unsigned)((1ull << 32) / (unsigned)d) + 1u}; };
-    const Map mp{magic(chunk * nqb), magic(chunk), magic(nloc % chunk ? nloc % chunk : chunk), magic(gm), magic(p.H), magic(p.group), nx, nloc};
+    const Map mp{magic(chunk * nqb), magic(chunk), magic(rest), magic(gm), magic(p.H), magic(p.group), nx, nfull};
     if (p.causal)
         hipLaunchKernelGGL((fmha_pipe128_kernel<E, true>), dim3((unsigned)(nqb * nbh)), dim3(64 * NW), 0, stream,
                            (const unsigned short*)Q->ptr, qs, (const unsigned short*)K->ptr, ks, (const unsigned short*)V->ptr, vs,
@@ -554,9 +563,11 @@ bool pipe128_pays(const Problem& p, int parts) {
     // (two per CU) and the walks be long enough to pay for the ramp: 2 x 32 heads, S = 2000 causal 82 : 115 us, 8 x 32 heads,
     // S = 506 causal 38 : 45, 1 x 32 heads, S = 2048 causal 64 : 70; but 640 workgroups of 19 halves, not causal, 54 : 45, 4 x
     // 32 heads, S = 1171 causal (1280 workgroups) 90 : 81, and 8 x 16 heads, S = 173 12.1 : 11.3.  On 700 further shapes,
-    // 220 of them taken, the times were 0.49 to 1.11 of the other kernel's, 0.76 in the mean.
+    // 220 of them taken, the times were 0.49 to 1.11 of the other kernel's, 0.76 in the mean.  Since the other kernel starts
+    // its long causal walks first, launches of three rounds and more are worth it from 48 halves only (4 x 64 heads, S = 653
+    // causal 62 : 57, 6 x 64, 712 102 : 93, 7 x 32, 1079 106 : 99; 5 x 16, 3766 347 : 362, 6 x 40, 1955 323 : 358).
     const int64_t rounds = (wgs + 511) / 512;
-    return wgs >= 448 && wgs * 100 >= rounds * 512 * (rounds <= 2 ? 78 : 90) && halves >= (wgs < 800 ? 32 : 8) && (p.causal || rounds <= 2);
+    return wgs >= 448 && wgs * 100 >= rounds * 512 * (rounds <= 2 ? 78 : 90) && halves >= (wgs < 800 ? 32 : rounds <= 2 ? 8 : 48) && (p.causal || rounds <= 2);
 }
 
 void pipe128_launch(const Problem& p, hipStream_t stream) {

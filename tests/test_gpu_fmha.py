@@ -370,6 +370,46 @@ def test_fmha_heads_of_128_both_sides_of_the_rule(ct, monkeypatch, batch, heads,
     assert float((a - b).norm() / b.norm()) < 2.0 ** -8
 
 
+@pytest.mark.parametrize("batch,heads,qg,sq,skv,causal,pos,T", [
+    (1, 24, 4, 546, 546, True, 0, torch.bfloat16), (1, 32, 8, 512, 512, True, 0, torch.float16),      # nine and eight tiles of keys
+    (5, 7, 7, 577, 577, True, 0, torch.float16), (4, 8, 2, 729, 729, False, 0, torch.bfloat16),       # one key, 25 keys in the last one
+    (6, 6, 1, 640, 640, False, 0, torch.float16), (6, 6, 3, 523, 772, True, 249, torch.bfloat16),     # a decode offset
+    (6, 6, 2, 523, 772, True, 0, torch.float16), (1, 24, 1, 700, 520, True, 0, torch.bfloat16),       # keys past every diagonal; fewer keys than queries
+    (1, 36, 4, 1030, 1030, True, 0, torch.float16), (1, 32, 4, 1100, 1100, True, 0, torch.bfloat16),  # more workgroups than CUs
+])
+@pytest.mark.parametrize("slope", [0.0, 6.0, -6.0])
+def test_fmha_two_groups_of_waves_share_the_keys(ct, orc, batch, heads, qg, sq, skv, causal, pos, T, slope):
+    """Heads of 128 where a workgroup's two groups of waves take every other key tile.  `slope`: scores that rise or fall
+    along the keys, so that the weights' reference follows the tile's maximum up, and down to its limit."""
+    data = fmha.prepare(batch=batch, heads=heads, seq_q=sq, seq_kv=skv, d_k=128, d_v=128, query_group_size=qg, causal=causal, T=T)
+    if slope:
+        data.Q = (data.Q.float() * 0.25 + 1.0).to(T)
+        at = torch.arange(skv, device="cuda") / skv
+        data.K = ((data.K.float() * 0.25 + 1.0) * (1.0 + abs(slope) * (at if slope > 0 else 1 - at))[None, None, :, None]).to(T)
+    big = torch.full((batch, heads, sq + 9, 128), 777.0, dtype=T, device="cuda")
+    out = big[:, :, :sq, :]
+    out.fill_(float("nan"))
+    fmha.cutile_fmha(data.Q, data.K, data.V, query_group_size=qg, causal=causal, input_pos=pos, out=out)
+    assert ct.last_variant() == "fmha_dma_q128_kv64_d128_w32q_keys2"
+    assert bool((big[:, :, sq:, :] == 777.0).all())
+    ref = orc.fmha_general(*(orc.to_julia(t) for t in (data.Q, data.K, data.V)), causal=causal, input_pos=pos)
+    check(orc, out, ref, 2e-2 if T == torch.float16 else 3e-2)
+
+
+@pytest.mark.parametrize("batch,heads,qg,sq,kernel", [
+    (66, 8, 1, 130, "pipe"), (53, 10, 5, 130, "pipe"),            # one full chunk of heads and a longer last one; no XCD with heads of its own
+    (9, 16, 2, 130, "dma"), (9, 9, 3, 200, "dma"), (40, 8, 1, 257, "dma"),
+])
+def test_fmha_heads_of_128_every_head_walked_once_longest_first(ct, orc, monkeypatch, batch, heads, qg, sq, kernel):
+    """The numbering of causal launches that starts the long walks of all heads first."""
+    monkeypatch.setenv("MI_FMHA_KERNEL", kernel)
+    data = fmha.prepare(batch=batch, heads=heads, seq_q=sq, seq_kv=sq, d_k=128, d_v=128, query_group_size=qg, causal=True, T=torch.float16)
+    out = torch.full_like(data.Q, float("nan"))
+    fmha.cutile_fmha(data.Q, data.K, data.V, query_group_size=qg, causal=True, out=out)
+    ref = orc.fmha_general(*(orc.to_julia(t) for t in (data.Q, data.K, data.V)), causal=True, input_pos=0)
+    check(orc, out, ref, 2e-2)
+
+
 def test_fmha_heads_of_128_rows_at_the_limit_of_their_offsets(ct, orc, monkeypatch):
     """Keys and values so far apart that the last byte offset of a head lies just below 2^32, and just above what the
     pipelined kernel addresses (rows * stride of 2^31 elements), which the general kernel takes."""
