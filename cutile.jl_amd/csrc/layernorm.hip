@@ -16,6 +16,7 @@
 // owns the slot (S == 1), device-scope float atomics otherwise.  No spin-lock: workgroups of
 // one grid have no forward-progress guarantee relative to each other on this hardware.
 #include "common.h"
+#include <algorithm>
 #include <type_traits>
 #include <math.h>
 #include <stdlib.h>
@@ -419,11 +420,13 @@ __global__ __launch_bounds__(BLOCK) void ln_bwd_kernel(float* __restrict__ DX, i
     }
 }
 
-// Backward with RG row groups of 256 lanes per workgroup (rows of up to 4096 elements, 16-byte
-// aligned): the groups walk different rows of the same partial slot and add their dW/dB
-// partials in LDS before the flush, which divides the number of memory-side float atomics --
-// the scarce resource of this kernel -- by RG at the same number of rows in flight.
+// Backward with RG row groups of BLOCK lanes per workgroup (rows of up to 8192 elements, 16-byte aligned): the groups walk
+// different rows of the same partial slot and add their dW / dB partials in LDS before the flush, which divides the number
+// of memory-side float atomics -- the scarce resource of this kernel -- by RG at the same number of rows in flight.
 // Workgroup (g, s): group h handles rows m = g + G*(RG*s + h), stepping by RG*G*S.
+// Large inputs are bound by memory, small ones by the chain load, reduction, flush: the groups leave their partials in LDS
+// side by side and one barrier later every lane adds up its columns' (one group after the other, dW and dB in two
+// passes, took 2 RG + 2 barriers: 1024 x 256, 64 slots 5.0 -> 3.8 us, 512 x 4096 15.3 -> 12.9).
 template <int BLOCK, int VPT, bool STREAM, int RG>
 __global__ __launch_bounds__(BLOCK * RG) void ln_bwd_rg_kernel(float* __restrict__ DX, int64_t lddx,
                                                          const float* __restrict__ DY, int64_t lddy,
@@ -437,7 +440,7 @@ __global__ __launch_bounds__(BLOCK * RG) void ln_bwd_rg_kernel(float* __restrict
     constexpr int NW = BLOCK / 64;
     static_assert(NW == 1 || NW == 4 || NW == 8, "the cross-wave sums are written out for 4 and 8 waves");
     __shared__ float red[RG][2 * NW];
-    __shared__ float stage[BLOCK * VPT * 4];
+    __shared__ __attribute__((aligned(16))) float stage[RG][2][BLOCK * VPT * 4];
     const int g = blockIdx.x % G, s = blockIdx.x / G;
     const int h = threadIdx.x / BLOCK, lt = threadIdx.x % BLOCK, lane = lt & 63, wave = lt >> 6;
     auto vec = [&](int v) { return (lt + v * BLOCK) * 4; };
@@ -539,32 +542,35 @@ __global__ __launch_bounds__(BLOCK * RG) void ln_bwd_rg_kernel(float* __restrict
         trip(Set0{}, it);
         if (it + 1 < trips) trip(Set1{}, it + 1);
     }
-    // the groups add their partials in LDS, one after the other; then everybody flushes with
-    // coalesced atomics
+    // every group leaves its partials in LDS; then everybody adds the groups' and flushes with coalesced atomics
+#pragma unroll
+    for (int v = 0; v < VPT; ++v) {
+        f32x4 t, u;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            t[q] = dw[v][q];
+            u[q] = db[v][q];
+        }
+        *reinterpret_cast<f32x4*>(&stage[h][0][vec(v)]) = t;
+        *reinterpret_cast<f32x4*>(&stage[h][1][vec(v)]) = u;
+    }
+    __syncthreads();
     float* dwp = DW + (int64_t)g * lddw;
     float* dbp = DB + (int64_t)g * lddb;
+    for (int c = threadIdx.x; c < N; c += BLOCK * RG) {
+        float t = stage[0][0][c], u = stage[0][1][c];
 #pragma unroll
-    for (int pass = 0; pass < 2; ++pass) {
-#pragma unroll
-        for (int turn = 0; turn < RG; ++turn) {
-            if (h == turn) {
-#pragma unroll
-                for (int v = 0; v < VPT; ++v)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const float val = pass == 0 ? dw[v][q] : db[v][q];
-                        if (turn == 0) stage[vec(v) + q] = val;
-                        else stage[vec(v) + q] += val;
-                    }
-            }
-            __syncthreads();
+        for (int k = 1; k < RG; ++k) {
+            t += stage[k][0][c];
+            u += stage[k][1][c];
         }
-        float* dst = pass == 0 ? dwp : dbp;
-        for (int c = threadIdx.x; c < N; c += BLOCK * RG) {
-            if (S == 1) dst[c] += stage[c];
-            else unsafeAtomicAdd(dst + c, stage[c]);
+        if (S == 1) {
+            dwp[c] += t;
+            dbp[c] += u;
+        } else {
+            unsafeAtomicAdd(dwp + c, t);
+            unsafeAtomicAdd(dbp + c, u);
         }
-        __syncthreads();
     }
 }
 
@@ -1167,18 +1173,22 @@ extern "C" int mi_layer_norm_bwd_dx_partial_dwdb(
     const bool stream_in = stream_hint(3 * M * N * (int64_t)sizeof(float));
     static const bool one_group = [] { const char* e = getenv("MI_LN_BWD_RG"); return e && e[0] == '1'; }();
     if (al && N % 4 == 0 && vecs <= 2048 && !one_group) {
-        // Row groups with two rows of look-ahead.  Up to 4096 elements a group is 256 lanes and two
-        // groups share a workgroup (same rows in flight, half the atomics; four groups measured no
-        // better); up to 8192 elements one group of 512 lanes.
-        // Up to 512 elements a group is a single wave (no barriers in the walk) and eight groups
-        // share a workgroup; there the chip wants four times as many groups in flight, since a
-        // group's rows are that much shorter.
-        const int rg = vecs <= 128 ? 8 : vecs <= 1024 ? 2 : 1;
-        if ((vecs <= 128 || vecs > 1024) && !getenv("MI_LN_BWD_SPLITS")) {
-            // (and a 512-lane group fills a CU by itself: one workgroup per CU, half the flushes)
-            S = cld((int64_t)(vecs <= 128 ? 2048 : 256), (int64_t)G);
-            if (S > cld(rows_per_slot, (int64_t)4)) S = cld(rows_per_slot, (int64_t)4);
-            if (S < 1) S = 1;
+        // Row groups with two rows of look-ahead.  Up to 4096 elements a group is 256 lanes and two groups share a workgroup
+        // (same rows in flight, half the atomics; four groups measured no better); up to 8192 elements one group of 512 lanes,
+        // which fills a CU by itself: one workgroup per CU, half the flushes.
+        // Up to 1024 elements a group is a single wave (no barriers in the walk) and eight groups share a workgroup, at most
+        // one per CU; with few rows each wave has one (64 slots, us, 256 lanes -> a wave: 1024 x 1024 6.8 -> 5.2, 4096 x
+        // 1024 12.6 -> 11.0, 4096 x 700 11.8 -> 9.7; at least four rows a wave -> one: 2000 x 512 6.4 -> 4.7).  Streamed
+        // inputs of more than 512 elements keep 256 lanes (where the two meet, 16384 x 1024, 38.2 and 39.3).
+        const bool one_wave = vecs <= (stream_in ? 128 : 256);
+        const int rg = one_wave ? 8 : vecs <= 1024 ? 2 : 1;
+        if (!getenv("MI_LN_BWD_SPLITS")) {
+            const int64_t per_cu = cld((int64_t)256, (int64_t)G);
+            if (one_wave) S = 8 * std::min(per_cu, cld(rows_per_slot, (int64_t)8));
+            else if (vecs > 1024) S = std::max((int64_t)1, std::min(per_cu, cld(rows_per_slot, (int64_t)4)));
+            // (few rows: two per group rather than four where that leaves less than a group per CU: 512 x 2048 8.4 -> 6.5,
+            // 400 x 4096 12.4 -> 9.5; 256 x 2048 5.4 either way)
+            else if (S < per_cu) S = std::min(per_cu, cld(rows_per_slot, (int64_t)2));
         }
         const int S2 = (int)cld(S, (int64_t)rg);
         dim3 grid2((unsigned)(G * S2));
@@ -1194,6 +1204,7 @@ extern "C" int mi_layer_norm_bwd_dx_partial_dwdb(
     } while (0)
         if (vecs <= 64) { RGS(64, 1, 8); set_variant("ln_bwd_regs_b512_v1_rg8"); }
         else if (vecs <= 128) { RGS(64, 2, 8); set_variant("ln_bwd_regs_b512_v2_rg8"); }
+        else if (one_wave) { RGS(64, 4, 8); set_variant("ln_bwd_regs_b512_v4_rg8"); }
         else if (vecs <= 256) { RGS(256, 1, 2); set_variant("ln_bwd_regs_b512_v1_rg2"); }
         else if (vecs <= 512) { RGS(256, 2, 2); set_variant("ln_bwd_regs_b512_v2_rg2"); }
         else if (vecs <= 1024) { RGS(256, 4, 2); set_variant("ln_bwd_regs_b512_v4_rg2"); }

@@ -444,6 +444,34 @@ def test_layernorm_bwd_wide_rows(ct, orc, M, N, G):
     close_f32(orc.to_julia(d.FINAL_DB), DB)
 
 
+@pytest.mark.parametrize("M,N,G,variant", [
+    (64, 516, 64, "v4_rg8"), (513, 1024, 64, "v4_rg8"), (1030, 700, 64, "v4_rg8"), (5000, 1000, 64, "v4_rg8"), (9, 1024, 300, "v4_rg8"),  # one row per slot, and one more than eight waves take; more slots than rows
+    (77, 1024, 1, "v4_rg8"), (2049, 512, 64, "v2_rg8"), (70, 260, 8, "v2_rg8"), (640, 256, 64, "v1_rg8"), (3, 4, 2, "v1_rg8"),
+    (19200, 1024, 64, "v1_rg2"),                                                                          # inputs that are streamed
+    (257, 1028, 64, "v2_rg2"), (449, 2048, 64, "v2_rg2"), (512, 4096, 64, "v4_rg2"), (513, 3000, 64, "v4_rg2"), (1, 2052, 1, "v4_rg2"), (300, 4100, 64, "v4_rg1"),
+])
+def test_layernorm_bwd_row_groups(ct, orc, M, N, G, variant):
+    """Row groups of one wave (up to 1024 elements) and of 256 lanes, at the edges of both, with fewer rows than groups
+    and one row more than they take; partial slots in wider buffers, added to what they hold."""
+    d = layernorm.prepare(M=M, N=N, GROUP_SIZE_M=G)
+    ct.layer_norm_fwd(d.X, d.W, d.B, d.Y, d.Mean, d.Rstd, d.eps, 1024)
+    wide = torch.zeros(2, G, N + 12, device="cuda")
+    wide[..., N:] = 7.0
+    wide[:, 0, :N] = 0.5
+    DWp, DBp = wide[0, :, :N], wide[1, :, :N]
+    d.DX.fill_(float("nan"))
+    ct.layer_norm_bwd_dx_partial_dwdb(d.DX, d.DY, DWp, DBp, d.X, d.W, d.Mean, d.Rstd, d.Locks, G, 1024)
+    assert ct.last_variant() == "ln_bwd_regs_b512_" + variant
+    assert bool((wide[..., N:] == 7.0).all())
+    wide[:, 0, :N] -= 0.5
+    ct.layer_norm_bwd_dwdb(DWp, DBp, d.FINAL_DW, d.FINAL_DB, 32, 1024)
+    X, W, DY = (orc.to_julia(t) for t in (d.X, d.W, d.DY))
+    DX, DW, DB = orc.layer_norm_bwd(X, W, DY, d.eps)
+    close_f32(orc.to_julia(d.DX), DX)
+    close_f32(orc.to_julia(d.FINAL_DW), DW)
+    close_f32(orc.to_julia(d.FINAL_DB), DB)
+
+
 @pytest.mark.parametrize("M,N,G,variant", [(130, 32768, 64, "ln_bwd_two_pass_b512_v16"), (37, 16388, 8, "ln_bwd_two_pass_b512_v16"),
                                            (300, 20000, 256, "ln_bwd_two_pass_b512_v16"), (5, 24580, 1, "ln_bwd_two_pass_b512_v16"),
                                            (9, 32772, 4, "ln_bwd_long_b256"), (6, 20001, 4, "ln_bwd_long_b256")])
