@@ -476,14 +476,27 @@ __global__ __launch_bounds__(128 * 2 / JT * KG) __attribute__((amdgpu_waves_per_
             sp = L / (nqb * nbh);
             L -= sp * (nqb * nbh);
         }
-        // Causal with equal query tiles: the long walks of all of an XCD's heads start first, so that what starts last is short
-        // (head by head, the last head's longest walk starts when nearly everything else has ended).
-        constexpr bool LONGEST = CAUSAL && !PAIRED && !SPLIT;
-        const int nx = nbh % 8 == 0 ? 8 : 1, idx = L / nx, per = nbh / nx, j = LONGEST ? idx % per : idx / nqb;
-        qb = LONGEST ? idx / per : idx % nqb;
-        const int gm = nx == 8 && pack == 1 && (nbh / group) % 8 == 0 ? group : 1;   // an XCD gets all heads that share a K / V head
-        bh = (L % nx + nx * (j / gm)) * gm + j % gm;
-        if (CAUSAL && !PAIRED) qb = nqb - 1 - qb;
+        if constexpr (CAUSAL && !PAIRED && !SPLIT) {
+            // Equal query tiles: the long walks of all of an XCD's heads start first, so that what starts last is short (head
+            // by head, the last head's longest walk starts when nearly everything else has ended).
+            const bool xcd = nbh % 8 == 0;
+            const int idx = xcd ? L >> 3 : L, per = xcd ? nbh >> 3 : nbh, j = idx % per;
+            qb = nqb - 1 - idx / per;
+            if (!xcd) bh = j;
+            else if (group > 1 && pack == 1 && (nbh / group) % 8 == 0)   // an XCD gets all heads that share a K / V head
+                bh = ((L & 7) + 8 * (j / group)) * group + j % group;
+            else bh = (L & 7) + 8 * j;
+        } else {
+            if (nbh % 8 == 0) {
+                const int idx = L >> 3;
+                bh = (L & 7) + 8 * (idx / nqb);
+                qb = idx % nqb;
+            } else {
+                bh = L / nqb;
+                qb = L % nqb;
+            }
+            if (CAUSAL && !PAIRED) qb = nqb - 1 - qb;
+        }
     }
     // (pack > 1: bh counts (batch, K / V head) pairs, H is their number per batch, and a row carries its head)
     const int batch = bh / H, hrem = bh % H;
