@@ -25,7 +25,8 @@
 // Causal balance: D = 64, a wave takes the 32-query tiles u and NT-1-u, so every wave walks the same number of KV tiles; D =
 // 128, the long walks of all of an XCD's heads start first (head by head, the last head's longest walk started when most of
 // the chip was idle: 7 x 4 heads, S = 3433 123 us, now 106, 8 x 16, 619 36 -> 26, 5 x 4, 4000 193 -> 113, 4 x 16, 2213 124 -> 107).
-// All query tiles of a (batch, head) run on one XCD, with those of the heads that share its K / V where their number allows it.
+// All query tiles of a (batch, head) run on one XCD, there with those of the heads that share its K / V where their number
+// allows it.
 // Causal tile skipping: the KV loop stops at the workgroup's last query, and a wave skips
 // tiles that lie wholly above its own last query.  Masking and the ragged KV tail use -Inf
 // as in the reference (fmha.jl:92-103).
