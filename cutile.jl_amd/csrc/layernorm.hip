@@ -1177,18 +1177,20 @@ extern "C" int mi_layer_norm_bwd_dx_partial_dwdb(
         // (same rows in flight, half the atomics; four groups measured no better); up to 8192 elements one group of 512 lanes,
         // which fills a CU by itself: one workgroup per CU, half the flushes.
         // Up to 1024 elements a group is a single wave (no barriers in the walk) and eight groups share a workgroup, at most
-        // one per CU; with few rows each wave has one (64 slots, us, 256 lanes -> a wave: 1024 x 1024 6.8 -> 5.2, 4096 x
-        // 1024 12.6 -> 11.0, 4096 x 700 11.8 -> 9.7; at least four rows a wave -> one: 2000 x 512 6.4 -> 4.7).  Streamed
-        // inputs of more than 512 elements keep 256 lanes (where the two meet, 16384 x 1024, 38.2 and 39.3).
+        // one per CU, with at least four rows a wave up to 512 elements (64 slots, us, 256 lanes -> a wave: 1024 x 1024 6.8 -> 5.2,
+        // 4096 x 1024 12.6 -> 11.0, 4096 x 700 11.8 -> 9.7).  Streamed inputs of more than 512 elements keep 256 lanes (where
+        // the two meet, 16384 x 1024, 38.2 and 39.3).
+        // A slot that one workgroup owns gets plain adds, and the same bits on every run; two add to a zero slot in either
+        // order with the same result; from three on the order of arrival decides the last bits.  One row a wave is
+        // quicker on many slots (64 slots, 2000 x 512 6.1 -> 5.6 us), but puts more workgroups on slots that have one or two now,
+        // and costs more than it gives on few slots (1 slot, 2000 x 400 7.1 -> 9.6); two rows a group above 1024 elements likewise.
         const bool one_wave = vecs <= (stream_in ? 128 : 256);
         const int rg = one_wave ? 8 : vecs <= 1024 ? 2 : 1;
         if (!getenv("MI_LN_BWD_SPLITS")) {
             const int64_t per_cu = cld((int64_t)256, (int64_t)G);
-            if (one_wave) S = 8 * std::min(per_cu, cld(rows_per_slot, (int64_t)8));
+            if (vecs <= 128) S = std::min(cld((int64_t)2048, (int64_t)G), cld(rows_per_slot, (int64_t)4));
+            else if (one_wave) S = 8 * std::min(per_cu, cld(rows_per_slot, (int64_t)8));
             else if (vecs > 1024) S = std::max((int64_t)1, std::min(per_cu, cld(rows_per_slot, (int64_t)4)));
-            // (few rows: two per group rather than four where that leaves less than a group per CU: 512 x 2048 8.4 -> 6.5,
-            // 400 x 4096 12.4 -> 9.5; 256 x 2048 5.4 either way)
-            else if (S < per_cu) S = std::min(per_cu, cld(rows_per_slot, (int64_t)2));
         }
         const int S2 = (int)cld(S, (int64_t)rg);
         dim3 grid2((unsigned)(G * S2));

@@ -472,6 +472,26 @@ def test_layernorm_bwd_row_groups(ct, orc, M, N, G, variant):
     close_f32(orc.to_julia(d.FINAL_DB), DB)
 
 
+@pytest.mark.parametrize("M,N,G,held", [
+    (2048, 512, 64, 0.0), (1100, 256, 64, 0.0), (640, 512, 64, 0.5), (1999, 64, 64, 0.5),   # one workgroup per slot: up to 32 rows of 512 elements,
+    (512, 2048, 64, 0.5), (300, 4096, 64, 0.5), (64, 1028, 8, 0.5), (512, 1024, 64, 0.5),   # up to 8 rows of more
+    (4096, 512, 64, 0.0), (512, 2048, 32, 0.0), (1024, 1024, 64, 0.0),                      # two that add to a slot of zeros
+])
+def test_layernorm_bwd_same_bits_on_every_run(ct, M, N, G, held):
+    """Up to the sizes where one workgroup adds to a partial slot the sums do not depend on timing, whatever the slot holds; with
+    two of them it has to hold zeros."""
+    d = layernorm.prepare(M=M, N=N, GROUP_SIZE_M=G)
+    ct.layer_norm_fwd(d.X, d.W, d.B, d.Y, d.Mean, d.Rstd, d.eps, 1024)
+    rng = torch.Generator(device="cuda").manual_seed(1)
+    start = held * torch.randn(d.partials.shape, device="cuda", generator=rng)
+    runs = []
+    for _ in range(24):
+        d.partials.copy_(start)
+        ct.layer_norm_bwd_dx_partial_dwdb(d.DX, d.DY, d.DW_partial, d.DB_partial, d.X, d.W, d.Mean, d.Rstd, d.Locks, G, 1024)
+        runs.append(d.partials.clone())
+    assert all(torch.equal(r, runs[0]) for r in runs[1:])
+
+
 @pytest.mark.parametrize("M,N,G,variant", [(130, 32768, 64, "ln_bwd_two_pass_b512_v16"), (37, 16388, 8, "ln_bwd_two_pass_b512_v16"),
                                            (300, 20000, 256, "ln_bwd_two_pass_b512_v16"), (5, 24580, 1, "ln_bwd_two_pass_b512_v16"),
                                            (9, 32772, 4, "ln_bwd_long_b256"), (6, 20001, 4, "ln_bwd_long_b256")])
