@@ -31,6 +31,7 @@
 // 40 instructions less per step, 4 MFMAs more) were tried and did not help.  Causal pays for its diagonals and for the
 // last, unequal workgroups.
 #include "fmha_common.h"
+#include "fmha_pipe128_map.h"
 
 #include <utility>
 
@@ -274,16 +275,6 @@ __device__ __forceinline__ void step(const unsigned short* Ks, const unsigned sh
     }
 }
 
-// Division by a launch constant: a multiply-high with floor(2^32 / d) + 1, exact while x * d < 2^32 (the host sees to it).
-struct Magic {
-    unsigned d, m;
-    __device__ __forceinline__ unsigned div(unsigned x) const { return m ? __umulhi(x, m) : x; }   // (m = 0: d = 1)
-};
-struct Map {
-    Magic span, heads, heads_last, gm, H, group;   // see the launch
-    int nx, nfull;   // XCDs told apart; groups of `heads` heads, the rest is the last group
-};
-
 template <typename E, bool CAUSAL>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1))) void fmha_pipe128_kernel(
     const unsigned short* __restrict__ Q, Strides qs, const unsigned short* __restrict__ K, Strides ks,
@@ -294,19 +285,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
 
     const int tid = threadIdx.x, lane = tid & 63, hb = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // Workgroup id -> (query block, head): see the launch.
+    // Workgroup id -> (query block, head): fmha_pipe128_map.h.
     int qb, bh;
-    {
-        const unsigned x = mp.nx == 8 ? blockIdx.x & 7u : 0u, idx = mp.nx == 8 ? blockIdx.x >> 3 : blockIdx.x;
-        unsigned cg = mp.span.div(idx);
-        if (cg > (unsigned)mp.nfull) cg = mp.nfull;
-        const unsigned r = idx - cg * mp.span.d, h0 = cg * mp.heads.d;
-        const bool last = cg == (unsigned)mp.nfull;
-        const unsigned qi = last ? mp.heads_last.div(r) : mp.heads.div(r);
-        const unsigned b = h0 + r - qi * (last ? mp.heads_last.d : mp.heads.d), bg = mp.gm.div(b);
-        qb = CAUSAL ? nqb - 1 - (int)qi : (int)qi;
-        bh = (int)((x + mp.nx * bg) * mp.gm.d + b - bg * mp.gm.d);
-    }
+    mp.at(blockIdx.x, nqb, CAUSAL, &qb, &bh);
     const int batch = (int)mp.H.div((unsigned)bh), head = bh - batch * H, kvh = (int)mp.group.div((unsigned)head);
     Q += (int64_t)head * qs.s2 + (int64_t)batch * qs.s3;
     O += (int64_t)head * os.s2 + (int64_t)batch * os.s3;
@@ -501,23 +482,7 @@ void launch_e(const Problem& p, hipStream_t stream) {
         vs{V->strides[1], V->strides[2], V->strides[3]}, os{O->strides[1], O->strides[2], O->strides[3]};
     const int Sq = (int)Q->sizes[1], Skv = (int)K->sizes[1];
     const int nqb = (Sq + 64 * NW - 1) / (64 * NW), nbh = (int)(Q->sizes[2] * Q->sizes[3]);
-    // Workgroup ids congruent mod 8 share an XCD: an XCD gets whole key / value heads (all query heads of a group with
-    // theirs) where their number allows it.  Within an XCD the ids walk `chunk` heads at a time, the query blocks with the
-    // longest key ranges first: as many heads as fill the XCD's 64 slots (two workgroups per CU), so that few K / V share
-    // its L2 at a time (4 x 32 ungrouped heads, S = 2048: 154 us, 158 with all heads at once, 163 with half as many).
-    const int nkv = nbh / p.group;
-    const int nx = nkv % 8 == 0 || nbh % 8 == 0 ? 8 : 1, gm = nkv % 8 == 0 ? p.group : 1, nloc = nbh / nx;
-    // The last group of a causal launch takes up to two chunks, so that the walks that start last are short ones (us, all
-    // chunks alike -> so: 4 x 12 heads, 2054 87 -> 74, 4 x 6, 4944 210 -> 181, 8 x 8, 1716 76 -> 67, 8 x 16, 673 40 -> 34; heads that
-    // no XCD has to itself, 512 slots: 4 x 7, 3433 149 -> 108, 5 x 6, 3755 164 -> 135).
-    const bool spread = nx == 1 && p.causal && (int64_t)nqb * nbh * (1024 / nqb + 2) < (1ll << 32);   // (the magic divisions)
-    int chunk = ((spread ? 512 : 64) + nqb - 1) / nqb;
-    if (chunk > nloc) chunk = nloc;
-    int nfull = (nloc + chunk - 1) / chunk - 1;
-    if (p.causal && nfull > 0) --nfull;
-    const int rest = nloc - nfull * chunk;
-    const auto magic = [](int d) { return Magic{(unsigned)d, d <= 1 ? 0u : (unsigned)((1ull << 32) / (unsigned)d) + 1u}; };
-    const Map mp{magic(chunk * nqb), magic(chunk), magic(rest), magic(gm), magic(p.H), magic(p.group), nx, nfull};
+    const Map mp = make_map(nqb, nbh, p.H, p.group, p.causal);
     if (p.causal)
         hipLaunchKernelGGL((fmha_pipe128_kernel<E, true>), dim3((unsigned)(nqb * nbh)), dim3(64 * NW), 0, stream,
                            (const unsigned short*)Q->ptr, qs, (const unsigned short*)K->ptr, ks, (const unsigned short*)V->ptr, vs,
@@ -538,9 +503,7 @@ bool pipe128_applicable(const Problem& p) {
     // 32-bit byte offsets within a head's keys
     const int64_t rows = K->sizes[1] + 2 * kHK;
     if (K->strides[1] < 0 || V->strides[1] < 0 || rows * K->strides[1] >= (1ll << 31) || rows * V->strides[1] >= (1ll << 31)) return false;
-    // the multiply-high divisions of the workgroup id are exact below 2^32 (id times divisor)
-    const int64_t nqb = (Q->sizes[1] + 127) / 128, nbh = Q->sizes[2] * Q->sizes[3], wgs = nqb * nbh;
-    if (wgs * (128 + 2 * nqb) >= (1ll << 32) || nbh * (p.H > 128 ? p.H : 128) >= (1ll << 32)) return false;
+    if (!map_exact((Q->sizes[1] + 127) / 128, Q->sizes[2] * Q->sizes[3], p.H)) return false;   // (its numbering's divisions)
     if (K->sizes[1] < kHK) return false;   // (the last half is the last 32 keys)
     return Q->sizes[1] > 64;               // (few queries: a group's heads are stacked in one tile, fmha.hip)
 }
