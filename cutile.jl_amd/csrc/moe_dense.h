@@ -68,9 +68,8 @@ bool dense_applicable(const DenseArgs& a);
 // Launches it and records the variant name.
 void dense_launch(const DenseArgs& a, hipStream_t s);
 // moe_prefill.hip: the kernel whose transfers have waves of their own, for launches that dense_applicable accepts.
-// Weight rows per tile (256 or 128) where it is the one to take, else 0; launches it and records the variant name.
-int prefill_rows(const DenseArgs& a);
-void prefill_launch(const DenseArgs& a, int rows, hipStream_t s);
+// Launches it and records the variant name where it is the one to take, else returns false.
+bool prefill_launch(const DenseArgs& a, hipStream_t s);
 
 }  // namespace moe
 }  // namespace mi

@@ -866,7 +866,7 @@ static int pick_j(const DenseArgs& a) {
 void dense_launch(const DenseArgs& a, hipStream_t s) {
     // (a forced shape of this kernel is this kernel)
     if (!getenv("MI_MOE_DENSE_J") && !getenv("MI_MOE_DENSE_WIDE") && !getenv("MI_MOE_DENSE_STREAM"))
-        if (const int rows = prefill_rows(a)) return prefill_launch(a, rows, s);
+        if (prefill_launch(a, s)) return;
     const int J = pick_j(a);
     const int n_blocks = a.silu ? (int)cld((int64_t)a.N / 2, (int64_t)(32 * J)) : (int)cld((int64_t)a.N, (int64_t)(64 * J));
     const int64_t tiles = (int64_t)a.num_blocks * (a.TILE_M / kRows) * n_blocks;

@@ -10,7 +10,8 @@
 // the first is close to the power limit.  The ring kernel takes 126 + 86.
 //
 //   tile = up to 160 slots x 256 weight rows, a wave all slots x 64 rows (10 MFMA 32x32x16 tiles), or up to 192 slots x 128
-//   rows, a wave every second 32-slot sub-tile x 64 rows; three stages of 52 / 40 KB.
+//   rows, a wave every second 32-slot sub-tile x 64 rows; three stages of 52 / 40 KB.  A launch picks one of the two from the table
+//   of runs below.
 //
 // Slots are dealt in 32-slot sub-tiles and not in blocks of 128: an expert's run of blocks is cut evenly into as few tiles as
 // hold its sub-tiles with tokens (a table of runs that every workgroup makes at its start, 2.4 us).  At 256 +- 16 slots per
@@ -72,108 +73,32 @@ struct Tile {
     int slot0, live, strip, expert;   // first slot, 32-slot sub-tiles, strip of weight rows, expert (0-based)
 };
 
+constexpr int max_live(int wc) { return wc == 4 ? 5 : 6; }          // sub-tiles of 32 slots per tile at most
+constexpr int stage_of(int wc) { return (32 * max_live(wc) + 64 * wc) * BK; }   // elements of a stage
+constexpr int kSlotsMax = 32 * max_live(2);
+
+// The runs of blocks of one expert.
+struct Runs {
+    const int *first, *slot, *live;   // (LDS) of every run: its first tile, its first slot, its 32-slot sub-tiles up to its last token | expert << 16
+    int runs, tiles;                  // their number (-1: one tile per 128 slots), and the tiles of all
+};
+
 // WC: groups of 64 weight rows, one or two waves each (WS slot groups).
 template <typename E, int MODE, int WC>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void moe_prefill_kernel(const DenseArgs a, int strips) {
-    constexpr int WS = 4 / WC, kMaxL = WC == 4 ? 5 : 6, kRows = (kMaxL + WS - 1) / WS;   // sub-tiles of 32 slots per tile / per wave at most
+__device__ __forceinline__ void walk_tiles(const DenseArgs& a, int strips, const Runs& table, unsigned short* ring, int (*s_tok)[kSlotsMax], float* s_wt) {
+    constexpr int WS = 4 / WC, kMaxL = max_live(WC), kRows = (kMaxL + WS - 1) / WS;      // sub-tiles of 32 slots per tile / per wave at most
     constexpr int kW = 64 * WC;                                                          // weight rows per tile
     constexpr int kSlots = 32 * kMaxL;
     constexpr int kStageT = kSlots * BK, kStage = kStageT + kW * BK;   // elements of a stage's token part / of a stage
+    static_assert(kStage == stage_of(WC), "the ring holds the stages");
     struct Frags {
         s16x8 t[kRows], w[2];
     };
-    __shared__ __attribute__((aligned(1024))) unsigned short ring[kStages * kStage];
-    __shared__ __attribute__((aligned(16))) int s_tok[2][kSlots];      // 1-based replica id of every slot of the tile (two tiles), 0 = no token
-    __shared__ __attribute__((aligned(16))) float s_wt[kSlots];        // its routed weight
-    __shared__ int r_first[kMaxRuns];     // run: its first tile,
-    __shared__ int r_slot[kMaxRuns];      //   first slot,
-    __shared__ int r_live[kMaxRuns];      //   32-slot sub-tiles up to its last token | expert << 16
-    __shared__ int s_runs, s_tiles, s_cnt[8];
     const int tid = threadIdx.x, lane = tid & 63, hb = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-
-    // ---- the runs of blocks of one expert, and how many of a run's sub-tiles hold tokens ----
-    const int nb = a.num_blocks;
-    {
-        int* ids = (int*)ring;                        // [nb] expert of every block, 0 = none
-        int* r_end = (int*)ring + kMaxBlocks;         // [kMaxRuns] last block of a run
-        for (int b = tid; b < nb; b += 512) {
-            const int e = a.sorted_expert_ids[b];
-            ids[b] = e >= 1 && e <= a.num_experts ? e : 0;
-        }
-        if (tid < kMaxRuns) r_live[tid] = 0;
-        __syncthreads();
-        int base = 0;
-        for (int c = 0; c < nb; c += 512) {
-            const int b = c + tid;
-            const int e = b < nb ? ids[b] : 0;
-            const bool start = e && (b == 0 || ids[b - 1] != e);
-            const bool end = e && (b == nb - 1 || ids[b + 1] != e);
-            const unsigned long long m = __ballot(start);
-            if (lane == 0) s_cnt[wave] = __popcll(m);
-            __syncthreads();
-            int before = base;
-            for (int w = 0; w < 8; ++w) {
-                if (w < wave) before += s_cnt[w];
-                base += s_cnt[w];
-            }
-            const int upto = before + __popcll(m & ((2ull << lane) - 1ull));   // starts up to and including this block
-            if (start && upto - 1 < kMaxRuns) r_slot[upto - 1] = b;
-            if (end && upto - 1 < kMaxRuns) r_end[upto - 1] = b;
-            __syncthreads();
-        }
-        const int runs = base;
-        if (runs <= kMaxRuns) {
-            // last sub-tile of a run's last block with a token in it (the blocks before it count as full)
-            const int per = a.TILE_M / 4;   // groups of four slots in a block
-            for (int g = tid; g < runs * per; g += 512) {
-                const int r = g / per, q = g - r * per;
-                const int slot = r_end[r] * a.TILE_M + 4 * q;
-                bool any = false;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int t = slot + i < a.num_slots ? a.sorted_token_ids[slot + i] : 0;
-                    any = any || (t >= 1 && t <= a.total_tokens);
-                }
-                if (any) atomicMax(&r_live[r], q / 8 + 1);
-            }
-            __syncthreads();
-            if (wave == 0) {
-                int tiles = 0;
-                for (int r0 = 0; r0 < runs; r0 += 64) {
-                    const int r = r0 + lane;
-                    int n = 0;
-                    if (r < runs) {
-                        const int b = r_slot[r], e = ids[b];
-                        int live = r_live[r];
-                        live = live ? live + (r_end[r] - b) * (a.TILE_M / 32) : (r_end[r] - b) * (a.TILE_M / 32);
-                        n = (live + kMaxL - 1) / kMaxL * strips;
-                        r_live[r] = live | (e - 1) << 16;
-                        r_slot[r] = b * a.TILE_M;
-                    }
-                    int pre = n;
-#pragma unroll
-                    for (int o = 1; o < 64; o <<= 1) {
-                        const int v = __shfl_up(pre, o, 64);
-                        if (lane >= o) pre += v;
-                    }
-                    if (r < runs) r_first[r] = tiles + pre - n;
-                    tiles += __shfl(pre, 63, 64);
-                }
-                if (lane == 0) {
-                    s_runs = runs;
-                    s_tiles = tiles;
-                }
-            }
-        } else if (tid == 0) {   // one tile per 128 slots and strip
-            s_runs = -1;
-            s_tiles = nb * (a.TILE_M / kBlock) * strips;
-        }
-        __syncthreads();
-    }
-    const int runs = s_runs, tiles_all = s_tiles;
+    const int runs = table.runs, tiles_all = table.tiles;
+    const int *const r_first = table.first, *const r_slot = table.slot, *const r_live = table.live;
     const int first0 = lane < runs ? r_first[lane] : 0x7fffffff, first1 = lane + 64 < runs ? r_first[lane + 64] : 0x7fffffff;
-    __syncthreads();   // (the ring's memory is free from here on)
 
     // Workgroup ids congruent mod 8 share an XCD; XCD x takes tiles [x * per, (x + 1) * per), its workgroups with a stride.
     const int per = (tiles_all + 7) >> 3, stride = gridDim.x >> 3;
@@ -444,72 +369,181 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
 }
 
+// Which tiles a launch has is known here only, where the routing is: `rows` = 256 or 128 weight rows per tile, or 0 for 128
+// where they come to no more rounds of the CUs than 256 (a round of them takes 0.82 of the time, 1.23 are two for one; 1800
+// launches of 360 shapes, from even to very uneven routing).  A few tiles more than CUs are a second round, and uneven
+// routing has them where even routing has not: 32 experts of 256, 2048 -> 1024, 256 rows 50 us, one round; experts
+// of 150 to 540 make 270 tiles and 73 us, 128 rows 56.
+template <typename E, int MODE>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void moe_prefill_kernel(const DenseArgs a, int strips4, int strips2, int rows) {
+    constexpr int kRing = kStages * (stage_of(4) > stage_of(2) ? stage_of(4) : stage_of(2));
+    __shared__ __attribute__((aligned(1024))) unsigned short ring[kRing];
+    __shared__ __attribute__((aligned(16))) int s_tok[2][kSlotsMax];   // 1-based replica id of every slot of the tile (two tiles), 0 = no token
+    __shared__ __attribute__((aligned(16))) float s_wt[kSlotsMax];     // its routed weight
+    __shared__ int r_first[kMaxRuns], r_slot[kMaxRuns], r_live[kMaxRuns];
+    __shared__ int s_runs, s_tiles, s_wide, s_cnt[8];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    auto rounds = [](int tiles) { return (((tiles + 7) >> 3) + 31) >> 5; };
+    auto choose = [&](int tiles4, int tiles2) { return rows ? rows == 256 : rounds(tiles2) > rounds(tiles4); };
+
+    // ---- the runs of blocks of one expert, and how many of a run's sub-tiles hold tokens ----
+    const int nb = a.num_blocks;
+    {
+        int* ids = (int*)ring;                        // [nb] expert of every block, 0 = none
+        int* r_end = (int*)ring + kMaxBlocks;         // [kMaxRuns] last block of a run
+        for (int b = tid; b < nb; b += 512) {
+            const int e = a.sorted_expert_ids[b];
+            ids[b] = e >= 1 && e <= a.num_experts ? e : 0;
+        }
+        if (tid < kMaxRuns) r_live[tid] = 0;
+        __syncthreads();
+        int base = 0;
+        for (int c = 0; c < nb; c += 512) {
+            const int b = c + tid;
+            const int e = b < nb ? ids[b] : 0;
+            const bool start = e && (b == 0 || ids[b - 1] != e);
+            const bool end = e && (b == nb - 1 || ids[b + 1] != e);
+            const unsigned long long m = __ballot(start);
+            if (lane == 0) s_cnt[wave] = __popcll(m);
+            __syncthreads();
+            int before = base;
+            for (int w = 0; w < 8; ++w) {
+                if (w < wave) before += s_cnt[w];
+                base += s_cnt[w];
+            }
+            const int upto = before + __popcll(m & ((2ull << lane) - 1ull));   // starts up to and including this block
+            if (start && upto - 1 < kMaxRuns) r_slot[upto - 1] = b;
+            if (end && upto - 1 < kMaxRuns) r_end[upto - 1] = b;
+            __syncthreads();
+        }
+        const int runs = base;
+        if (runs <= kMaxRuns) {
+            // last sub-tile of a run's last block with a token in it (the blocks before it count as full)
+            const int per = a.TILE_M / 4;   // groups of four slots in a block
+            for (int g = tid; g < runs * per; g += 512) {
+                const int r = g / per, q = g - r * per;
+                const int slot = r_end[r] * a.TILE_M + 4 * q;
+                bool any = false;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int t = slot + i < a.num_slots ? a.sorted_token_ids[slot + i] : 0;
+                    any = any || (t >= 1 && t <= a.total_tokens);
+                }
+                if (any) atomicMax(&r_live[r], q / 8 + 1);
+            }
+            __syncthreads();
+            if (wave == 0) {
+                int tiles = 0, tiles4 = 0, tiles2 = 0;
+                for (int r = lane; r < runs; r += 64) {
+                    const int live = r_live[r] + (r_end[r] - r_slot[r]) * (a.TILE_M / 32);
+                    tiles4 += (live + max_live(4) - 1) / max_live(4) * strips4;
+                    tiles2 += (live + max_live(2) - 1) / max_live(2) * strips2;
+                    r_live[r] = live;
+                }
+#pragma unroll
+                for (int o = 32; o; o >>= 1) {
+                    tiles4 += __shfl_xor(tiles4, o, 64);
+                    tiles2 += __shfl_xor(tiles2, o, 64);
+                }
+                const bool wide = choose(tiles4, tiles2);
+                const int most = wide ? max_live(4) : max_live(2), strips = wide ? strips4 : strips2;
+                for (int r0 = 0; r0 < runs; r0 += 64) {
+                    const int r = r0 + lane;
+                    int n = 0;
+                    if (r < runs) {
+                        const int b = r_slot[r], e = ids[b], live = r_live[r];
+                        n = (live + most - 1) / most * strips;
+                        r_live[r] = live | (e - 1) << 16;
+                        r_slot[r] = b * a.TILE_M;
+                    }
+                    int pre = n;
+#pragma unroll
+                    for (int o = 1; o < 64; o <<= 1) {
+                        const int v = __shfl_up(pre, o, 64);
+                        if (lane >= o) pre += v;
+                    }
+                    if (r < runs) r_first[r] = tiles + pre - n;
+                    tiles += __shfl(pre, 63, 64);
+                }
+                if (lane == 0) {
+                    s_runs = runs;
+                    s_tiles = tiles;
+                    s_wide = wide;
+                }
+            }
+        } else if (tid == 0) {   // one tile per 128 slots and strip
+            const int blocks = nb * (a.TILE_M / kBlock);
+            const bool wide = choose(blocks * strips4, blocks * strips2);
+            s_runs = -1;
+            s_tiles = blocks * (wide ? strips4 : strips2);
+            s_wide = wide;
+        }
+        __syncthreads();
+    }
+    // (the ring's memory is free from here on; the same for all lanes, and known to be, as there are barriers in either branch)
+    const Runs table = {r_first, r_slot, r_live, __builtin_amdgcn_readfirstlane(s_runs), __builtin_amdgcn_readfirstlane(s_tiles)};
+    if (__builtin_amdgcn_readfirstlane(s_wide)) walk_tiles<E, MODE, 4>(a, strips4, table, ring, s_tok, s_wt);
+    else walk_tiles<E, MODE, 2>(a, strips2, table, ring, s_tok, s_wt);
+}
+
 }  // namespace
 
 namespace mi {
 namespace moe {
 
 static bool prefill_applicable(const DenseArgs& a) {
-    return !a.a8 && !a.w8 && a.num_blocks <= kMaxBlocks && (int64_t)a.num_blocks * (a.TILE_M / 32) < 65536 && a.num_experts < 32768 &&
+    return !a.a8 && !a.w8 && a.num_blocks > 0 && a.num_blocks <= kMaxBlocks && (int64_t)a.num_blocks * (a.TILE_M / 32) < 65536 && a.num_experts < 32768 &&
            // (32-bit byte offsets of a token's column and of a weight row within its expert)
            (int64_t)a.num_a_cols * a.lda * 2 <= 0xffffffffll && (int64_t)a.N * a.ldb * 2 <= 0xffffffffll;
 }
 
-// Weight rows per tile, 256 or 128, or 0 where the ring kernel is the better one (or the only one).
-// n = replicas per expert on average, give or take their root (random routing).  256 rows where the tiles come to at least
-// 0.7 of the CUs and fill their last round to four fifths, 128 where that makes one nearly full round; neither where the number
-// of tiles per expert hangs on the routing (a few tiles more than CUs are a second round: 64 experts of 170, down
-// projection, 128 rows: 21 -> 32 us), nor below 112 replicas, where the blocks of 128 slots are as good (90: 1.0-1.5 times the ring
-// kernel's time), and with a K below 1024 only from 200 on (128 replicas, K = 512: 0.94-1.26).
-// Of 224 shapes (8 to 64 experts, 36 to 1024 replicas each, hidden 512 / 1024, inter 512 to 2048) the choice takes 0.96 (gate / up)
-// and 0.94 (down) of the ring kernel's time in the mean, 0.75-0.9 and 0.7-0.85 from 256 replicas and K = 1024 on, and
-// 1.01 at worst; always the quickest of the three would be 0.94 and 0.93.
-// MI_MOE_PREFILL = 0 | 2 | 4: never / 128 / 256 rows wherever possible (read at every call).
-int prefill_rows(const DenseArgs& a) {
-    if (!prefill_applicable(a)) return 0;
-    const char* env = getenv("MI_MOE_PREFILL");
-    const int force = env ? atoi(env) : -1;
-    if (force == 2) return 128;
-    if (force == 4) return 256;
-    const double n = (double)a.total_tokens / a.num_experts, dev = sqrt(n);
-    if (force == 0 || n < 112 || a.num_blocks == 0) return 0;
-    const auto tiles = [](double slots, int most) { return cld(cld((int64_t)ceil(slots), (int64_t)32), (int64_t)most); };
-    const int64_t half = a.silu ? 2 : 1;
-    const double rounds4 = a.num_experts * (double)(tiles(n + 2 * dev, 5) * cld((int64_t)a.N / half, 256 / half)) / 256.0;
-    const double rounds2 = a.num_experts * (double)(tiles(n + 2 * dev, 6) * cld((int64_t)a.N / half, 128 / half)) / 256.0;
-    const bool even4 = tiles(n - dev, 5) == tiles(n + 2 * dev, 5), even2 = tiles(n - dev, 6) == tiles(n + 2 * dev, 6);
-    const bool fit2 = even2 && rounds2 >= 0.7 && rounds2 <= 1.0;
-    const bool fit4 = (even4 || rounds4 >= 4.5) && rounds4 >= 0.7 && (rounds4 > 2.5 || rounds4 >= 0.8 * ceil(rounds4)) &&
-                      (a.K >= 1024 || n >= 200);
-    return fit4 && !(fit2 && rounds4 <= 0.7) ? 256 : fit2 ? 128 : 0;
+// True where this kernel is the one to take.  The host knows the replicas per expert n only, not how evenly they are dealt,
+// so the line lies where the kernel is the quicker one for even and for uneven routing alike (router logits ~ N(0, 1) with
+// an offset per expert of 0, 0.25, 0.5, 1 or 2 deviations).  `w`: rounds of the CUs that tiles of 160 x 256 make, an expert's last
+// tile half full; the kernel wins where the last round is well filled, or where there are many, the sooner the longer K is (with
+// K = 512 a tile is over before its transfers are spread: 1.0-1.1 of the ring kernel's time at 3 to 5 rounds), and below 112
+// replicas the blocks of 128 slots are as good (90: 1.0-1.5).
+// 300 shapes (8 to 64 experts, 112 to 1100 replicas each, hidden 512 / 1024, inter 512 to 2048) at the five degrees of
+// unevenness: 0.90-0.91 (gate / up, 97 shapes taken) and 0.83-0.84 (down, 68) of the ring kernel's time at each degree, 1.02 at worst
+// in a shape's mean over them, 1.09 in one launch.  A line drawn for even routing alone was off by up to 1.65.
+static bool pays(double n, int K, double w) {
+    if (n < 112) return false;
+    if (K >= 2048) return w >= 1.28 || (w >= 0.48 && w <= 1.15);
+    if (K >= 1024) return w >= 2.45 || (n >= 200 && ((w >= 1.37 && w <= 1.9) || (w >= 0.84 && w <= 1.05)));
+    return K >= 512 && w >= 5.1;
 }
 
-void prefill_launch(const DenseArgs& a, int rows, hipStream_t s) {
-    const bool wide = rows == 256;
-    const int kW = wide ? 256 : 128;
-    const int strips = a.silu ? (int)cld((int64_t)a.N / 2, (int64_t)(kW / 2)) : (int)cld((int64_t)a.N, (int64_t)kW);
-    const int64_t tiles = (int64_t)a.num_blocks * (a.TILE_M / 32) * strips;   // (at most)
+// MI_MOE_PREFILL = 0 | 2 | 4: never / with 128 / with 256 weight rows per tile wherever possible (read at every call).
+bool prefill_launch(const DenseArgs& a, hipStream_t s) {
+    if (!prefill_applicable(a)) return false;
+    const char* env = getenv("MI_MOE_PREFILL");
+    const int force = env ? atoi(env) : -1, rows = force == 4 ? 256 : force == 2 ? 128 : 0;
+    const int64_t half = a.silu ? 2 : 1;
+    const int strips4 = (int)cld((int64_t)a.N / half, 256 / half), strips2 = (int)cld((int64_t)a.N / half, 128 / half);
+    const double n = (double)a.total_tokens / a.num_experts;
+    if (!rows && (force == 0 || !pays(n, a.K, a.num_experts * (n / 160 + 0.5) * strips4 / 256.0))) return false;
+    const int64_t tiles = (int64_t)a.num_blocks * (a.TILE_M / 32) * strips2;   // (at most)
     const int64_t per_xcd = cld(tiles, (int64_t)8) < 32 ? cld(tiles, (int64_t)8) : 32;
     const dim3 grid((unsigned)(per_xcd * 8));
-#define LAUNCH(ET, MODE)                                                                                       \
-    do {                                                                                                       \
-        if (wide) hipLaunchKernelGGL((moe_prefill_kernel<ET, MODE, 4>), grid, dim3(512), 0, s, a, strips);     \
-        else hipLaunchKernelGGL((moe_prefill_kernel<ET, MODE, 2>), grid, dim3(512), 0, s, a, strips);          \
-    } while (0)
+#define LAUNCH(ET, MODE) hipLaunchKernelGGL((moe_prefill_kernel<ET, MODE>), grid, dim3(512), 0, s, a, strips4, strips2, rows)
+#define NAME(P, WIDE, NARROW) set_variant(rows == 256 ? P "_t128_to160_" WIDE "_k64_ring3" : rows == 128 ? P "_t128_to192_" NARROW "_k64_ring3" : P "_t128_to160_" WIDE "_or_to192_" NARROW "_k64_ring3")
     if (a.silu) {
         if (a.bf16) LAUNCH(BF16, MODE_SILU);
         else LAUNCH(F16, MODE_SILU);
-        set_variant(wide ? "fused_moe_dense_silu_t128_to160_n128x2_k64_ring3" : "fused_moe_dense_silu_t128_to192_n64x2_k64_ring3");
+        NAME("fused_moe_dense_silu", "n128x2", "n64x2");
     } else if (a.acc_shift >= 0) {
         if (a.bf16) LAUNCH(BF16, MODE_ACC);
         else LAUNCH(F16, MODE_ACC);
-        set_variant(wide ? "fused_moe_dense_acc_t128_to160_n256_k64_ring3" : "fused_moe_dense_acc_t128_to192_n128_k64_ring3");
+        NAME("fused_moe_dense_acc", "n256", "n128");
     } else {
         if (a.bf16) LAUNCH(BF16, MODE_PLAIN);
         else LAUNCH(F16, MODE_PLAIN);
-        set_variant(wide ? "fused_moe_dense_t128_to160_n256_k64_ring3" : "fused_moe_dense_t128_to192_n128_k64_ring3");
+        NAME("fused_moe_dense", "n256", "n128");
     }
+#undef NAME
 #undef LAUNCH
+    return true;
 }
 
 }  // namespace moe

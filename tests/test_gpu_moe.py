@@ -839,6 +839,36 @@ def test_prefill_kernel_gives_the_streaming_kernels_bits(ct, orc, make, rows, mo
     check(J(got["separate"]), ref, 5e-2 if d.hidden_states.dtype == torch.bfloat16 else 2e-2)
 
 
+@pytest.mark.parametrize("counts,kw,names", [
+    # (weight rows per tile as the launch picks them: gate / up 256 and down 256; 256 and 128; down 128 in one round; 256 and 256)
+    ([256] * 32, dict(topk=2, hidden_size=1024, intermediate_size=2048), ("silu_", "acc_")),
+    ([20, 150, 170, 200, 220, 250, 260, 270, 280, 290, 300, 330, 350, 380, 400, 226] * 2, dict(topk=2, hidden_size=1024, intermediate_size=2048), ("silu_", "acc_")),
+    ([120, 344] * 8, dict(topk=1, hidden_size=1024, intermediate_size=2048, T=torch.bfloat16), ("", "acc_")),
+    ([560, 1, 900, 219] * 8, dict(topk=2, hidden_size=512, intermediate_size=2048, T=torch.bfloat16), ("silu_", "acc_")),
+    # where a few tiles more than CUs would be a round of their own: the ring kernel
+    ([305] * 32, dict(topk=2, hidden_size=512, intermediate_size=512), ("", "")),
+    ([314] * 16, dict(topk=1, hidden_size=1024, intermediate_size=512), ("", "")),
+])
+def test_prefill_kernel_picks_its_tiles_from_the_routing(ct, counts, kw, names):
+    """Even and uneven routing through the rule as it stands: the streaming kernels' bits whichever tiles a launch picks."""
+    d = _routed(counts, **kw)
+    with _dense_knob("0"):
+        want = _every_path(d, 128)
+    got = _every_path(d, 128)
+    for k in want:
+        assert torch.equal(got[k], want[k]), k
+    tok, exp = ct.moe_align_tile_size_device(d.topk_ids, 128, d.num_experts)
+    c2 = torch.full((d.num_tokens * d.topk, d.intermediate_size), float("nan"), dtype=d.hidden_states.dtype, device="cuda")
+    moe.invoke_fused_moe_kernel(d.hidden_states, d.w1, c2, d.topk_weights, tok, exp, mul_routed_weight=False, num_token_replicas=d.topk,
+                                tile_m=128, tile_n=128, tile_k=64, fuse_silu=True)
+    up = ct.last_variant()
+    out = torch.zeros(d.num_tokens, d.hidden_size, dtype=d.hidden_states.dtype, device="cuda")
+    ct.fused_moe_accumulate_kernel(c2, d.w2, out, d.topk_weights, tok, exp, 128, 128, 64)
+    assert torch.equal(out, want["fused"])
+    for name, part in zip((up, ct.last_variant()), names):
+        assert ("_to160_" in name and "_or_to192_" in name and part in name) if part else "k32_ring" in name, name
+
+
 @pytest.mark.parametrize("rows", ["2", "4"])
 def test_prefill_kernel_on_arrays_that_no_sort_made(ct, rows, monkeypatch):
     """Slots without a token anywhere in a block, whole blocks without one, blocks of one expert apart from each other, blocks
