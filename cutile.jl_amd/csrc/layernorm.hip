@@ -557,6 +557,12 @@ __global__ __launch_bounds__(BLOCK * RG) void ln_bwd_rg_kernel(float* __restrict
     __syncthreads();
     float* dwp = DW + (int64_t)g * lddw;
     float* dbp = DB + (int64_t)g * lddb;
+    if (RG == 1 && S > 1) {   // (rows of more than 4096 elements: all of dW, then all of dB; in turns: 8 slots, 1024 x 4100 17.9 -> 21.2 us)
+        for (int c = threadIdx.x; c < N; c += BLOCK) unsafeAtomicAdd(dwp + c, stage[0][0][c]);
+        __syncthreads();
+        for (int c = threadIdx.x; c < N; c += BLOCK) unsafeAtomicAdd(dbp + c, stage[0][1][c]);
+        return;
+    }
     for (int c = threadIdx.x; c < N; c += BLOCK * RG) {
         float t = stage[0][0][c], u = stage[0][1][c];
 #pragma unroll
@@ -1178,8 +1184,8 @@ extern "C" int mi_layer_norm_bwd_dx_partial_dwdb(
         // which fills a CU by itself: one workgroup per CU, half the flushes.
         // Up to 1024 elements a group is a single wave (no barriers in the walk) and eight groups share a workgroup, at most
         // one per CU, with at least four rows a wave up to 512 elements (64 slots, us, 256 lanes -> a wave: 1024 x 1024 6.8 -> 5.2,
-        // 4096 x 1024 12.6 -> 11.0, 4096 x 700 11.8 -> 9.7).  Streamed inputs of more than 512 elements keep 256 lanes (where
-        // the two meet, 16384 x 1024, 38.2 and 39.3).
+        // 4096 x 1024 12.6 -> 11.0, 4096 x 700 11.8 -> 9.7; with one or two rows a slot 0.1-0.4 us slower, 4 x 1024 3.8 -> 4.1).
+        // Streamed inputs of more than 512 elements keep 256 lanes (where the two meet, 16384 x 1024, 38.2 and 39.3).
         // A slot that one workgroup owns gets plain adds, and the same bits on every run; two add to a zero slot in either
         // order with the same result; from three on the order of arrival decides the last bits.  One row a wave is
         // quicker on many slots (64 slots, 2000 x 512 6.1 -> 5.6 us), but puts more workgroups on slots that have one or two now,
