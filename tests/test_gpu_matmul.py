@@ -255,6 +255,20 @@ def test_matmul_ragged_sizes_split_or_with_transfer_waves_exact(ct, orc, M, N, K
     assert bool((buf[N:] == -77.0).all()) and bool((buf[:, M:] == -77.0).all())
 
 
+@pytest.mark.parametrize("M,N,K,waves", [
+    (502, 349, 1194, False), (850, 1007, 1565, False), (519, 1153, 1595, False), (513, 1153, 1609, True),   # below 60 tiles
+    (898, 1154, 1291, False), (897, 1154, 1309, True), (998, 1666, 998, False), (998, 1666, 1002, True),    # below 112, from there on
+    (292, 3763, 1676, False), (511, 3587, 1700, False),                                                    # few tiles along M
+])
+def test_matmul_misaligned_rows_both_sides_of_the_transfer_waves_rule(ct, orc, M, N, K, waves):
+    rng = np.random.default_rng(K)
+    A = rng.integers(-1, 2, (M, K)).astype(np.float32); B = rng.integers(-1, 2, (K, N)).astype(np.float32)
+    C = torch.empty((N, M), dtype=torch.float32, device="cuda")
+    ct.matmul_kernel(orc.from_julia(A).to(torch.float16).cuda(), orc.from_julia(B).to(torch.float16).cuda(), C, 64, 64, 64)
+    assert ("x64_ring3" in ct.last_variant()) == waves, ct.last_variant()
+    assert np.array_equal(orc.to_julia(C), A @ B)
+
+
 def test_batch_matmul_ragged_split_and_transfer_waves(ct, orc):
     """The same through mi_batch_matmul_kernel: odd batch strides, parts of every entry in slices of their own."""
     rng = np.random.default_rng(12)
