@@ -15,15 +15,15 @@
 //                    (ragged edges are zero-padded on load and clipped on store, as
 //                    ct.load(padding_mode=Zero) / ct.store do).
 //   gemm16_mid       f16/bf16, 128x128x32 workgroup tile with a register look-ahead of one K step, any
-//                    shape; used for larger problems that gemm16_big does not take (rows that are
-//                    not 16-byte aligned, K below 256).
+//                    shape; used for larger problems that gemm16_big does not take (K below 256, rows
+//                    that overlap).
 //   gemm16_big       (gemm_big.hip) f16/bf16, 256x256 workgroup tile, 4 waves of 128x128 (or 256x128 /
 //                    128x128 tiles for problems with few tiles), K step 32 through a ring of four LDS
 //                    stages filled by direct global->LDS loads, XOR-swizzled LDS layouts; used from K = 256
 //                    and 16 tiles of 128x128, or K = 320, on (any alignment and ragged edges in M, N and K are
 //                    handled on the way in; few tiles and a long K are split over K).
 //   gemm16_pc        (gemm_pc.hip) f16/bf16, 128x128 and 256x128 tiles with waves of their own for the
-//                    transfers, for rows off 16-byte boundaries and K >= 1000.
+//                    transfers, for rows off 16-byte boundaries where K is long and tiles are many enough.
 //   gemm32           fp32 via v_mfma_f32_32x32x2_f32 (gfx950 has no TF32-class MFMA;
 //                    the reference rounds fp32 operands to TF32, matmul.jl:49-52), 128x128x16 tile,
 //                    any shape; gemm32_big (gemm32_big.hip), the fp32 sibling of gemm16_big, takes
@@ -516,9 +516,8 @@ int run(const Problem& p, hipStream_t s, bool may_split) {
     }
     const bool f32out = p.out_dtype == MI_F32;
     const int64_t tiles_mid = (int64_t)cld((int64_t)p.M, (int64_t)MT) * cld((int64_t)p.N, (int64_t)MT) * p.batch;
-    // The direct-to-LDS kernel wherever it applies (16-byte aligned rows, K >= 256: with a shorter K the
-    // problem is bound by the stores of C and smaller workgroups in several rounds overlap them better;
-    // it picks its own tile size);
+    // The direct-to-LDS kernels wherever they apply (any alignment, K >= 256: with a shorter K the problem is bound by
+    // the stores of C and smaller workgroups in several rounds overlap them better; they pick tile size and kernel themselves);
     // the register-staged 128x128 kernel for other shapes whose tiles give at least half the CUs work;
     // the 64x64 kernel for what is left (small problems).
     if (big16_applicable(p) && (force == 3 || force == 0)) {

@@ -484,7 +484,7 @@ void big16_launch(const Problem& p, hipStream_t s) {
     // K from 1000 to 4000 the 123 that are taken are at 0.93 of the other kernel's time in the mean, 0.84 to 1.12.
     const int64_t tiles = tiles_of(p, 128, 128);
     if (t != 44 && p.M > 512 && p.K >= (tiles >= 112 ? 1000 : tiles >= 60 ? 1300 : 1600) && misaligned(p) && tiles_of(p, t == 22 ? 128 : 256, 128) <= 256) {
-        pc16_launch(p, t, dma_extent(p), 1, 0, s);
+        pc16_launch(p, t, dma_extent(p), s);
         set_variant(t == 22 ? "gemm16_big_128x128x64_ring3" : "gemm16_big_256x128x64_ring3");
         return;
     }

@@ -1,4 +1,5 @@
-// Pieces shared by the two direct-to-LDS GEMM kernels (gemm_big.hip: 16-bit operands, gemm32_big.hip: fp32).
+// Pieces shared by the direct-to-LDS GEMM kernels (gemm_big.hip and gemm_pc.hip: 16-bit operands, gemm32_big.hip: fp32,
+// moe_dense.hip and moe_prefill.hip: grouped).
 #pragma once
 #include <cstdlib>
 
@@ -26,6 +27,19 @@ __device__ __forceinline__ void stage_barrier() {
     // following LDS reads.  gfx9 encoding: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt[15:14].
     constexpr int imm = (VMCNT & 15) | (7 << 4) | (0 << 8) | ((VMCNT >> 4) << 14);
     __builtin_amdgcn_s_waitcnt(imm);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// waits until at most N transfers are in flight
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
+    asm volatile("" ::: "memory");
+}
+__device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(0xc07f); }   // lgkmcnt(0)
+__device__ __forceinline__ void meet() {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -102,8 +116,8 @@ inline int pick_direct_tile(const Problem& p, int64_t* cost = nullptr) {
 }
 
 // gemm_pc.hip: the kernel whose transfers have waves of their own, with tiles of 256 x 128 (tile = 42) or 128 x 128 (22); kd: the
-// extent of K that the transfers walk; parts > 1: split over K in parts of kchunk into slices of C (see gemm_big.hip).
-void pc16_launch(const Problem& p, int tile, int kd, int parts, int kchunk, hipStream_t s);
+// extent of K that the transfers walk.
+void pc16_launch(const Problem& p, int tile, int kd, hipStream_t s);
 
 }  // namespace gemm
 }  // namespace mi

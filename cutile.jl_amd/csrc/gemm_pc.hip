@@ -2,19 +2,21 @@
 // operands whose rows start off 16-byte boundaries (an odd M or K).
 //
 // What bounds those products is the path into LDS, not the matrix cores: a CU brings 103-118 GB/s of aligned 16-byte chunks,
-// 77 of chunks on 4-byte boundaries, 57 of any others, whatever is in flight, and 2999 x 2100 x 3001 on the kernel of gemm_big.hip
-// takes 60 us, 38 without its transfers.  There a wave that asks for more than the path takes stands at the instruction and
-// multiplies nothing meanwhile.  Here four waves only transfer and four only multiply, one of each per SIMD, which meet
-// once per stage of 64 k; a stage's row of B is one 128-byte line where stages of 32 k ask for every line twice (64-byte
-// runs: 70 GB/s against 94 on the mix of a 256 x 256 tile).
+// 77 of chunks on 4-byte boundaries, 57 of any others, less where the lines come from memory, whatever is in flight.  On the
+// kernel of gemm_big.hip a wave that asks for more than the path takes stands at the instruction and multiplies nothing
+// meanwhile.  Here four waves only transfer and four only multiply, one of each per SIMD, which meet once per stage of 64 k;
+// a stage's row of B is one 128-byte line where stages of 32 k ask for every line twice (64-byte runs: 70 GB/s against 94 on
+// the mix of a 256 x 256 tile).  2999 x 2100 x 3001: transfers alone 55 us (56 with the fragments' reads as well: LDS itself is
+// not short), products alone 33, together 61.
 //
 //   tile 128 x 128 (three stages of 32 KB) or 256 x 128 (of 48 KB), one workgroup per CU; a multiplying wave has 64 x 64 or
 //   128 x 64 of it.  Layouts, fragments, edges and the register-fed step behind the last chunk of k are gemm_big.hip's, with
 //   chunk c of row n of B at position c ^ ((n >> 1) & 7).
 //
-// Measured (us, gemm_big.hip -> this): 2496 x 825 x 3247 35.8 -> 30.1, 3776 x 768 x 1459 20.2 -> 18.2, 2432 x 1536 x 2313
-// 29.1 -> 25.1, 965 x 2048 x 3859 49.4 -> 43.1; 256 x 128 tiles 3000 x 2100 x 3001 49.6 -> 46.7, 2999 x 2100 x 3001 58.6 -> 58.3.
-// With aligned rows it is ahead or behind by up to 10 % without a pattern and is not used.
+// Measured (us, gemm_big.hip -> this, one session): 2496 x 825 x 3247 35.4 -> 30.0, 3776 x 768 x 1459 18.6 -> 17.3, 2432 x 1536 x
+// 2313 27.5 -> 25.4, 965 x 2048 x 3859 49.0 -> 42.3; 256 x 128 tiles 1946 x 2255 x 2995 45.8 -> 41.6, 2999 x 2100 x 3000 61.3 ->
+// 58.1, 3000 x 2100 x 3001 52.9 -> 50.8, 2999 x 2100 x 3001, with both operands on 2-byte boundaries, 64.2 either way.  The rule
+// stands in gemm_big.hip.  With aligned rows it is ahead or behind by up to 10 % without a pattern and is not used.
 //
 // Tried and not kept: A read straight into registers (4 bytes per lane and row of k, transposed by v_perm; no LDS for A): the
 // 256 x 128 tile as fast as before, the 128 x 128 tile 15-20 % slower, as 4-byte requests take the path's time of 16-byte ones.
@@ -31,41 +33,18 @@ constexpr int kStages = 3;
 // Source of every chunk that lies past K.
 __device__ __attribute__((aligned(16))) const unsigned zeros16c[4] = {0u, 0u, 0u, 0u};
 
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-    asm volatile("" ::: "memory");
-}
-__device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(0xc07f); }   // lgkmcnt(0)
-__device__ __forceinline__ void meet() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
-
 // Tile (64*I) m x (64*J) n, a multiplying wave's part (32*I) x (32*J).
 template <typename E, typename OutT, int I, int J>
 __global__ __launch_bounds__(512) void gemm16_pc(const unsigned short* __restrict__ A, int64_t lda, int64_t sa, const unsigned short* __restrict__ B,
                                                  int64_t ldb, int64_t sb, OutT* __restrict__ C, int64_t ldc, int64_t sc, int M, int N, int K,
-                                                 int tiles_m, int tiles_n, int batch, int ksplit, int kchunk, int kpeel) {
+                                                 int tiles_m, int tiles_n, int batch, int kpeel) {
     // K: the extent the transfers walk (a multiple of 8); kpeel: values of k behind it for the register-fed step
     constexpr int BTM = 64 * I, BTN = 64 * J, kStageA = BTM * BK, kStage = kStageA + BTN * BK;
     __shared__ __attribute__((aligned(1024))) unsigned short ring[kStages * kStage];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int total = tiles_m * tiles_n, total_all = total * batch;
-    int L = blockIdx.x, part = 0;
-    if (ksplit > 1) {
-        part = L % ksplit;
-        L /= ksplit;
-        if (part < ksplit - 1) {
-            K = kchunk;
-            kpeel = 0;
-        } else {
-            K -= part * kchunk;
-        }
-    }
-    L = xcd_tile(L, total_all);
+    int L = xcd_tile(blockIdx.x, total_all);
     const int bz = L / total;
     L -= bz * total;
     constexpr int GM = 4;
@@ -73,10 +52,9 @@ __global__ __launch_bounds__(512) void gemm16_pc(const unsigned short* __restric
     const int first_m = (L / per_group) * GM;
     const int gsz = tiles_m - first_m < GM ? tiles_m - first_m : GM;
     const int bm = first_m + (L % per_group) % gsz, bn = (L % per_group) / gsz;
-    const int64_t k_first = (int64_t)part * kchunk;
     const int KD = (K + BK - 1) / BK;   // stages, >= 3 (checked on the host)
-    A += (int64_t)bz * sa + k_first * lda;
-    B += (int64_t)bz * sb + k_first;
+    A += (int64_t)bz * sa;
+    B += (int64_t)bz * sb;
 
     if (wave >= 4) {
         // ---- transfers ----
@@ -212,7 +190,7 @@ __global__ __launch_bounds__(512) void gemm16_pc(const unsigned short* __restric
         spread();
     }
 
-    if (kpeel > 0) {   // (same for all workgroups of a part)
+    if (kpeel > 0) {   // (same for the whole grid)
         // k = K .. K + kpeel - 1 as the first values of one 16-wide MFMA step: the lower half-wave holds k 0..7 of its
         // row of B / column of A, the upper half-wave zeros.
         const unsigned short *Ap = A + (int64_t)K * lda, *Bp = B + K;
@@ -232,7 +210,7 @@ __global__ __launch_bounds__(512) void gemm16_pc(const unsigned short* __restric
         }
         mma(fp);
     }
-    C += ((int64_t)bz * ksplit + part) * sc;
+    C += (int64_t)bz * sc;
     store_tile<E, OutT, I, J>(acc, C, ldc, M, N, bm * BTM, bn * BTN, wm, wn, BTM, BTN, lane);
 }
 
@@ -241,12 +219,12 @@ __global__ __launch_bounds__(512) void gemm16_pc(const unsigned short* __restric
 namespace mi {
 namespace gemm {
 
-void pc16_launch(const Problem& p, int tile, int kd, int parts, int kchunk, hipStream_t s) {
+void pc16_launch(const Problem& p, int tile, int kd, hipStream_t s) {
     const int btm = tile == 42 ? 256 : 128, tiles_m = (p.M + btm - 1) / btm, tiles_n = (p.N + 127) / 128;
-    const dim3 grid((unsigned)(tiles_m * tiles_n * p.batch * parts));
+    const dim3 grid((unsigned)(tiles_m * tiles_n * p.batch));
 #define PC(E, O, I, J)                                                                                                                     \
     hipLaunchKernelGGL((gemm16_pc<E, O, I, J>), grid, dim3(512), 0, s, (const unsigned short*)p.A, p.lda, p.sa, (const unsigned short*)p.B, p.ldb, \
-                       p.sb, (O*)p.C, p.ldc, p.sc, p.M, p.N, kd, tiles_m, tiles_n, p.batch, parts, kchunk, p.K - kd)
+                       p.sb, (O*)p.C, p.ldc, p.sc, p.M, p.N, kd, tiles_m, tiles_n, p.batch, p.K - kd)
 #define TILE(E, O)                         \
     do {                                   \
         if (tile == 42) PC(E, O, 4, 2);    \

@@ -1,13 +1,14 @@
 // Token-gather grouped GEMM of the MoE for prefill sizes (fused_moe_kernel, examples/moe.jl:45-105): the products of
 // moe_dense.hip with waves of their own for the transfers.
 //
-// What bounds it: a CU brings operands into LDS at 118 GB/s at most (whole, aligned 128-byte lines from the L2; 50-70 GB/s in
-// runs of 64 bytes), and a wave that asks for more than the path takes stands at the instruction.  On the ring kernel of
-// moe_dense.hip, whose waves multiply and transfer, that time is lost to the matrix cores.  Here a workgroup (one per CU,
-// persistent) is four waves that only transfer and four that only multiply, one of each per SIMD, which meet once per stage
-// of 64 k, so a stage's rows are whole lines.  Without transfers 4096 tokens top-2 of 32 experts (1024 hidden, 2048 inter) take
-// 78 + 47 us (gate / up + down projection), without products 89 + 58, together 107 + 60; zeros in place of the data take 90 + 59:
-// the first is close to the power limit.  The ring kernel takes 126 + 86.
+// What bounds it: the transfers into LDS at the latency of memory.  A CU brings 118 GB/s of whole, aligned 128-byte lines from
+// the L2 (50-70 in runs of 64 bytes), but requests are answered in order, and token rows that the L2 has wait behind weight
+// lines that it has not: 40-46 GB/s here.  On the ring kernel of moe_dense.hip, whose waves multiply and transfer, a wave that
+// asks for more than the path takes stands at the instruction, and that time is lost to the matrix cores.  Here a workgroup
+// (one per CU, persistent) is four waves that only transfer and four that only multiply, one of each per SIMD, which meet once
+// per stage of 64 k, so a stage's rows are whole lines.  4096 tokens top-2 of 32 experts, evenly routed (1024 hidden, 2048 inter,
+// gate / up + down projection): without products 78 + 41 us, 7 of the latter the packed atomics of the one round's
+// end, without transfers 70 + 42, together 93 + 51.  The ring kernel takes 115 + 66.
 //
 //   tile = up to 160 slots x 256 weight rows, a wave all slots x 64 rows (10 MFMA 32x32x16 tiles), or up to 192 slots x 128
 //   rows, a wave every second 32-slot sub-tile x 64 rows; three stages of 52 / 40 KB.  A launch picks one of the two from the table
@@ -46,17 +47,6 @@ constexpr int MODE_PLAIN = 0, MODE_SILU = 1, MODE_ACC = 2;
 // Source of every chunk that lies past K.
 __device__ __attribute__((aligned(16))) const unsigned zeros16p[4] = {0u, 0u, 0u, 0u};
 
-__device__ __forceinline__ void wait_lds() { __builtin_amdgcn_s_waitcnt(0xc07f); }   // lgkmcnt(0)
-__device__ __forceinline__ void meet() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-    __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-    asm volatile("" ::: "memory");
-}
 // waits until at most the transfers of the youngest STAGES stages, W + live sub-tiles each, are in flight
 template <int STAGES, int W>
 __device__ __forceinline__ void wait_transfers(int live) {
