@@ -41,8 +41,9 @@
 // Heads of 128 with about one workgroup per CU and a walk of eight tiles or more (pick_inside): two groups of four waves
 // share a workgroup's queries and take every other tile (KG = 2), so that a SIMD has two waves to choose from; their
 // accumulators meet in LDS.  Bound then by the SIMDs' issue of exponentials and products: 1.03 us a tile, 1.37 with one
-// group.  The weights refer to each tile's own maximum (OWN), so that no result is further from float64 than the split
-// over workgroups, which has a maximum per part, left it (180 shapes: 0.95 to 1.00 of its error; 1.03 with one reference).
+// group.  The weights refer to each tile's own maximum (OWN), so that no result is further from float64 than the kernels that
+// took these launches before left it (the split over workgroups, which has a maximum per part: 216 shapes, 0.94 to 1.00 of its
+// error, 1.03 with one reference; the pipelined kernel: 62 shapes, 0.95 in the mean, 0.99 at most; normal and peaked scores).
 //
 // Grouped heads with few queries (`pack` = QUERY_GROUP_SIZE when Sq <= 64): the heads that share a K / V head are
 // stacked as rows of one query tile -- row r is query r % Sq of head r / Sq of the group -- so their common keys are
@@ -1095,22 +1096,21 @@ extern "C" int mi_fmha_kernel(const mi_tile_array* Q, const mi_tile_array* K, co
     // A decode offset that already exposes every key to the first query makes the mask a no-op.
     const bool causal = CAUSAL != 0 && input_pos < Skv - 1;
     {
-        // MI_FMHA_KERNEL=dma keeps the double-buffered kernel below for every shape (comparison runs).
-        static const bool no_pipe = [] {
-            const char* e = getenv("MI_FMHA_KERNEL");
-            return e && strcmp(e, "dma") == 0;
-        }();
+        // MI_FMHA_KERNEL, read at every call: dma keeps the double-buffered kernel below for every shape (comparison runs), pipe
+        // takes the pipelined kernel for heads of 128 whenever it can run.
+        const char* const e = getenv("MI_FMHA_KERNEL");
+        const bool no_pipe = e && strcmp(e, "dma") == 0;
         fmha::Problem pr{Q, K, V, Out, H, QUERY_GROUP_SIZE, scale2, input_pos, causal, dt == MI_BF16};
         if (!no_pipe && fmha::pipe_applicable(pr)) {
             fmha::pipe_launch(pr, s);
             return launch_status();
         }
         if (!no_pipe && fmha::pipe128_applicable(pr)) {
-            // (pipe: the kernel for heads of 128 whenever it can run; read at every call)
-            const char* e = getenv("MI_FMHA_KERNEL");
             const int64_t wgs = cld(Sq, (int64_t)kQB) * B * H;
             const int parts = pick_parts(wgs, B * H * Sq, 128, (int)Sq, (int)Skv, causal, input_pos);
-            // (not causal, keys of another sequence: as before the kernel with two groups of waves, 45 us : 31 us there)
+            // (Strides of 2^24 elements and more are not for two groups of waves.  Launches that are not causal and have another number
+            // of keys than queries stay on the pipelined kernel, the slower of the two there: 1 x 32 heads, 954 queries of 1787 keys 53 us, 39
+            // with two groups; 0.70-0.80 of the time on 24 shapes.)
             const bool inside = (causal || Sq == Skv) && K->strides[1] < (1 << 24) && V->strides[1] < (1 << 24) &&
                                 pick_inside(wgs, B * H * Sq, 128, (int)Sq, (int)Skv, causal, input_pos, scale2, parts);
             if ((e && strcmp(e, "pipe") == 0) || (!inside && fmha::pipe128_pays(pr, parts))) {

@@ -406,6 +406,7 @@ def test_fmha_heads_of_128_every_head_walked_once_longest_first(ct, orc, monkeyp
     data = fmha.prepare(batch=batch, heads=heads, seq_q=sq, seq_kv=sq, d_k=128, d_v=128, query_group_size=qg, causal=True, T=torch.float16)
     out = torch.full_like(data.Q, float("nan"))
     fmha.cutile_fmha(data.Q, data.K, data.V, query_group_size=qg, causal=True, out=out)
+    assert ct.last_variant() == ("fmha_pipe_d128_q128_kv32_ring4" if kernel == "pipe" else "fmha_dma_q128_kv64_d128_w32q")
     ref = orc.fmha_general(*(orc.to_julia(t) for t in (data.Q, data.K, data.V)), causal=True, input_pos=0)
     check(orc, out, ref, 2e-2)
 
