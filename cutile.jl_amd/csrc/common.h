@@ -127,7 +127,8 @@ __device__ __forceinline__ float block_reduce(float v, float* red, Op op, float 
 }
 
 // fp32 -> bfloat16 bits, round to nearest even: one v_cvt_pk_bf16_f32 where the integer formula (add half an ulp and the
-// parity bit, NaNs apart) takes five instructions and a select.  Same bits for all 2^32 inputs, NaNs included.
+// parity bit, NaNs quieted apart) takes five instructions and a select.  The same bits, compared on the device for all 2^32
+// inputs; the GEMM tests hold ties, overflow, infinities and NaN to the formula.
 __device__ __forceinline__ unsigned short to_bf16(float v) { return __builtin_bit_cast(unsigned short, (__bf16)v); }
 
 // Storage-type conversion helpers (fp32 compute).

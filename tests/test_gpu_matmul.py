@@ -269,6 +269,38 @@ def test_matmul_misaligned_rows_both_sides_of_the_transfer_waves_rule(ct, orc, M
     assert np.array_equal(orc.to_julia(C), A @ B)
 
 
+@pytest.mark.parametrize("K", [16, 256, 1001])
+def test_matmul_bf16_results_round_to_nearest_even(ct, K):
+    """The same product stored as fp32 and as bf16, the latter against the integer formula on the former's bits: ties and their
+    neighbours, the largest values, infinities, NaN, and what the matrix cores leave of denormal sums."""
+    rng = np.random.default_rng(K)
+    M, N = 20_001, 9
+    bits = (rng.integers(0, 2**32, M, dtype=np.uint64) & 0xFFFF0000).astype(np.uint32)
+    bits |= rng.choice(np.array([0, 1, 0x7FFF, 0x8000, 0x8001, 0xFFFF], dtype=np.uint32), M)      # the 16 bits that go
+    bits[::5] ^= rng.integers(0, 2**16, bits[::5].size).astype(np.uint32)
+    bits[:12] = [0x7F7F7FFF, 0x7F7F8000, 0x7F7FFFFF, 0xFF7F8000, 0x7F800000, 0xFF800000, 0x7FC00000, 0x00008000, 0x00018000, 0x80008000, 0x007FFFFF, 0]
+    x = torch.from_numpy(bits.view(np.float32).copy())
+    # three bfloat16 pieces that add up to x without rounding (by truncation, so that none overflows)
+    cut = lambda v: (v.view(torch.int32) & -65536).view(torch.float32)
+    hi = cut(x)
+    mid = torch.where(hi.isfinite(), cut(x - hi), 0.0)
+    lo = torch.where(hi.isfinite(), x - hi - mid, 0.0)
+    A = torch.zeros(K, M, dtype=torch.bfloat16)
+    for row, piece in zip((1, K // 2, K - 1), (hi, mid, lo)):
+        A[row] = piece.to(torch.bfloat16)
+    A, B = A.cuda(), torch.ones(N, K, dtype=torch.bfloat16, device="cuda")
+    wide, narrow = (torch.empty(N, M, dtype=t, device="cuda") for t in (torch.float32, torch.bfloat16))
+    ct.matmul_kernel(A, B, wide, 64, 64, 64)
+    ct.matmul_kernel(A, B, narrow, 64, 64, 64)
+    u = wide.cpu().numpy().view(np.uint32).astype(np.uint64)
+    nan = (u & 0x7FFFFFFF) > 0x7F800000
+    want = np.where(nan, (u >> 16) | 0x40, (u + 0x7FFF + ((u >> 16) & 1)) >> 16).astype(np.uint16)
+    assert np.array_equal(narrow.view(torch.int16).cpu().numpy().view(np.uint16), want)
+    normal = ((bits & 0x7F800000) != 0) & ((bits & 0x7FFFFFFF) <= 0x7F800000) & ((bits & 0x7F800000) > (24 << 23))
+    assert np.array_equal(u[0][normal], bits[normal].astype(np.uint64))      # (the sums are what they are meant to be)
+    assert nan[:, 6].all() and ((want & 0x7FFF) == 0x7F80).any()
+
+
 def test_batch_matmul_ragged_split_and_transfer_waves(ct, orc):
     """The same through mi_batch_matmul_kernel: odd batch strides, parts of every entry in slices of their own."""
     rng = np.random.default_rng(12)
