@@ -674,7 +674,7 @@ def parity_errors(ct):
 
 
 def headline(ct, steps, warmup):
-    """configs[1]: LayerNorm fwd+bwd and softmax on 4096x4096 fp32.  Returns seconds per step,
+    """LayerNorm fwd+bwd and softmax on 4096x4096 fp32.  Returns seconds per step,
     per-stage average durations from events inside the timed region, and algorithmic bytes."""
     import torch
     from cutile_jl_amd.examples import layernorm, softmax

@@ -480,7 +480,7 @@ void big16_launch(const Problem& p, hipStream_t s) {
     // cores' meanwhile (gemm_pc.hip; one workgroup per CU).  With aligned rows the two kernels are within 10 % either way, and so
     // they are with a short K or an M of few tiles, where the other kernel's four waves are through their first stages sooner:
     // the fewer tiles of 128 x 128, the longer K has to be (us, gemm_big.hip : this, 502 x 349 x 1194 12.8 : 13.6, 1584 x 344 x 1450
-    // 14.2 : 15.2, 292 x 3763 x 1676 15.6 : 17.0; 2267 x 366 x 1722 24.9 : 21.7, 2739 x 777 x 1694 24.8 : 21.2).  Of 260 shapes with
+    // 14.2 : 15.2, 292 x 3763 x 1676 15.6 : 17.0; 2267 x 366 x 1722 24.9 : 21.7, 2739 x 777 x 1694 24.8 : 21.2).  Of 340 shapes with
     // K from 1000 to 4000 the 123 that are taken are at 0.93 of the other kernel's time in the mean, 0.84 to 1.12.
     const int64_t tiles = tiles_of(p, 128, 128);
     if (t != 44 && p.M > 512 && p.K >= (tiles >= 112 ? 1000 : tiles >= 60 ? 1300 : 1600) && misaligned(p) && tiles_of(p, t == 22 ? 128 : 256, 128) <= 256) {

@@ -359,11 +359,11 @@ __device__ __forceinline__ void walk_tiles(const DenseArgs& a, int strips, const
     }
 }
 
-// Which tiles a launch has is known here only, where the routing is: `rows` = 256 or 128 weight rows per tile, or 0 for 128
-// where they come to no more rounds of the CUs than 256 (a round of them takes 0.82 of the time, 1.23 are two for one; 1800
-// launches of 360 shapes, from even to very uneven routing).  A few tiles more than CUs are a second round, and uneven
-// routing has them where even routing has not: 32 experts of 256, 2048 -> 1024, 256 rows 50 us, one round; experts
-// of 150 to 540 make 270 tiles and 73 us, 128 rows 56.
+// `rows`: 256 or 128 weight rows per tile, or 0 for whichever is the quicker with the routing at hand, which is known here only:
+// 128 where they make no more rounds of the CUs than 256 (as many rounds: 0.82 of the time of 256; two for one: 1.23; 3600 launches
+// of 360 shapes, from even to very uneven routing).  A few tiles more than CUs are a second round, and uneven routing has them
+// where even routing has not: 32 experts of 256, 2048 -> 1024, take 50 us with 256 rows, one round; with experts of 150 to 540
+// they are 270 tiles and take 73, with 128 rows 56.
 template <typename E, int MODE>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void moe_prefill_kernel(const DenseArgs a, int strips4, int strips2, int rows) {
     constexpr int kRing = kStages * (stage_of(4) > stage_of(2) ? stage_of(4) : stage_of(2));
