@@ -69,7 +69,7 @@ def test_few_queries_is_no_further_off_than_the_kernels_it_replaces(ct, monkeypa
         assert not ct.last_variant().startswith("fmha_few")
         monkeypatch.delenv("MI_FMHA_FEW")
         ref = _reference(Q, K, V, 0, True)
-        assert _err(got, ref) <= 1.005 * _err(old, ref)
+        assert _err(got, ref) <= (0.8 if dim == 64 else 1.0) * _err(old, ref)
 
 
 @pytest.mark.parametrize("dim,B,H,sq,skv,few", [
@@ -86,14 +86,52 @@ def test_both_sides_of_the_rule(ct, dim, B, H, sq, skv, few):
     assert _err(got[:1, :4], _reference(Q[:1, :4], K[:1, :4], V[:1, :4], 0, False)) <= 2**-10
 
 
-def test_few_queries_infinities_and_nan(ct):
-    """A NaN in a key reaches the queries that see it and no others; an infinite value likewise."""
+@pytest.mark.parametrize("dim", [64, 128])
+def test_few_queries_infinities_and_nan(ct, dim):
+    """A NaN in a key reaches the queries that see it and no others; an infinite value, and a score of either infinity, likewise."""
     g = torch.Generator(device="cuda").manual_seed(3)
-    Q, K, V = (torch.empty(1, 4, 200, 64, device="cuda", dtype=torch.float16).normal_(0, 1, generator=g) for _ in range(3))
-    clean = fmha.cutile_fmha(Q, K, V, causal=True)
-    assert ct.last_variant().startswith("fmha_few")
-    K[0, 1, 70, 5] = float("nan")
-    got = fmha.cutile_fmha(Q, K, V, causal=True)
-    bad = torch.isnan(got.float()).any(-1)[0]
-    assert bad[1, 70:].all() and not bad[1, :70].any() and not bad[[0, 2, 3]].any()
-    assert torch.equal(got[0, 1, :70], clean[0, 1, :70])
+    Q, K, V = (torch.empty(1, 4, 200, dim, device="cuda", dtype=torch.float16).normal_(0, 1, generator=g) for _ in range(3))
+    Q[..., 5] = Q[..., 5].abs() + 0.25
+    def attend(K, V):
+        got = fmha.cutile_fmha(Q, K, V, causal=True)
+        assert ct.last_variant().startswith(f"fmha_few_d{dim}")
+        return got
+    clean = attend(K, V)
+    for value in (float("nan"), float("inf")):
+        k = K.clone(); k[0, 1, 70, 5] = value                       # (a score of +inf: inf - inf)
+        got = attend(k, V)
+        bad = torch.isnan(got.float()).any(-1)[0]
+        assert bad[1, 70:].all() and not bad[1, :70].any() and not bad[[0, 2, 3]].any()
+        assert torch.equal(got[0, 1, :70], clean[0, 1, :70])
+    k = K.clone(); k[0, 1, 70, 5] = float("-inf")                   # a weight of zero
+    got = attend(k, V)
+    keep = [i for i in range(200) if i != 70]
+    ref = _reference(Q[:, 1:2, 71:], K[:, 1:2, keep].contiguous(), V[:, 1:2, keep].contiguous(), 70, True)
+    assert _err(got[:, 1:2, 71:], ref) <= 2**-11 and torch.equal(got[0, 1, :70], clean[0, 1, :70])
+    v = V.clone(); v[0, 1, 70, 9] = float("inf")
+    got = attend(K, v)
+    assert (got[0, 1, 70:, 9] == float("inf")).all()
+    got[0, 1, 64:, 9] = clean[0, 1, 64:, 9]                         # (queries that walk its half without seeing it: 0 * inf)
+    assert torch.equal(got, clean)
+
+
+@pytest.mark.parametrize("T", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("dim,B,H,S,waves", [(64, 1, 4, 1408, 4), (64, 2, 32, 755, 2), (128, 1, 4, 1408, 4), (128, 6, 8, 576, 2)])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("levels", [
+    (0, 20, -30, 10, 25, -60, 24), (25, 0), (0, 25), (-40, -38, -36, -34, -32, -30, -28, -26), (24, 18, 12, 6, 0, -6, -12, -18),
+    (20, -45, 20, -45), (3, -3),
+], ids=["up_down_up", "down", "up", "rising", "falling", "every_second", "within_the_limit"])
+def test_few_queries_scores_that_rise_and_fall_from_half_to_half(ct, dim, B, H, S, waves, T, causal, levels):
+    """Each half of 32 keys has scores around a level of its own, the levels repeating along the keys (in units of log 2 up to 36 and
+    -87 apart): what a wave's reference follows up, and heads of 128 down as far as 2^-8 of the largest weight."""
+    g = torch.Generator(device="cuda").manual_seed(S)
+    Q, K, V = (torch.empty(B, H, S, dim, device="cuda").normal_(0, 1, generator=g) for _ in range(3))
+    Q[..., 0] = math.sqrt(dim)
+    K[..., 0] = torch.tensor([float(levels[(k // 32) % len(levels)]) for k in range(S)], device="cuda")
+    Q, K, V = (x.to(T) for x in (Q, K, V))
+    got = fmha.cutile_fmha(Q, K, V, causal=causal)
+    if causal:
+        assert ct.last_variant() == f"fmha_few_d{dim}_q32_keys{waves}", ct.last_variant()
+    # (the bounds of test_few_queries)
+    assert _err(got, _reference(Q, K, V, 0, causal)) <= (2**-8 if T == torch.bfloat16 else 2**-11)

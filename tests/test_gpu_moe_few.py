@@ -72,3 +72,88 @@ def test_which_launches_the_rule_takes(ct, orc, tokens, E, K, N, off, routed, fe
     assert ct.last_variant().startswith("fused_moe_few_") == few, ct.last_variant()
     ref = np.stack([W[t % E].float().numpy() @ A[t].float().cpu().numpy() for t in range(tokens)])
     assert np.array_equal(C.float().cpu().numpy(), ref)
+
+
+def _exact(orc, tokens, topk, E, K, N, T, e4m3, seed=0):
+    """Small integers, so every product below is exact: (A, B, b_scale, tok, exp, weights (tokens, topk), result before the weights)."""
+    rng = np.random.default_rng(seed + K + N)
+    A = rng.integers(-2, 3, (tokens, K)).astype(np.float32); W = rng.integers(-1, 2, (E, N, K)).astype(np.float32)
+    ids = np.stack([rng.permutation(E)[:topk] + 1 for _ in range(tokens)]).astype(np.int64)
+    tok, exp = orc.moe_align_tile_size(ids, 32, E)
+    scale = 2.0 ** rng.integers(-1, 2, (E, N))
+    ref = np.stack([W[e - 1] @ A[t] * (scale[e - 1] if e4m3 else 1) for t in range(tokens) for e in ids[t]])
+    weights = (2.0 ** rng.integers(-1, 2, (tokens, topk))).astype(np.float32)
+    cuda = lambda x, t: torch.from_numpy(np.ascontiguousarray(x)).to(t).cuda()
+    return (cuda(A, T), cuda(W, torch.float8_e4m3fn if e4m3 else T), cuda(scale, torch.float32) if e4m3 else None, cuda(tok, torch.int32),
+            cuda(exp, torch.int32), cuda(weights.T, T), weights, ref)
+
+
+@pytest.mark.parametrize("T", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("e4m3", [False, True])
+@pytest.mark.parametrize("N,pad,off", [(258, 0, 0), (257, 0, 0), (321, 7, 0), (256, 2, 0), (256, 4, 2), (260, 4, 4), (259, 5, 1), (63, 1, 3)])
+def test_results_off_the_stores_of_four(ct, orc, N, pad, off, e4m3, T):
+    """N, a leading dimension and a start of C that are no multiples of four: the stores go element by element, and nothing around them
+    is touched."""
+    A, B, scale, tok, exp, w2d, weights, ref = _exact(orc, 13, 2, 4, 272, N, T, e4m3)
+    flat = torch.full((off + 26 * (N + pad) + 16,), 99.0, dtype=T, device="cuda")
+    C = flat[off:off + 26 * (N + pad)].view(26, N + pad)[:, :N]
+    for mul in (False, True):
+        flat.fill_(99.0)
+        ct.fused_moe_kernel(A, B, C, w2d, tok, exp, 2, mul, 32, 128, 64, b_scale=scale)
+        assert ct.last_variant().startswith("fused_moe_few_t32"), ct.last_variant()
+        want = ref * weights.reshape(-1, 1) if mul else ref
+        # (integers up to 2^11 and a power of two are exact in f16; those beyond 2^8 in bf16 are rounded to nearest)
+        assert torch.equal(C.cpu(), torch.from_numpy(want).to(T))
+        assert flat.ne(99.0).sum().item() <= 26 * N and bool((flat[:off] == 99.0).all()) and bool((flat[off + 26 * (N + pad):] == 99.0).all())
+        assert pad == 0 or bool((flat[off:off + 26 * (N + pad)].view(26, N + pad)[:, N:] == 99.0).all())
+
+
+@pytest.mark.parametrize("e4m3", [False, True])
+@pytest.mark.parametrize("half", [129, 130, 31, 128])
+def test_silu_results_off_the_stores_of_four(ct, orc, half, e4m3):
+    """The epilogue against the projection and silu_and_mul_kernel one after the other, bit for bit."""
+    A, B, scale, tok, exp, w2d, weights, ref = _exact(orc, 13, 2, 4, 272, 2 * half, torch.float16, e4m3)
+    A = A * 0.0625
+    flat = torch.full((26 * (half + 1) + 8,), 99.0, dtype=torch.float16, device="cuda")
+    C = flat[:26 * (half + 1)].view(26, half + 1)[:, :half]
+    ct.fused_moe_silu_kernel(A, B, C, w2d, tok, exp, 2, False, 32, 128, 64, b_scale=scale)
+    assert ct.last_variant().startswith("fused_moe_few_silu"), ct.last_variant()
+    both = torch.empty(26, 2 * half, dtype=torch.float16, device="cuda"); want = torch.empty(26, half, dtype=torch.float16, device="cuda")
+    ct.fused_moe_kernel(A, B, both, w2d, tok, exp, 2, False, 32, 128, 64, b_scale=scale)
+    ct.silu_and_mul_kernel(both[:, :half], both[:, half:], want, 256)
+    assert torch.equal(C, want) and bool((flat[:26 * (half + 1)].view(26, half + 1)[:, half:] == 99.0).all()) and bool((flat[26 * (half + 1):] == 99.0).all())
+
+
+@pytest.mark.parametrize("form", ["plain", "silu", "accumulate"])
+@pytest.mark.parametrize("bad", [0, 5, -3, 2**30])
+def test_experts_out_of_range_and_slots_without_a_token(ct, orc, form, bad):
+    """A block of an expert that does not exist writes nothing, neither does a slot whose token does not exist, and the routed weights may
+    be a strided view."""
+    N = 264
+    A, B, _, tok, exp, w2d, weights, ref = _exact(orc, 13, 2, 4, 272, N, torch.float16, False)
+    total, exp, tok = 26, exp.clone(), tok.clone()
+    first = tok[:32].clone()
+    exp[0] = bad                                                             # the first expert's tokens
+    second = tok[32:64]; live = int((second <= total).sum())
+    dropped = int(second[live - 1]); second[live - 1] = -7                     # and the last of the second's
+    lost = sorted({int(t) - 1 for t in first if 1 <= int(t) <= total} | {dropped - 1})
+    keep = [f for f in range(total) if f not in lost]
+    wide = torch.full((3, 2 * 13 + 3), float("nan"), dtype=torch.float16, device="cuda")
+    view = wide[:2, 1:27:2]; view.copy_(w2d)
+    if form == "accumulate":
+        # (one replica per column of A: the second projection's input)
+        A2 = A.repeat_interleave(2, 0).contiguous()
+        out = torch.zeros(13, N, dtype=torch.float16, device="cuda")
+        ct.fused_moe_accumulate_kernel(A2, B, out, view, tok, exp, 32, 128, 64)
+        want = ref * weights.reshape(-1, 1); want[lost] = 0
+        assert ct.last_variant().startswith("fused_moe_few_acc"), ct.last_variant()
+        assert torch.equal(out.cpu(), torch.from_numpy(want.reshape(13, 2, N).sum(1)).half())
+        return
+    n = N // 2 if form == "silu" else N
+    C = torch.full((total, n), 99.0, dtype=torch.float16, device="cuda")
+    launch = ct.fused_moe_silu_kernel if form == "silu" else ct.fused_moe_kernel
+    launch(A * 0.0625 if form == "silu" else A, B, C, view, tok, exp, 2, form == "plain", 32, 128, 64)
+    assert ct.last_variant().startswith("fused_moe_few_"), ct.last_variant()
+    assert bool((C[lost] == 99.0).all()) and not bool((C[keep] == 99.0).all(1).any())
+    if form == "plain":
+        assert torch.equal(C[keep].cpu(), torch.from_numpy((ref * weights.reshape(-1, 1))[keep]).half())
