@@ -122,10 +122,16 @@ __device__ __forceinline__ void place_group(int e, int N, int& col, int& skip) {
         skip = e + 4 <= N ? 0 : e < N ? e + 4 - N : 4;
     }
 }
+// (A template's parameter would lose the typedef's alignment and promise 16 bytes: loads at 4-byte boundaries are written out here.)
 typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 template <bool ALIGNED, bool NT>
 __device__ __forceinline__ f32x4 load_group(const float* p) {
-    return ALIGNED ? ld_global<NT>(reinterpret_cast<const f32x4*>(p)) : (f32x4)ld_global<NT>(reinterpret_cast<const f32x4_any*>(p));
+    if constexpr (ALIGNED) {
+        return ld_global<NT>(reinterpret_cast<const f32x4*>(p));
+    } else {
+        const f32x4_any* const q = reinterpret_cast<const f32x4_any*>(p);
+        return NT ? __builtin_nontemporal_load(q) : *q;
+    }
 }
 // (rows off 16 bytes through the L2, where the lines that two stores share meet; streamed, each part went to memory by itself)
 template <bool ALIGNED>
