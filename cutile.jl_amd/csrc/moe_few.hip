@@ -251,10 +251,12 @@ namespace moe {
 // tokens top-2 of 16, K = 1408 e4m3 33 : 29, 224 top-2 of 8 35 : 28, 512 top-2 of 16, 320 workgroups, 46 : 37; but 256 top-4 of 32, 384
 // workgroups, K = 1024 and 1408 37.2 : 38.0 and 46.2 : 47.5, K = 512 and 2048 30.2 : 29.3 and 63.6 : 59.6; 283 top-4, 816, 93 : 103).
 // The line is the same for every epilogue of a projection, so fused and separate launches of a call add in the same order.  MI_MOE_FEW=0,
-// read at every call, and the settings that force another kernel switch it off.
+// read at every call, and the settings that force another kernel or a shape of one (MI_MOE_DENSE*, MI_MOE_PREFILL) switch it off.
 bool few_launch(const DenseArgs& a, hipStream_t s) {
     const char* env = getenv("MI_MOE_FEW");
-    if (a.a8 || (env && atoi(env) == 0) || getenv("MI_MOE_DENSE") || getenv("MI_MOE_PREFILL")) return false;
+    if (a.a8 || (env && atoi(env) == 0)) return false;
+    for (const char* forced : {"MI_MOE_DENSE", "MI_MOE_PREFILL", "MI_MOE_DENSE_J", "MI_MOE_DENSE_WIDE", "MI_MOE_DENSE_STREAM"})
+        if (getenv(forced)) return false;
     const int per16 = a.w8 ? 16 : 8;   // weights per 16-byte chunk
     if (a.TILE_M % kTS || a.K % per16 || a.K < 256 || a.N < 1 || (a.silu && a.N % 2)) return false;
     if (!aligned(a.A, 16) || !aligned(a.B, 16) || a.lda % 8 || a.ldb % per16 || a.sbe % per16 || a.lda < 0 || a.ldb < 0) return false;

@@ -157,3 +157,19 @@ def test_experts_out_of_range_and_slots_without_a_token(ct, orc, form, bad):
     assert bool((C[lost] == 99.0).all()) and not bool((C[keep] == 99.0).all(1).any())
     if form == "plain":
         assert torch.equal(C[keep].cpu(), torch.from_numpy((ref * weights.reshape(-1, 1))[keep]).half())
+
+
+@pytest.mark.parametrize("switch,value", [("MI_MOE_DENSE_J", "2"), ("MI_MOE_DENSE_J", "4"), ("MI_MOE_DENSE_WIDE", "0"), ("MI_MOE_DENSE_STREAM", "0"),
+                                          ("MI_MOE_DENSE", "0"), ("MI_MOE_PREFILL", "0")])
+def test_a_forced_kernel_is_forced(ct, orc, monkeypatch, switch, value):
+    """The settings that force a kernel, or a shape of one, leave no launch to this one."""
+    A, B, _, tok, exp, w2d, weights, ref = _exact(orc, 64, 2, 4, 512, 256, torch.float16, False)
+    tok, exp = (x.cuda() for x in map(torch.from_numpy, orc.moe_align_tile_size(np.stack([[t % 4 + 1, (t + 1) % 4 + 1] for t in range(64)]).astype(np.int64), 128, 4)))
+    C = torch.empty(128, 256, dtype=torch.float16, device="cuda")
+    run = lambda: ct.fused_moe_kernel(A, B, C, w2d, tok, exp, 2, False, 128, 128, 64) or ct.last_variant()
+    assert run().startswith("fused_moe_few_")
+    want = C.clone()
+    monkeypatch.setenv(switch, value)
+    name = run()
+    assert name.startswith("fused_moe_t64_" if switch == "MI_MOE_DENSE" else "fused_moe_dense_"), name
+    assert torch.equal(C, want)
