@@ -239,17 +239,23 @@ namespace mi {
 namespace moe {
 
 // True where this kernel is the one to take; launches it.  `live`: tiles of 32 slots that hold tokens, about; with their strips of 64
-// rows they are the workgroups that do something.  Below 32 tokens per expert a weight row is read once, and (us of the whole call with
-// weights that come from memory, f16 and e4m3, 8 to 64 experts, 512 or 1024 hidden, 512 to 2048 inter, 3 or 16 tokens per expert)
-//  * the first projection runs on the streaming kernel's wide strips, which are ahead from about 700 workgroups on, as the ramp of a
-//    second round is: up to 512 of them -1.1 in the mean (-3.5 to +1.3), 1024 +2.1, 2048 and more +6 (16-bit weights of 1024 hidden in just 512: 31.4 : 34.4);
-//  * the second one (the launch that multiplies by the routed weights) runs there on 32- or 64-channel strips whose waves split K between
-//    two barriers: -1.8 in the mean (+1.8 to -9.8) but for 16-bit rows of 4 KB and more in 512 workgroups or more (32 experts, 1024 of 2048
-//    +4.5; 256 workgroups -1.1), whose eight rows of a transfer start in the same place of a page, and for as long ones in fewer than
-//    192 (8 experts, 128 workgroups: 12 and 18 tokens per expert +0.3 and +0.7, 30 of them -1.2).
+// rows they are the workgroups that do something (`work`).  Measured as whole calls of cutile_moe with weights that come from memory, this
+// kernel : the ones that take the launch otherwise, f16 and bf16 and e4m3, 500 shapes of 8 to 64 experts, 512 or 1024 hidden and 512 to 2048
+// inter and 340 of up to 256 experts, 7168 hidden and 4096 inter.  Below 32 tokens per expert a weight row is read once, and
+//  * the first projection runs otherwise on the streaming kernel's wide strips, which are ahead from about 700 workgroups on, as the ramp
+//    of a second round is: up to 512 of them -1.1 us in the mean (-3.5 to +1.3), 1024 +2.1, 2048 and more +6 (16-bit weights of 1024 hidden
+//    in just 512: 31.4 : 34.4, e4m3 of 7168 106 : 102);
+//  * the second one (the launch that multiplies by the routed weights) on 32- or 64-channel strips whose waves split K between two barriers:
+//    -1.8 us in the mean up to 1024 workgroups (1312 56 : 64 and 1536 80 : 83 with less than a token per expert), and behind from
+//    1800 on (2048 and more 1.02-1.17 of the call, 28672, 256 experts of 7168, 975 : 909).  Where its lines lie is measured and no more:
+//    16-bit rows of 4 KB pay from 192 to 511 workgroups (32 experts, 1024 of 2048, 512 of them +4.5; 256 -0.9 to -1.8; 8 experts, 128 of
+//    them, 12 and 18 tokens each +0.3 and +0.7), rows of 8 KB never (256 workgroups 75 : 70 and 97 : 91); e4m3 rows of 4 KB below 512 (64
+//    experts, 1024 of them, 172 : 157), of 2 KB where the other kernel runs on its 64-channel strips below 1024 (87 : 84).
 // From 32 tokens per expert on a strip is read once per 32 slots and not per 128: up to 450 workgroups with e4m3 weights, 352 with others (432
 // tokens top-2 of 16, K = 1408 e4m3 33 : 29, 224 top-2 of 8 35 : 28, 512 top-2 of 16, 320 workgroups, 46 : 37; but 256 top-4 of 32, 384
-// workgroups, K = 1024 and 1408 37.2 : 38.0 and 46.2 : 47.5, K = 512 and 2048 30.2 : 29.3 and 63.6 : 59.6; 283 top-4, 816, 93 : 103).
+// workgroups, K = 1024 and 1408 37.2 : 38.0 and 46.2 : 47.5, K = 512 and 2048 30.2 : 29.3 and 63.6 : 59.6; 283 top-4, 816, 93 : 103), 320 with
+// rows of 4 KB (8 experts, 70 to 75 tokens each, 336 and 352 workgroups 42.7 : 41).
+// With these lines no shape of the 500 takes more than 1.02 of what it took without this kernel, of the 340 none more than 1.025.
 // The line is the same for every epilogue of a projection, so fused and separate launches of a call add in the same order.  MI_MOE_FEW=0,
 // read at every call, and the settings that force another kernel or a shape of one (MI_MOE_DENSE*, MI_MOE_PREFILL) switch it off.
 bool few_launch(const DenseArgs& a, hipStream_t s) {
@@ -267,12 +273,14 @@ bool few_launch(const DenseArgs& a, hipStream_t s) {
     const bool once = a.total_tokens < 32ll * a.num_experts;
     const int64_t live = !once ? a.total_tokens / 32 + a.num_experts / 2 : a.total_tokens < a.num_experts ? a.total_tokens : a.num_experts;
     const int64_t work = live * strips;
+    const int64_t row = a.ldb * (a.w8 ? 1 : 2);   // bytes
     if (!once) {
-        if (work > (a.w8 ? 450 : 352)) return false;
+        if (work > (a.w8 ? 450 : row >= 4096 ? 320 : 352)) return false;
     } else if (!a.mul_routed_weight) {
-        if (work > (a.w8 ? 512 : 480)) return false;
-    } else if (!a.w8 && a.ldb * 2 >= 4096 && (work >= 512 || work < 192)) {
-        return false;
+        if (work > (a.w8 && row < 4096 ? 512 : 480)) return false;
+    } else {
+        if (work > 1280 || (row >= 4096 && work >= 512)) return false;
+        if (a.w8 ? row >= 2048 && a.K % 256 == 0 && work >= 1024 : row >= 8192 || (row >= 4096 && work < 192)) return false;
     }
 #define LAUNCH(ET, MODE)                                                                                                                     \
     do {                                                                                                                                     \

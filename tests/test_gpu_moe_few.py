@@ -49,11 +49,33 @@ def test_few_tokens_per_expert(ct, orc, make, e4m3):
     check(J(want), ref, 5e-2 if d.hidden_states.dtype == torch.bfloat16 else 2e-2)
 
 
+@pytest.mark.parametrize("K,N,routed,few", [
+    (256, 20480, True, True), (256, 20544, True, False), (2048, 16320, True, True), (2048, 16384, True, False), (2064, 16384, True, True),
+    (4096, 8128, True, True), (4096, 8192, True, False), (4096, 1024, True, True), (512, 8192, False, True), (4096, 7680, False, True), (4096, 8192, False, False),
+])
+def test_which_launches_of_e4m3_weights_the_rule_takes(ct, orc, K, N, routed, few):
+    """Rows of 2 KB below 1024 workgroups, unless the other kernel has no 64-channel strips for their K; of 4 KB below 512; 1280 at most."""
+    E, tokens = 4, 16
+    rng = np.random.default_rng(K + N)
+    tok, exp = orc.moe_align_tile_size(np.arange(tokens, dtype=np.int64)[:, None] % E + 1, 32, E)
+    A = torch.from_numpy(rng.integers(-2, 3, (tokens, K)).astype(np.float16)).cuda()
+    W = torch.randint(-1, 2, (E, N, K), dtype=torch.int8, generator=torch.Generator().manual_seed(K)).cuda().half()
+    C = torch.empty(tokens, N, dtype=torch.float16, device="cuda")
+    ct.fused_moe_kernel(A, W.to(torch.float8_e4m3fn), C, torch.ones(tokens, dtype=torch.float16, device="cuda"), torch.from_numpy(tok).cuda(),
+                        torch.from_numpy(exp).cuda(), 1, routed, 32, 128, 64, b_scale=torch.ones(E, N, device="cuda"))
+    assert ct.last_variant().startswith("fused_moe_few_") == few, ct.last_variant()
+    # (integers below 2^11, so f16 holds them and fp32 sums are exact)
+    assert torch.equal(C.float(), torch.stack([W[t % E].float() @ A[t].float() for t in range(tokens)]))
+
+
 @pytest.mark.parametrize("tokens,E,K,N,off,routed,few", [
     (31, 1, 256, 256, 0, False, True), (16, 4, 256, 7680, 0, False, True), (16, 4, 256, 7744, 0, False, False),    # first projection: 480 workgroups
     (16, 4, 256, 8256, 0, True, True), (16, 4, 2048, 8192, 0, True, False), (16, 4, 2040, 8192, 0, True, True),    # second: rows of 4 KB from 512 on
     (16, 4, 2048, 8064, 0, True, True),
     (16, 4, 2048, 3008, 0, True, False), (16, 4, 2048, 3072, 0, True, True),                                        # and from 192 on
+    (16, 4, 4096, 3072, 0, True, False), (16, 4, 4088, 3072, 0, True, True),                                        # of 8 KB never
+    (16, 4, 256, 20480, 0, True, True), (16, 4, 256, 20544, 0, True, False),                                        # 1280 workgroups
+    (128, 4, 2048, 3392, 0, False, True), (128, 4, 2048, 3456, 0, False, False),                                    # 32 per expert, rows of 4 KB: 320
     (128, 4, 512, 3712, 0, False, True), (128, 4, 512, 3776, 0, False, False), (128, 4, 512, 3776, 0, True, False),  # 32 per expert: 352 workgroups
     (16, 4, 248, 256, 0, False, False), (16, 4, 260, 256, 0, False, False), (16, 4, 256, 256, 4, False, False),    # K below 256, off the chunks; rows off 16 bytes
 ])
