@@ -1,6 +1,6 @@
 // Small f16/bf16 GEMM: C(M,N) = A(M,K) * B(K,N), column-major, fp32 accumulate, for products of up to 128 tiles of 128 x 128.
 //
-// What bounds a product that leaves most CUs idle is what one CU bstagess into its LDS, about 95 GB/s: a K step of 32 of a
+// What bounds a product that leaves most CUs idle is what one CU brings into its LDS, about 95 GB/s: a K step of 32 of a
 // 128 x 128 tile is 16 KB, the 0.18 us that it takes on gemm_big.hip's kernel.  So the tiles here are as small as it takes to
 // give every CU one -- 32 x 32, 64 x 32, 64 x 64 or 128 x 64, whichever small_estimate says is through first -- and the
 // four waves of a workgroup do not share a tile's extent but its K: wave w takes the stages w, w + 4, ... of 64 k, with an LDS

@@ -60,7 +60,10 @@ def test_few_tiles_batched_exact(ct, orc, M, N, K, nb):
 
 
 @pytest.mark.parametrize("M,N,K,small", [(512, 512, 255, False), (512, 512, 256, True), (256, 256, 4096, True), (256, 256, 4104, False),
-                                         (2048, 1024, 320, False), (2049, 1024, 2048, False), (1536, 735, 576, True), (1664, 1792, 832, False)])
+                                         (2048, 1024, 320, False), (2049, 1024, 2048, False), (1536, 735, 576, True), (1664, 1792, 832, False),
+                                         # estimated close to the other kernels: 128 x 64 tiles, and against a split
+                                         (512, 3584, 1216, False), (832, 2240, 1280, False), (2816, 384, 2191, False), (1397, 727, 3136, False),
+                                         (512, 1443, 3043, True)])
 def test_both_sides_of_the_rule(ct, orc, M, N, K, small):
     A, B, ref = _operands(orc, M, N, K, torch.float16, (0, 0))
     C = torch.empty((N, M), dtype=torch.float32, device="cuda")
