@@ -89,7 +89,8 @@ def test_few_tiles_infinities_and_nan_stay_in_their_rows_and_columns(ct, orc):
     (128, 100, 1024, 2, (0, 0), "small_32x32x32"), (101, 63, 1023, 3, (0, 0), "small_32x32x32"),
     (720, 128, 500, 3, (0, 0), "small_64x32x32"), (249, 181, 384, 8, (0, 0), "small_64x32x32"), (629, 141, 143, 9, (2, 3), "small_64x32x32"),
     # the tiles of gemm32_big.hip where they are estimated to be the quicker ones
-    (832, 384, 489, 12, (0, 0), "big_"), (320, 2007, 160, 10, (0, 0), "big_64x64x16_ring4"), (2056, 2311, 388, 1, (0, 0), "big_64x64x16_ring4"),
+    (832, 384, 489, 12, (0, 0), "big_"), (765, 256, 384, 8, (0, 0), "big_64x64x16_ring4"), (192, 1283, 383, 6, (0, 0), "big_64x64x16_ring4"),
+    (576, 201, 384, 12, (0, 0), "big_64x64x16_ring4"), (320, 2007, 160, 10, (0, 0), "big_64x64x16_ring4"), (2056, 2311, 388, 1, (0, 0), "big_64x64x16_ring4"),
 ])
 def test_few_fp32_tiles_exact(ct, orc, M, N, K, nb, pad, kernel):
     A, B, ref = _operands(orc, M, N, K, torch.float32, pad, nb)
