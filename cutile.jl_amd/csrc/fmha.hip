@@ -940,25 +940,34 @@ bool pick_inside(int64_t wgs, int64_t rows, int D, int Sq, int Skv, bool causal,
 }
 
 // Launches of few queries (fmha_few.hip) where that kernel is estimated to be through first; launched and true.  `other`: the kernel
-// that takes the launch otherwise.  Estimates in us: a launch, the longest walk and what each SIMD has to do, fitted for every kernel to
-// the shapes that it takes (batches of 1 to 8 with 4 to 32 heads, 256 to 4096 queries; standard deviation 4 to 11 %).  Heads of 64 with
-// another number of keys than queries count as the pipelined kernel's, which is quicker than what they have.  Of 198 shapes with heads of
-// 64 and up to 120 halves per SIMD 150 are taken, at 0.75 of the time in the mean, of 237 with heads of 128 125, at 0.71; 33 more would gain
-// 4 to 15 %.  Not causal against the pipelined kernel for heads of 128 the estimate is 10 to 20 % short: 0.8.
-enum FewOther { PIPE64, PLAIN128, KEYS2, SPLITKV, PIPE128 };
-bool few_instead(const fmha::Problem& p, FewOther other, hipStream_t s) {
+// that takes the launch otherwise, `parts`: in how many parts it would split the keys.  Estimates in us: a launch, the longest walk and what
+// each SIMD has to do, fitted for every kernel to the shapes that it takes (batches of 1 to 16 with 1 to 64 heads, 65 to 4096 queries, 32 to
+// 5120 keys; standard deviation 4 to 11 %).  Of 8400 such shapes that are taken 17 take 1.02 to 1.10 of the other kernel's time and one 1.25
+// (16 x 16 heads of 64, 104 of 1493 keys); the mean is 0.72 with as many keys as queries and 0.73 with others.  Where an estimate is least sure the
+// kernel has to promise more: launches of 7 to 10 us on the kernels that walk the keys alone (128: 16 x 16 heads, S = 113, 8.1 : 8.6; 64: 4 x 64, 331
+// of 41 keys 9.3 : 10.0), and against the pipelined kernel for heads of 128 launches that are not causal (10 to 20 % short) or are with another
+// number of keys, whose walks are mostly of one length (1 x 32 heads, 1943 of 555 keys 26.5 : 32.4).
+enum FewOther { PIPE64, SPLIT64, PLAIN64, PLAIN128, KEYS2, SPLITKV, PIPE128 };
+bool few_instead(const fmha::Problem& p, FewOther other, int parts, hipStream_t s) {
     const fmha::Walks w = fmha::walks_of(p);
+    const int64_t Sq = p.Q->sizes[1], rows = Sq * p.Q->sizes[2] * p.Q->sizes[3];
+    const bool d64 = p.Q->sizes[0] == 64, same = Sq == p.K->sizes[1];
     // (no further than what was measured; the pipelined kernel for heads of 64 is level from about 60 halves per SIMD on: 1 x 32 heads,
-    // S = 2565 causal, 104 of them, 44 : 49)
-    if (w.longest > 160 || w.halves > (other == PIPE64 ? 60 : 120)) return false;
-    const bool ragged = p.Q->sizes[1] % 128 != 0;
+    // S = 2565 causal, 104 of them, 44 : 49; many tiles that walk three or four halves each, 4 x 8 heads of 64, 3536 of 98 keys, 13.6 : 14.5; keys
+    // and values that stay in no cache from one tile of a head to the next, 16 x 8 heads of 128, 93 of 3283 keys, 215 MB, 62 : 75)
+    const int64_t kv_bytes = 4 * p.K->sizes[0] * p.K->sizes[1] * p.K->sizes[2] * p.K->sizes[3];
+    if (w.longest > 160 || w.halves > (d64 ? 60 : 120) || (other == PLAIN64 && w.tiles > 2.5) || kv_bytes > (192ll << 20)) return false;
+    const bool ragged = Sq % 128 != 0;
     const double us = other == PIPE64     ? (ragged ? 6.53 + 0.191 * w.longest + 0.297 * w.halves : 5.48 + 0.209 * w.longest + 0.272 * w.halves)
+                      : other == SPLIT64  ? 11.6 + 0.93 * ceil(w.longest / 2) / parts + 1.14e-4 * (double)rows * parts + 0.29 * w.halves
+                      : other == PLAIN64  ? 5.0 + 0.557 * w.longest + 0.427 * w.halves + 0.35 * w.tiles
                       : other == PLAIN128 ? 8.69 + 0.131 * w.longest + 0.594 * w.halves
                       : other == KEYS2    ? 7.46 + 0.413 * w.longest + 0.180 * w.halves
                       : other == SPLITKV  ? fmin(13.8 + 0.109 * w.longest + 0.774 * w.halves, 14.0 + 1.16 * w.halves)   // (few workgroups: 1 x 8, 136 of 2396 keys 18.1)
                                           : 13.8 + 0.346 * w.longest + 0.369 * w.halves;
+    const double margin = other == PLAIN64 ? 0.81 : other == PLAIN128 ? 0.84 : other != PIPE128 ? 0.92 : !p.causal ? 0.8 : same ? 0.92 : 0.7;
     int waves = 0;
-    if (fmha::few_estimate(p, w, &waves) > us * (other == PIPE128 && !p.causal ? 0.8 : 0.92)) return false;
+    if (fmha::few_estimate(p, w, &waves) > us * margin) return false;
     fmha::few_launch(p, waves, s);
     return true;
 }
@@ -1127,21 +1136,24 @@ extern "C" int mi_fmha_kernel(const mi_tile_array* Q, const mi_tile_array* K, co
         fmha::Problem pr{Q, K, V, Out, H, QUERY_GROUP_SIZE, scale2, input_pos, causal, dt == MI_BF16};
         static const bool split_forced = getenv("MI_FMHA_SPLIT") != nullptr;
         const bool may_few = !e && !split_forced && fmha::few_applicable(pr);
-        if (D == 64 && may_few && few_instead(pr, PIPE64, s)) return launch_status();
+        const int64_t wgs = cld(Sq, (int64_t)kQB) * B * H;
+        if (D == 64 && may_few) {
+            const int parts = pick_parts(wgs, B * H * Sq, 64, (int)Sq, (int)Skv, causal, input_pos);
+            if (few_instead(pr, fmha::pipe_applicable(pr) ? PIPE64 : parts ? SPLIT64 : PLAIN64, parts, s)) return launch_status();
+        }
         if (!no_pipe && fmha::pipe_applicable(pr)) {
             fmha::pipe_launch(pr, s);
             return launch_status();
         }
         if (!no_pipe && fmha::pipe128_applicable(pr)) {
-            const int64_t wgs = cld(Sq, (int64_t)kQB) * B * H;
             const int parts = pick_parts(wgs, B * H * Sq, 128, (int)Sq, (int)Skv, causal, input_pos);
             // (Strides of 2^24 elements and more are not for two groups of waves.  Launches that are not causal and have another number
             // of keys than queries stay on the pipelined kernel, the slower of the two there: 1 x 32 heads, 954 queries of 1787 keys 53 us, 39
             // with two groups; 0.70-0.80 of the time on 24 shapes.)
-            const bool inside = (causal || Sq == Skv) && K->strides[1] < (1 << 24) && V->strides[1] < (1 << 24) &&
-                                pick_inside(wgs, B * H * Sq, 128, (int)Sq, (int)Skv, causal, input_pos, scale2, parts);
+            const bool two = pick_inside(wgs, B * H * Sq, 128, (int)Sq, (int)Skv, causal, input_pos, scale2, parts);
+            const bool inside = two && (causal || Sq == Skv) && K->strides[1] < (1 << 24) && V->strides[1] < (1 << 24);
             const bool pipe = (e && strcmp(e, "pipe") == 0) || (!inside && fmha::pipe128_pays(pr, parts));
-            if (may_few && few_instead(pr, inside ? KEYS2 : pipe ? PIPE128 : parts ? SPLITKV : PLAIN128, s)) return launch_status();
+            if (may_few && few_instead(pr, pipe ? PIPE128 : two ? KEYS2 : parts ? SPLITKV : PLAIN128, parts, s)) return launch_status();
             if (pipe) {
                 fmha::pipe128_launch(pr, s);
                 return launch_status();

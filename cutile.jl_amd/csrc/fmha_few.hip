@@ -316,8 +316,8 @@ double few_estimate(const Problem& p, const Walks& w, int* waves) {
     const double rounds = w.tiles * (*waves == 4 ? 2.0 : 1.0);
     const double tail = d64 || p.causal || rounds <= 1.0 ? 1.0 : 1.0 + 0.45 * (ceil(rounds) / rounds - 1.0);
     // A half of a wave's walk takes 0.8 us by itself, from its request to its products (1 x 8 heads, 136 of 2396 keys 19.7, 4 x 4, 134 of 1384 13.7,
-    // 1 x 4, 160 of 637 8.5).
-    const double alone = d64 ? 0.0 : 4.0 + 0.8 * (*waves == 4 ? c4 : c2);
+    // 1 x 4, 160 of 637 8.5), with heads of 64 0.55 (1 x 1 to 1 x 16, 65 to 512 of 3300 keys 17, 4000 20, 5120 24: a split takes 15 to 17 there).
+    const double alone = (d64 ? 2.2 : 4.0) + (d64 ? 0.545 : 0.8) * (*waves == 4 ? c4 : c2);
     return fmax(tail * (*waves == 4 ? t4 : t2), alone);
 }
 

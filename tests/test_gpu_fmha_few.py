@@ -73,7 +73,11 @@ def test_few_queries_is_no_further_off_than_the_kernels_it_replaces(ct, monkeypa
 
 
 @pytest.mark.parametrize("dim,B,H,sq,skv,few", [
-    (64, 1, 4, 64, 640, False), (64, 1, 4, 65, 640, True), (64, 1, 1, 128, 5120, True), (64, 1, 1, 128, 5121, False),
+    (64, 1, 4, 64, 640, False), (64, 1, 4, 65, 640, True), (64, 1, 16, 512, 5120, True), (64, 1, 16, 512, 5121, False),
+    # the walk of a wave by itself against a split (5120 keys 23.9 us : 15.6, 2700 14.2 : 17.5), and the kernels that walk few keys
+    (64, 1, 1, 128, 5120, False), (64, 1, 1, 128, 2700, True), (64, 4, 64, 331, 41, False), (128, 2, 8, 2375, 57, False),
+    # not causal with other keys: two groups of waves, 59 us : 70
+    (128, 1, 32, 838, 3111, False),
     (128, 1, 1, 128, 5121, False), (64, 8, 32, 1024, 1024, False), (128, 4, 32, 1024, 1024, False), (128, 1, 32, 1280, 1280, False),
     # walks of one length: 512 workgroups are one round, 576 leave a nearly empty second one
     (128, 1, 8, 2048, 1619, True), (128, 1, 8, 2282, 1619, False), (128, 1, 8, 136, 2396, False), (128, 1, 8, 136, 1000, True),
@@ -84,6 +88,16 @@ def test_both_sides_of_the_rule(ct, dim, B, H, sq, skv, few):
     got = fmha.cutile_fmha(Q, K, V, causal=False)
     assert ct.last_variant().startswith("fmha_few") == few, ct.last_variant()
     assert _err(got[:1, :4], _reference(Q[:1, :4], K[:1, :4], V[:1, :4], 0, False)) <= 2**-10
+
+
+@pytest.mark.parametrize("B,H,sq,skv,pos,few", [(1, 32, 1943, 555, 0, False), (16, 8, 268, 1612, 1344, False), (2, 4, 300, 555, 255, True)])
+def test_both_sides_of_the_rule_causal_with_other_keys(ct, B, H, sq, skv, pos, few):
+    """Heads of 128: walks of one length, which the pipelined kernel is ahead on."""
+    g = torch.Generator(device="cuda").manual_seed(sq + skv)
+    Q, K, V = (torch.empty(B, H, s, 128, device="cuda", dtype=torch.float16).normal_(0, 1, generator=g) for s in (sq, skv, skv))
+    got = fmha.cutile_fmha(Q, K, V, input_pos=pos, causal=True)
+    assert ct.last_variant().startswith("fmha_few" if few else "fmha_pipe_d128"), ct.last_variant()
+    assert _err(got[:1, :4], _reference(Q[:1, :4], K[:1, :4], V[:1, :4], pos, True)) <= 2**-10
 
 
 @pytest.mark.parametrize("dim", [64, 128])
