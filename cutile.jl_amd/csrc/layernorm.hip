@@ -456,7 +456,7 @@ __global__ __launch_bounds__(BLOCK) void ln_bwd_kernel(float* __restrict__ DX, i
     }
 }
 
-// Backward with RG row groups of BLOCK lanes per workgroup (rows of up to 8192 elements, 16-byte aligned): the groups walk
+// Backward with RG row groups of BLOCK lanes per workgroup (rows of 4 to 8192 elements; ALIGNED: a multiple of four, on 16 bytes): the groups walk
 // different rows of the same partial slot and add their dW / dB partials in LDS before the flush, which divides the number
 // of memory-side float atomics -- the scarce resource of this kernel -- by RG at the same number of rows in flight.
 // Workgroup (g, s): group h handles rows m = g + G*(RG*s + h), stepping by RG*G*S.
@@ -1033,8 +1033,8 @@ constexpr int kMaxRegsN = 256 * 16 * 4;
 
 // Persistent look-ahead forward: used when every workgroup gets at least two rows.  Rows off 16 bytes as well: against the
 // element-by-element one-row kernels, fwd alone, 200000 x 283 127 -> 113 us, 60000 x 1001 100 -> 95, 16000 x 5001 157 -> 133;
-// a workgroup of 1024 lanes has to walk some rows to gain there (1024 x 8195 23.3 -> 28.6, 2000 x 8195 46.1 -> 47.3, 4000 x 10001
-// 93 -> 88, 4000 x 16381 138 -> 117), so such rows take it from seven on.
+// a workgroup of 1024 lanes, whose 128 registers a lane do not hold both rows (17 spilled; 13 on rows of 16 bytes), has to walk some to gain there
+// (1024 x 8195 23.3 -> 28.6, 2000 x 8195 46.1 -> 47.3, 4000 x 10001 93 -> 88, 4000 x 16381 138 -> 117), so such rows take it from seven on.
 template <bool AL, bool ST>
 bool launch_fwd_pipe(int vecs, hipStream_t s, const float* X, int64_t ldx, const float* W, const float* B,
                      float* Y, int64_t ldy, float* Mean, float* Rstd, float eps, int N, int64_t M) {
@@ -1232,18 +1232,25 @@ extern "C" int mi_layer_norm_bwd_dx_partial_dwdb(
         // Up to 1024 elements a group is a single wave (no barriers in the walk) and eight groups share a workgroup, at most
         // one per CU, with at least four rows a wave up to 512 elements (64 slots, us, 256 lanes -> a wave: 1024 x 1024 6.8 -> 5.2,
         // 4096 x 1024 12.6 -> 11.0, 4096 x 700 11.8 -> 9.7; with one or two rows a slot 0.1-0.4 us slower, 4 x 1024 3.8 -> 4.1).
-        // Streamed inputs of more than 512 elements keep 256 lanes (where the two meet, 16384 x 1024, 38.2 and 39.3).
+        // Streamed inputs of more than 512 elements keep 256 lanes (where the two meet, 16384 x 1024, 38.2 and 39.3) where their rows are
+        // on 16 bytes; rows off them, whose loads are not streamed, take a wave from five rows a slot on (256 lanes : a wave, 96 x 783,
+        // 64 slots, 4.4 : 5.9, 115 x 545, 32 slots, 5.0 : 5.9; 24 x 819, 4 slots, 5.9 : 5.9, 128 x 657, 16 slots, 6.7 : 6.2, 16184 x 591, 256
+        // slots, 32 : 24, 30843 x 861 65 : 59).  Against the kernels of one row per workgroup, which had them before, rows off 16 bytes take
+        // 0.74 of the time in the mean of 630 shapes; 4097 to 8192 elements with few rows 0.85 to 1.06 (288 x 7037, 32 slots, 13.9 : 14.8).
         // A slot that one workgroup owns gets plain adds, and the same bits on every run; two add to a zero slot in either
         // order with the same result; from three on the order of arrival decides the last bits.  One row a wave is
         // quicker on many slots (64 slots, 2000 x 512 6.1 -> 5.6 us), but puts more workgroups on slots that have one or two now,
         // and costs more than it gives on few slots (1 slot, 2000 x 400 7.1 -> 9.6); two rows a group above 1024 elements likewise.
-        const bool one_wave = vecs <= 128 || (vecs <= 256 && (al ? !stream_in : rows_per_slot > 1));
+        const bool one_wave = vecs <= 128 || (vecs <= 256 && (al ? !stream_in : rows_per_slot > 4));
         const int rg = one_wave ? 8 : vecs <= 1024 ? 2 : 1;
         if (!getenv("MI_LN_BWD_SPLITS")) {
             const int64_t per_cu = cld((int64_t)256, (int64_t)G);
             if (vecs <= 128) S = std::min(cld((int64_t)2048, (int64_t)G), cld(rows_per_slot, (int64_t)4));
             else if (one_wave) S = 8 * std::min(per_cu, cld(rows_per_slot, (int64_t)8));
             else if (vecs > 1024) S = std::max((int64_t)1, std::min(per_cu, cld(rows_per_slot, (int64_t)4)));
+            // (rows off 16 bytes, five to eight a slot: a group has two rows and not four, us 320 x 1314, 64 slots, 7.3 -> 5.7, 112 x 1717, 16
+            // slots, 8.2 -> 5.6, 224 x 3661, 32 slots, 12.2 -> 8.7; more than 128 slots fill the CUs with one workgroup each, 1149 x 1103, 256
+            // slots, 8.0 : 8.1)
             else if (!al && vecs > 256 && S == 2 && G <= 128) S = 4;
         }
         const int S2 = (int)cld(S, (int64_t)rg);

@@ -75,3 +75,15 @@ def test_rows_of_any_length_and_alignment(ct, M, N, G, pad, off):
     close(DB, torch.zeros(G, N, dtype=torch.float64).index_add_(0, slot, dy), "partial db")
     assert untouched(yb, Y, 7.0) and untouched(dxb, DX, 7.0) and untouched(DWb, DW, 0.0) and untouched(DBb, DB, 0.0)
     assert untouched(xb, X, nan) and untouched(dyb, DY, nan)
+
+
+@pytest.mark.parametrize("M,N,G,kernel", [(256, 1001, 64, "v1_rg2"), (257, 1001, 64, "v4_rg8"), (8, 513, 4, "v1_rg2"), (17, 1023, 4, "v4_rg8"),
+                                          (256, 511, 64, "v2_rg8"), (400, 1025, 64, "v2_rg2")])
+def test_which_groups_walk_rows_off_16_bytes(ct, M, N, G, kernel):
+    """513 to 1024 elements: a wave per group from five rows a slot on."""
+    X, DY, DX = (torch.randn(M, N, device="cuda") for _ in range(3))
+    W, mean, rstd = torch.randn(N, device="cuda"), X.mean(1), 1 / X.std(1)
+    dw, db = torch.zeros(2, G, N, device="cuda")
+    ct.layer_norm_bwd_dx_partial_dwdb(DX, DY, dw, db, X, W, mean, rstd, torch.zeros(G, dtype=torch.int64, device="cuda"), G, 1024)
+    assert ct.last_variant() == "ln_bwd_regs_b512_" + kernel, ct.last_variant()
+    close(db.sum(0), DY.double().sum(0), "db")
