@@ -64,7 +64,6 @@ using namespace mi::fmha;
 
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kQB = 128;  // queries per workgroup
 constexpr int kKV = 64;   // keys per LDS tile
@@ -970,10 +969,6 @@ bool few_instead(const fmha::Problem& p, FewOther other, int parts, hipStream_t 
     if (fmha::few_estimate(p, w, &waves) > us * margin) return false;
     fmha::few_launch(p, waves, s);
     return true;
-}
-
-bool vec16(const mi_tile_array* a) {
-    return aligned(a->ptr, 16) && a->strides[1] % 8 == 0 && a->strides[2] % 8 == 0 && a->strides[3] % 8 == 0;
 }
 
 template <typename E, int D>

@@ -11,6 +11,7 @@ typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 #define LDS_PTR(T, p) ((T __attribute__((address_space(3)))*)(p))
@@ -55,6 +56,11 @@ struct BF16 {
         return r;
     }
 };
+
+// Rows of an array that the kernels read and write in pieces of 16 bytes.
+inline bool vec16(const mi_tile_array* a) {
+    return aligned(a->ptr, 16) && a->strides[1] % 8 == 0 && a->strides[2] % 8 == 0 && a->strides[3] % 8 == 0;
+}
 
 struct Strides {
     int64_t s1, s2, s3;  // element strides of dims 1..3 (dim 0 is contiguous)

@@ -22,6 +22,7 @@
 // 28 -> 18, 2 x 8, 2688 not causal 69 -> 52; heads of 128 4 x 4, 512 causal 15.0 -> 7.6, 1 x 4, 3328 47 -> 27, 3 x 4, 1408 28.8 -> 16.4, 1 x 8, 3520
 // 60 -> 42, 6 x 8, 817 28.8 -> 20.7.
 #include "fmha_common.h"
+#include "lds_transfer.h"
 
 namespace mi {
 namespace fmha {
@@ -29,14 +30,6 @@ namespace {
 
 constexpr int kHK = 32;   // keys per half
 constexpr int kQT = 32;   // queries per workgroup
-
-// One 1 KB transfer, 16 bytes per lane: to LDS byte address `lds` from sbase + voff / from a lane's own address.
-__device__ __forceinline__ void load_lds(unsigned lds, unsigned voff, const char* sbase) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds), "v"(voff), "s"(sbase) : "m0", "memory");
-}
-__device__ __forceinline__ void load_lds_at(unsigned lds, const char* p) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds), "v"(p) : "m0", "memory");
-}
 
 template <typename E, int D, bool CAUSAL, int NW>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(D == 64 ? 4 : 2))) void fmha_few_kernel(
@@ -226,7 +219,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(D == 64
         sum += mw == -INFINITY ? 0.f : s_l[w][lane & 31] * __builtin_amdgcn_exp2f(mw - most);
     }
     const float f = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - most);
-    typedef float f32x4 __attribute__((ext_vector_type(4)));
     char* const mine = (char*)areas + wave * (AREA * 2);
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
@@ -271,10 +263,6 @@ void launch_t(const Problem& p, hipStream_t stream) {
     else
         hipLaunchKernelGGL((fmha_few_kernel<E, D, false, NW>), grid, blk, 0, stream, (const unsigned short*)Q->ptr, qs, (const unsigned short*)K->ptr, ks,
                            (const unsigned short*)V->ptr, vs, (unsigned short*)O->ptr, os, Sq, Skv, p.H, p.group, p.scale2, p.input_pos, nqt, nbh);
-}
-
-bool vec16(const mi_tile_array* a) {
-    return ((uintptr_t)a->ptr % 16) == 0 && a->strides[1] % 8 == 0 && a->strides[2] % 8 == 0 && a->strides[3] % 8 == 0;
 }
 
 }  // namespace

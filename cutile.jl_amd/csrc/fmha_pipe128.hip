@@ -471,10 +471,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(1, 1)))
     }
 }
 
-bool vec16(const mi_tile_array* a) {
-    return ((uintptr_t)a->ptr % 16) == 0 && a->strides[1] % 8 == 0 && a->strides[2] % 8 == 0 && a->strides[3] % 8 == 0;
-}
-
 template <typename E>
 void launch_e(const Problem& p, hipStream_t stream) {
     const mi_tile_array *Q = p.Q, *K = p.K, *V = p.V, *O = p.O;

@@ -2,22 +2,12 @@
 // gemm32_small.hip: fp32, moe_few.hip: grouped).
 #pragma once
 #include "gemm_direct.h"
+#include "lds_transfer.h"
 
 namespace mi {
 namespace gemm {
 
 constexpr int kSplitWaves = 4;
-
-#pragma clang diagnostic ignored "-Winline-asm"  // m0 is named as clobbered on purpose
-
-// One 1 KB transfer, 16 bytes per lane: to LDS byte address `lds` from sbase + voff / from a lane's own address.  (Inline
-// assembly, so that the compiler does not tie reads of one stage to transfers into another; the waits are counted by hand.)
-__device__ __forceinline__ void load_lds(unsigned lds, unsigned voff, const char* sbase) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds), "v"(voff), "s"(sbase) : "m0", "memory");
-}
-__device__ __forceinline__ void load_lds_at(unsigned lds, const char* p) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds), "v"(p) : "m0", "memory");
-}
 
 // The four waves' sums of a (32*I) x (32*J) tile, added through the LDS in the order of the waves; a wave stores a quarter of
 // the tile, at (m0, n0) of C.  `areas`: one of AREA bytes per wave, at least 4096 * I * J, whose wave is done with it.

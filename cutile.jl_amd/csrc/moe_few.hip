@@ -39,8 +39,8 @@ template <typename E, int MODE, bool W8>
 __global__ __launch_bounds__(64 * NW) void moe_few_kernel(const DenseArgs a, int strips, int blocks) {
     constexpr int STAGE_T = kTS * BK * 2, STAGE_W = kTW * BK * (W8 ? 1 : 2), AREA = STAGE_T + STAGE_W;   // bytes
     constexpr int TT = STAGE_T / 1024, TW = STAGE_W / 1024;                                             // transfers per stage
-    __shared__ __attribute__((aligned(1024))) char areas[NW * (AREA > 8192 ? AREA : 8192)];             // a wave's stage, and later its sums (8 KB)
-    constexpr int STEP = AREA > 8192 ? AREA : 8192;
+    static_assert(AREA >= 8192, "a wave's sums fit its area");
+    __shared__ __attribute__((aligned(1024))) char areas[NW * AREA];                                    // a wave's stage, and later its sums
     const int lane = threadIdx.x & 63, hb = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // Workgroup -> 32-slot tile and strip: the first tile of every block, then the second of every block, ... (those of a block behind
@@ -83,7 +83,7 @@ __global__ __launch_bounds__(64 * NW) void moe_few_kernel(const DenseArgs a, int
         }
         pW[t] = W8 ? Bx + (int64_t)row * a.ldb + 16 * cW : Bx + ((int64_t)row * a.ldb + 8 * cT[t & 1]) * 2;
     }
-    const unsigned lds0 = (unsigned)(size_t)LDS_PTR(char, areas) + wave * STEP;
+    const unsigned lds0 = (unsigned)(size_t)LDS_PTR(char, areas) + wave * AREA;
     const int nk = (a.K + BK - 1) / BK;
     auto issue = [&](int c) __attribute__((always_inline)) {
         const int64_t ko = (int64_t)c * BK;
@@ -112,7 +112,7 @@ __global__ __launch_bounds__(64 * NW) void moe_few_kernel(const DenseArgs a, int
         fw[u] = W8 ? STAGE_T + row * BK + 16 * (u ^ ((row >> 2) & 3)) + 8 * hb : STAGE_T + ft[u];
     }
     f32x16 acc[2] = {f32x16{0}, f32x16{0}};
-    const char* const S = areas + wave * STEP;
+    const char* const S = areas + wave * AREA;
     for (int c = wave; c < nk; c += NW) {
         wait_vm<0>();
         s16x8 t[4], w[4][2];
@@ -141,20 +141,19 @@ __global__ __launch_bounds__(64 * NW) void moe_few_kernel(const DenseArgs a, int
     }
 
     // ---- the waves' sums, added in their order; wave q takes register group q of both tiles -------------------------------------
-    char* const mine = areas + wave * STEP;
+    char* const mine = areas + wave * AREA;
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int q = 0; q < 4; ++q)
             *reinterpret_cast<f32x4*>(mine + ((4 * j + q) * 64 + lane) * 16) = f32x4{acc[j][4 * q], acc[j][4 * q + 1], acc[j][4 * q + 2], acc[j][4 * q + 3]};
     __syncthreads();
-    if (wave >= 4) return;
     f32x4 v[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         v[j] = *reinterpret_cast<const f32x4*>(areas + ((4 * j + wave) * 64 + lane) * 16);
 #pragma unroll
-        for (int x = 1; x < NW; ++x) v[j] += *reinterpret_cast<const f32x4*>(areas + x * STEP + ((4 * j + wave) * 64 + lane) * 16);
+        for (int x = 1; x < NW; ++x) v[j] += *reinterpret_cast<const f32x4*>(areas + x * AREA + ((4 * j + wave) * 64 + lane) * 16);
     }
     auto weight_of = [&](int tk) {
         float wt = 1.f;
