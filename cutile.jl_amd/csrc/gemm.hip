@@ -428,6 +428,7 @@ bool edge_split(const Problem& p, hipStream_t s, int* status) {
             (void)pick_direct_tile(q, &c);
             return c * 1.37 * ks;
         }
+        // (by rounds, as big32_launch chooses for it: a main part has at least 3456 tiles of 64 x 64, and small32_try chooses up to 2048)
         return big32_cost(q) * 59.0 * ks;
     };
     // a strip of r rows or columns by itself (us): f16 splits it over K (two launches; with K off the chunks its rows are

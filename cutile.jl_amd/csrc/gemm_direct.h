@@ -97,7 +97,7 @@ __device__ __forceinline__ void store_tile(const f32x16 (&acc)[I][J], OutT* C, i
 // Whether a product's results are stored past the L2.  The 32 lanes of a half-wave store 64 or 128 bytes of a column of C: whole
 // segments where every column starts on a 64-byte boundary.  Off them a store ends inside a segment that the next one goes on
 // with; streamed, each piece went to memory by itself, while ordinary stores meet in the L2 (us, streamed : ordinary, f16 3241 x 1985
-// x 1723 to fp32 45.1 : 35.5, 2723 x 2496 x 704 25.2 : 20.9, 4095^3 151 : 140, bf16 2999 x 2100 x 3001 58.8 : 55.3, fp32 8 x 1021 x
+// x 1723 to fp32 45.1 : 35.5, 2723 x 2496 x 704 25.2 : 20.9, 4095^3 151 : 140, bf16 2999 x 2100 x 3001 57.2 : 55.1, fp32 8 x 1021 x
 // 2047 x 509 171 : 140).  On them the streamed ones are ahead (f16 1024 x 3072 x 961 to fp32 11.8 : 12.6, 320 x 1344 x 2944 13.4 : 14.4).
 // A template parameter: with both kinds in one kernel the branches are made one, of ordinary stores, or the code is half as long again.
 inline bool streamed_stores(const Problem& p) {

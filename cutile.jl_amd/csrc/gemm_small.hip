@@ -6,8 +6,9 @@
 // four waves of a workgroup do not share a tile's extent but its K: wave w takes the stages w, w + 4, ... of 64 k, with an LDS
 // area and accumulators of its own.  Nothing is shared before the sums are, so there is no barrier in the walk: a wave waits
 // for its own transfers, reads all fragments of the stage into registers, requests its next stage into the same place and
-// multiplies meanwhile.  (A ring of two or three stages per wave is no faster: with 32 to 64 KB per workgroup two or more fit
-// a CU, and one's transfers run under another's products.  Eight waves, and stages of 32 k, are slower.)  A wave adds
+// multiplies meanwhile.  (A ring of two or three stages per wave is no faster; eight waves, and stages of 32 k, are slower.)
+// Two or more workgroups of the two smaller tiles fit a CU, and one's transfers run under another's products; 64 x 64 tiles have 259
+// registers a lane and 128 x 64 all 512 with four spilled, one workgroup to a CU.  A wave adds
 // every second step of 16 k (fourth on 32 x 32 tiles) into a chain of its own, 8 (16) chains per element in all, so the sums are no further from
 // exact than those of the split over K that this kernel replaces; the waves' sums are added through the LDS in their order.
 //

@@ -1080,6 +1080,8 @@ void launch_fwd(int vecs, dim3 grid, hipStream_t s, const float* X, int64_t ldx,
 #undef FWD
 }
 
+// The backward of one row per workgroup: rows of less than four elements, of more than 8192 that ln_bwd_wide_kernel does not take, and
+// with MI_LN_BWD_RG=1, for comparisons, every other.
 template <bool AL, bool ST>
 void launch_bwd(int vecs, dim3 grid, hipStream_t s, float* DX, int64_t lddx, const float* DY,
                 int64_t lddy, float* DW, int64_t lddw, float* DB, int64_t lddb, const float* X,
