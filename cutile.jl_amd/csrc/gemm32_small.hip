@@ -182,12 +182,13 @@ namespace gemm {
 // The kernel and tile that are estimated to be through first (us), for products of up to 2048 tiles of 64 x 64 and a K of 64 to 1024:
 // this one's, gemm32_big.hip's 64 x 64, 128 x 128 or 256 x 128, or where that does not apply the register-staged kernel.  A launch,
 // and per round of the CUs a ramp and the walk, in whole stages for each wave, dearer with rows off 16-byte boundaries; fitted to 420
-// shapes of 2 to 12 times 128..1024 x 128..2048 x 128..512, each with all of the tiles, off by 5 to 9 % (standard deviation): against
-// the 64 x 64 tile, whose two workgroups to a CU the count by rounds does not know (8 x 765 x 256 x 384 16.5 : 19.8), 32 x 32 tiles have to
-// promise 15 % and 64 x 32 ones 10.  Of 5700 shapes that this rule sends elsewhere than the rule by rounds alone (1 to 40 times 4..2048 x
-// 1..4096 x 64..1024) 5 take 1.02 to 1.04 of the time; without these margins 51 of 6000, up to 1.20.  The mean is 0.67 within the 128..1024
-// x 128..2048 x 128..512 of 1 to 12 entries, 0.37 of the others.  (7 x 832 x 384 x 489: 128 x 128 36, 64 x 64 31, 32 x 32 29.)
-// MI_GEMM_SMALL=0, read at every call, leaves all to that rule, and so does a forced tile.
+// shapes of 2 to 12 times 128..1024 x 128..2048 x 128..512, each with all of the tiles, off by 5 to 9 % (standard deviation).  Five
+// workgroups of the 32 x 32 tile fit a CU by their LDS, three of the 64 x 32 one: what comes sixth runs by itself, and there the 64 x 64 tile,
+// which has 1.3 to 1.5 rounds then, is the quicker one (8 x 765 x 256 x 384 16.5 : 19.8, of 67 such shapes 38 by more than 2 %); with three
+// rounds of 64 x 32 tiles likewise, and with five of 32 x 32 ones the estimate has to promise 12 %.  Of 5000 shapes that this rule sends elsewhere
+// than the rule by rounds alone (1 to 40 times 4..2048 x 1..4096 x 64..1024, three sets of operands in turn) 25 take 1.02 to 1.15 of the time; without
+// these lines 50 of 4500, up to 1.24.  The mean is 0.66 within the 128..1024 x 128..2048 x 128..512 of 1 to 12 entries, 0.38 of the others.  (7 x 832 x
+// 384 x 489: 128 x 128 36, 64 x 64 31, 32 x 32 29.)  MI_GEMM_SMALL=0, read at every call, leaves all to that rule, and so does a forced tile.
 bool small32_try(const Problem& p, int* big_tile, hipStream_t s) {
     static const bool forced = getenv("MI_GEMM_KERNEL") || getenv("MI_GEMM_BIG_TILE");
     if (forced || p.out_dtype != MI_F32 || p.M < 4 || p.K < 64 || p.K > 1024 || tiles_of(p, 64, 64) > 2048) return false;
@@ -210,7 +211,7 @@ bool small32_try(const Problem& p, int* big_tile, hipStream_t s) {
         const double b42 = us(1.55, rounds(256, 128), 7.36, k64, 107.3e-3, 7.4e-3);
         other = b11 < b22 && b11 < b42 ? b11 : b22 < b42 ? b22 : b42;
         *big_tile = other == b11 ? 11 : other == b22 ? 22 : 42;
-        if (*big_tile == 11) margin = t11 <= t21 ? 0.85 : 0.90;
+        if (*big_tile == 11) margin = t11 > t21 ? (rounds(64, 32) == 3 ? 0.0 : 0.94) : rounds(32, 32) == 6 ? 0.0 : rounds(32, 32) == 5 ? 0.88 : 0.94;
     } else {
         other = us(2.5, rounds(128, 128), 2.8, p.K, 115e-3, 0.0);
     }

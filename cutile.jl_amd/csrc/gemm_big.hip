@@ -467,10 +467,11 @@ bool big16_applicable(const Problem& p) {
 // Up to 128 tiles of 128 x 128 -- half the CUs, which is where the larger tiles lose to what one CU can bring in -- whichever
 // kernel is estimated to be through first.  A longer K is the split's (160 x 1200 x 11376 19 : 29 us), a shorter one the register-staged
 // kernels' (2056 x 736 x 41 5.0 : 6.6).  The estimates are least sure where the two are close: 128 x 64 tiles (whole 128 x 128 ones of the
-// other kernel are quicker than the mean that it is counted with, 512 x 3584 x 1216 10.5 : 12.6) and against a split (2560 x 384 x 3737 18.7 : 22.3),
-// so those have to promise 12 to 20 %.  Of 9800 shapes that are taken (256 to 4096 each way, 8 x 1 and up, batches of up to 64) 13 take 1.02 to 1.07 of
-// the other kernels' time, without these margins 34 of 7000, up to 1.20; the mean is 0.64 of those with 256 and more each way, 0.45-0.51 of the others.
-// MI_GEMM_SMALL=0, read at every call, leaves them all to the other kernels, and so do the settings that force one of those.
+// other kernel are quicker than the mean that it is counted with, 512 x 3584 x 1216 10.5 : 12.6) and against a split (2816 x 384 x 2191 16.8 : 18.2),
+// so those have to promise 10 to 16 %.  Of 6000 shapes that are taken (256 to 4096 each way, 8 x 1 and up, batches of up to 64; three sets of
+// operands in turn) 12 take 1.02 to 1.06 of the other kernels' time, without these margins 27 of 4200, up to 1.18; the mean is 0.65 of those with
+// 256 and more each way, 0.49-0.54 of the others.  MI_GEMM_SMALL=0, read at every call, leaves them all to the other kernels, and so do the
+// settings that force one of those.
 bool small16_try(const Problem& p, hipStream_t s) {
     static const bool forced = getenv("MI_GEMM_KERNEL") || getenv("MI_GEMM_SPLITK") || getenv("MI_GEMM_BIG_TILE");
     if (forced || tiles_of(p, 128, 128) > 128 || p.M < 8 || p.K < 256 || p.K > 4096) return false;
@@ -482,9 +483,10 @@ bool small16_try(const Problem& p, hipStream_t s) {
     double other = 0.0;
     // (more than eight parts are more chains than a wave of the larger tiles has)
     const int parts = pick_split(p, &kchunk, &other);
+    const double close = other;
     if (p.K > 3072) other *= 0.9;   // (744 x 721 x 4063 20.1 : 22.8; the fit is short there)
     const double us = small16_estimate(p, misaligned(p), &tile);
-    if (us > other * (tile == 42 ? 0.84 : tile == 11 || !parts ? 1.0 : tile == 22 ? 0.80 : 0.88) || (parts > 8 && tile != 11)) return false;
+    if (us > other || us > close * (tile == 42 ? 0.90 : tile == 11 || !parts ? 1.0 : tile == 22 ? 0.84 : 0.88) || (parts > 8 && tile != 11)) return false;
     small16_launch(p, tile, dma_extent(p), s);
     return true;
 }

@@ -62,8 +62,8 @@ def test_few_tiles_batched_exact(ct, orc, M, N, K, nb):
 @pytest.mark.parametrize("M,N,K,small", [(512, 512, 255, False), (512, 512, 256, True), (256, 256, 4096, True), (256, 256, 4104, False),
                                          (2048, 1024, 320, False), (2049, 1024, 2048, False), (1536, 735, 576, True), (1664, 1792, 832, False),
                                          # estimated close to the other kernels: 128 x 64 tiles, and against a split
-                                         (512, 3584, 1216, False), (832, 2240, 1280, False), (2816, 384, 2191, False), (1397, 727, 3136, False),
-                                         (512, 1443, 3043, True)])
+                                         (512, 3584, 1216, False), (832, 2240, 1280, False), (2816, 384, 2191, False), (512, 1443, 3043, True),
+                                         (1249, 704, 4032, True)])
 def test_both_sides_of_the_rule(ct, orc, M, N, K, small):
     A, B, ref = _operands(orc, M, N, K, torch.float16, (0, 0))
     C = torch.empty((N, M), dtype=torch.float32, device="cuda")
@@ -89,8 +89,9 @@ def test_few_tiles_infinities_and_nan_stay_in_their_rows_and_columns(ct, orc):
     (128, 100, 1024, 2, (0, 0), "small_32x32x32"), (101, 63, 1023, 3, (0, 0), "small_32x32x32"),
     (720, 128, 500, 3, (0, 0), "small_64x32x32"), (249, 181, 384, 8, (0, 0), "small_64x32x32"), (629, 141, 143, 9, (2, 3), "small_64x32x32"),
     # the tiles of gemm32_big.hip where they are estimated to be the quicker ones
-    (832, 384, 489, 12, (0, 0), "big_"), (765, 256, 384, 8, (0, 0), "big_64x64x16_ring4"), (192, 1283, 383, 6, (0, 0), "big_64x64x16_ring4"),
-    (576, 201, 384, 12, (0, 0), "big_64x64x16_ring4"), (320, 2007, 160, 10, (0, 0), "big_64x64x16_ring4"), (2056, 2311, 388, 1, (0, 0), "big_64x64x16_ring4"),
+    (832, 384, 489, 12, (0, 0), "big_"), (320, 2007, 160, 10, (0, 0), "big_64x64x16_ring4"), (2056, 2311, 388, 1, (0, 0), "big_64x64x16_ring4"),
+    (765, 256, 384, 8, (0, 0), "big_64x64x16_ring4"), (192, 1283, 383, 6, (0, 0), "big_64x64x16_ring4"),
+    (576, 201, 384, 12, (0, 0), "big_64x64x16_ring4"),   # (two of them share a CU)
 ])
 def test_few_fp32_tiles_exact(ct, orc, M, N, K, nb, pad, kernel):
     A, B, ref = _operands(orc, M, N, K, torch.float32, pad, nb)
