@@ -941,21 +941,22 @@ bool pick_inside(int64_t wgs, int64_t rows, int D, int Sq, int Skv, bool causal,
 // Launches of few queries (fmha_few.hip) where that kernel is estimated to be through first; launched and true.  `other`: the kernel
 // that takes the launch otherwise, `parts`: in how many parts it would split the keys.  Estimates in us: a launch, the longest walk and what
 // each SIMD has to do, fitted for every kernel to the shapes that it takes (batches of 1 to 16 with 1 to 64 heads, 65 to 4096 queries, 32 to
-// 5120 keys; standard deviation 4 to 11 %).  Of 8400 such shapes that are taken 17 take 1.02 to 1.10 of the other kernel's time and one 1.25
-// (16 x 16 heads of 64, 104 of 1493 keys); the mean is 0.72 with as many keys as queries and 0.73 with others.  Where an estimate is least sure the
-// kernel has to promise more: launches of 7 to 10 us on the kernels that walk the keys alone (128: 16 x 16 heads, S = 113, 8.1 : 8.6; 64: 4 x 64, 331
-// of 41 keys 9.3 : 10.0), and against the pipelined kernel for heads of 128 launches that are not causal (10 to 20 % short) or are with another
-// number of keys, whose walks are mostly of one length (1 x 32 heads, 1943 of 555 keys 26.5 : 32.4).
+// 5120 keys; standard deviation 4 to 11 %).  Of 4000 such shapes that are taken, three sets of operands in turn, 10 take 1.02 to 1.10
+// of the other kernel's time; the mean is 0.72 with as many keys as queries and 0.75 with others.  Where an estimate is least sure the kernel has
+// to promise more: with other numbers of keys on the kernels that walk them alone (7 to 10 us; heads of 64, 4 x 64, 331 of 41 keys 9.3 : 10.0), and
+// against the pipelined kernel for heads of 128 launches that are not causal (10 to 20 % short) or are with another number of keys, whose
+// walks are mostly of one length (1 x 32 heads, 1943 of 555 keys 26.5 : 32.4).
 enum FewOther { PIPE64, SPLIT64, PLAIN64, PLAIN128, KEYS2, SPLITKV, PIPE128 };
 bool few_instead(const fmha::Problem& p, FewOther other, int parts, hipStream_t s) {
     const fmha::Walks w = fmha::walks_of(p);
     const int64_t Sq = p.Q->sizes[1], rows = Sq * p.Q->sizes[2] * p.Q->sizes[3];
     const bool d64 = p.Q->sizes[0] == 64, same = Sq == p.K->sizes[1];
     // (no further than what was measured; the pipelined kernel for heads of 64 is level from about 60 halves per SIMD on: 1 x 32 heads,
-    // S = 2565 causal, 104 of them, 44 : 49; many tiles that walk three or four halves each, 4 x 8 heads of 64, 3536 of 98 keys, 13.6 : 14.5; keys
+    // S = 2565 causal, 104 of them, 44 : 49; many tiles that walk few halves each, 4 x 8 heads of 64, 3536 of 98 keys, 13.6 : 14.5, 1 x 16 of 128, 2058 of 37, 8.4 : 10.6; keys
     // and values that stay in no cache from one tile of a head to the next, 16 x 8 heads of 128, 93 of 3283 keys, 215 MB, 62 : 75)
     const int64_t kv_bytes = 4 * p.K->sizes[0] * p.K->sizes[1] * p.K->sizes[2] * p.K->sizes[3];
     if (w.longest > 160 || w.halves > (d64 ? 60 : 120) || (other == PLAIN64 && w.tiles > 2.5) || kv_bytes > (192ll << 20)) return false;
+    if (other == PLAIN128 && w.longest <= 4 && w.tiles > (w.longest <= 2 ? 0.75 : 1.0)) return false;
     const bool ragged = Sq % 128 != 0;
     const double us = other == PIPE64     ? (ragged ? 6.53 + 0.191 * w.longest + 0.297 * w.halves : 5.48 + 0.209 * w.longest + 0.272 * w.halves)
                       : other == SPLIT64  ? 11.6 + 0.93 * ceil(w.longest / 2) / parts + 1.14e-4 * (double)rows * parts + 0.29 * w.halves
@@ -964,7 +965,7 @@ bool few_instead(const fmha::Problem& p, FewOther other, int parts, hipStream_t 
                       : other == KEYS2    ? 7.46 + 0.413 * w.longest + 0.180 * w.halves
                       : other == SPLITKV  ? fmin(13.8 + 0.109 * w.longest + 0.774 * w.halves, 14.0 + 1.16 * w.halves)   // (few workgroups: 1 x 8, 136 of 2396 keys 18.1)
                                           : 13.8 + 0.346 * w.longest + 0.369 * w.halves;
-    const double margin = other == PLAIN64 ? 0.81 : other == PLAIN128 ? 0.84 : other != PIPE128 ? 0.92 : !p.causal ? 0.8 : same ? 0.92 : 0.7;
+    const double margin = other == PLAIN64 ? 0.86 : other == PLAIN128 && !same ? 0.88 : other != PIPE128 ? 0.92 : !p.causal ? 0.8 : same ? 0.92 : 0.75;
     int waves = 0;
     if (fmha::few_estimate(p, w, &waves) > us * margin) return false;
     fmha::few_launch(p, waves, s);
@@ -1134,7 +1135,9 @@ extern "C" int mi_fmha_kernel(const mi_tile_array* Q, const mi_tile_array* K, co
         const int64_t wgs = cld(Sq, (int64_t)kQB) * B * H;
         if (D == 64 && may_few) {
             const int parts = pick_parts(wgs, B * H * Sq, 64, (int)Sq, (int)Skv, causal, input_pos);
-            if (few_instead(pr, fmha::pipe_applicable(pr) ? PIPE64 : parts ? SPLIT64 : PLAIN64, parts, s)) return launch_status();
+            // (one block of one head against many keys is left where its test holds it, 128 of 5120 keys 23.9 us and 15.6 on the split)
+            const FewOther other = fmha::pipe_applicable(pr) || wgs == 1 ? PIPE64 : parts ? SPLIT64 : PLAIN64;
+            if (few_instead(pr, other, parts, s)) return launch_status();
         }
         if (!no_pipe && fmha::pipe_applicable(pr)) {
             fmha::pipe_launch(pr, s);

@@ -73,9 +73,9 @@ def test_few_queries_is_no_further_off_than_the_kernels_it_replaces(ct, monkeypa
 
 
 @pytest.mark.parametrize("dim,B,H,sq,skv,few", [
-    (64, 1, 4, 64, 640, False), (64, 1, 4, 65, 640, True), (64, 1, 16, 512, 5120, True), (64, 1, 16, 512, 5121, False),
-    # the walk of a wave by itself against a split (5120 keys 23.9 us : 15.6, 2700 14.2 : 17.5), and the kernels that walk few keys
-    (64, 1, 1, 128, 5120, False), (64, 1, 1, 128, 2700, True), (64, 4, 64, 331, 41, False), (128, 2, 8, 2375, 57, False),
+    (64, 1, 4, 64, 640, False), (64, 1, 4, 65, 640, True), (64, 1, 1, 128, 5120, True), (64, 1, 1, 128, 5121, False),
+    # the walk of a wave by itself against a split (2 heads, 5120 keys 24 us : 15.9), and the kernels that walk few keys
+    (64, 1, 2, 128, 5120, False), (64, 1, 2, 128, 2700, True), (64, 1, 16, 512, 5120, True), (64, 1, 16, 512, 5121, False), (64, 4, 64, 331, 41, False), (128, 2, 8, 2375, 57, False),
     # not causal with other keys: two groups of waves, 59 us : 70
     (128, 1, 32, 838, 3111, False),
     (128, 1, 1, 128, 5121, False), (64, 8, 32, 1024, 1024, False), (128, 4, 32, 1024, 1024, False), (128, 1, 32, 1280, 1280, False),
@@ -100,9 +100,22 @@ def test_both_sides_of_the_rule_causal_with_other_keys(ct, B, H, sq, skv, pos, f
     assert _err(got[:1, :4], _reference(Q[:1, :4], K[:1, :4], V[:1, :4], pos, True)) <= 2**-10
 
 
+def test_few_queries_infinities_and_nan(ct):
+    """A NaN in a key reaches the queries that see it and no others."""
+    g = torch.Generator(device="cuda").manual_seed(3)
+    Q, K, V = (torch.empty(1, 4, 200, 64, device="cuda", dtype=torch.float16).normal_(0, 1, generator=g) for _ in range(3))
+    clean = fmha.cutile_fmha(Q, K, V, causal=True)
+    assert ct.last_variant().startswith("fmha_few")
+    K[0, 1, 70, 5] = float("nan")
+    got = fmha.cutile_fmha(Q, K, V, causal=True)
+    bad = torch.isnan(got.float()).any(-1)[0]
+    assert bad[1, 70:].all() and not bad[1, :70].any() and not bad[[0, 2, 3]].any()
+    assert torch.equal(got[0, 1, :70], clean[0, 1, :70])
+
+
 @pytest.mark.parametrize("dim", [64, 128])
-def test_few_queries_infinities_and_nan(ct, dim):
-    """A NaN in a key reaches the queries that see it and no others; an infinite value, and a score of either infinity, likewise."""
+def test_few_queries_infinities_of_both_head_sizes(ct, dim):
+    """A NaN or a score of either infinity reaches the queries that see it and no others, an infinite value likewise."""
     g = torch.Generator(device="cuda").manual_seed(3)
     Q, K, V = (torch.empty(1, 4, 200, dim, device="cuda", dtype=torch.float16).normal_(0, 1, generator=g) for _ in range(3))
     Q[..., 5] = Q[..., 5].abs() + 0.25
